@@ -1,5 +1,6 @@
 // static.hip -- the static (augmented-reality) collider set: range image -> scene points and
 // normals, the static points' grid index, and the DEM of the dynamic particles against them.
+#include "coop_cells.hpp"
 #include "csr_fill.hpp"
 #include "kernels.hpp"
 
@@ -94,49 +95,83 @@ __global__ void k_static_reorder(const unsigned *__restrict__ keys, const unsign
 //    through the static sorted index, every particle: pForce += F, pTorque += relativePos x F.
 //  engine: the exact static cell table and sorted normals, body particles only: pForce += F (the
 //    torque is relativePos x pForce, formed by the reduction).
+// A workgroup first tests its particles one per thread for any candidate (the 9 rows of cells, three
+// consecutive cells each), then takes those that have some 16 lanes each (coop_cells): the walk of a
+// particle on a scanned surface, about a thousand candidates, was one serial chain per thread, bound by
+// the latency of its loads.  16,384 particles on the points of a 640 x 480 depth image: 1,280 -> 97 us;
+// a 2^20-particle scene over a floor of 2^20 points (few particles near it): step 286 -> 210 us.  Without
+// the first test every particle takes 16 lanes, and that scene over 65,536 points costs 240 us a step
+// instead of 187 (one thread per particle: 213).
+constexpr int kStaticBlock = 128;
 template <bool REF>
-__global__ void k_dem_static(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
-                             const unsigned *__restrict__ sIdx, int n, const float4 *__restrict__ stPos,
-                             const float4 *__restrict__ stNorm, const unsigned *__restrict__ stIdx,
-                             const unsigned *__restrict__ cs, const unsigned *__restrict__ ce, DevPhys ph,
-                             SceneGeom g, float4 *__restrict__ pForce, float4 *__restrict__ pTorque,
-                             const float4 *__restrict__ relPos) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float4 P = sPos[i];
-    if (!REF && __float_as_int(P.w) < 0) return;
-    const f3 pa = xyz(P), va = xyz(sVel[i]);
-    int gx, gy, gz;
-    grid_pos(pa, g, gx, gy, gz);
-    f3 F = mk3(0.f, 0.f, 0.f);
-    for (int z = -1; z <= 1; ++z)
-        for (int y = -1; y <= 1; ++y)
-            for (int x = -1; x <= 1; ++x) {
-                const unsigned h = grid_hash(gx + x, gy + y, gz + z, g);
-                f3 csum = mk3(0.f, 0.f, 0.f);
-                unsigned j, e;
-                if (REF) {
-                    j = cs[h];
-                    e = j == kEmpty ? j : ce[h];
-                } else {
-                    j = cs[h];
-                    e = cs[h + 1];
-                }
-                for (; j < e; ++j) {
-                    const f3 ps = xyz(stPos[j]);
-                    const f3 ns = xyz(stNorm[REF ? stIdx[j] : j]);
-                    f3 fj;
-                    if (static_force(pa, ps, ns, va, ph, fj)) csum = add3(csum, fj);
-                }
-                F = add3(F, csum);
+__global__ __launch_bounds__(kStaticBlock) void k_dem_static(
+    const float4 *__restrict__ sPos, const float4 *__restrict__ sVel, const unsigned *__restrict__ sIdx, int n,
+    int perBlock, const float4 *__restrict__ stPos, const float4 *__restrict__ stNorm,
+    const unsigned *__restrict__ stIdx, const unsigned *__restrict__ cs, const unsigned *__restrict__ ce, DevPhys ph,
+    SceneGeom g, float4 *__restrict__ pForce, float4 *__restrict__ pTorque, const float4 *__restrict__ relPos) {
+    __shared__ CoopGroupLds sGroup[kStaticBlock / kCoopLanes];
+    __shared__ int sList[kStaticBlock];
+    __shared__ int sCount;
+    const int t = (int)threadIdx.x, first = xcd_block((int)blockIdx.x, (int)gridDim.x) * perBlock;
+    if (t == 0) sCount = 0;
+    __syncthreads();
+    if (t < perBlock && first + t < n) {
+        const float4 P = sPos[first + t];
+        bool some = false;
+        if (REF || __float_as_int(P.w) >= 0) {
+            int gx, gy, gz;
+            grid_pos(xyz(P), g, gx, gy, gz);
+            for (int r = 0; r < 9; ++r) {
+                const unsigned h0 = grid_hash(gx - 1, gy + r % 3 - 1, gz + r / 3 - 1, g);
+                const unsigned h1 = grid_hash(gx, gy + r % 3 - 1, gz + r / 3 - 1, g);
+                const unsigned h2 = grid_hash(gx + 1, gy + r % 3 - 1, gz + r / 3 - 1, g);
+                if (REF) some = some | (cs[h0] != kEmpty) | (cs[h1] != kEmpty) | (cs[h2] != kEmpty);
+                else if (h2 == h0 + 2u) some = some | (cs[h0] != cs[h0 + 3u]);
+                else some = some | (cs[h0] != cs[h0 + 1u]) | (cs[h1] != cs[h1 + 1u]) | (cs[h2] != cs[h2 + 1u]);
             }
-    const unsigned o = sIdx[i];
-    const float4 old = pForce[o];
-    pForce[o] = make_float4(old.x + F.x, old.y + F.y, old.z + F.z, old.w + 0.0f);
-    if (REF) {
-        const float4 t = pTorque[o];
-        const f3 tq = cross3(xyz(relPos[o]), F);
-        pTorque[o] = make_float4(t.x + tq.x, t.y + tq.y, t.z + tq.z, t.w + 0.0f);
+        }
+        if (some) sList[atomicAdd(&sCount, 1)] = first + t;   // (each particle is written by itself: any order)
+        else if (REF) {   // nothing to add: a sum of no contacts is +0
+            const unsigned o = sIdx[first + t];
+            const float4 f = pForce[o], q = pTorque[o];
+            const f3 tq = cross3(xyz(relPos[o]), mk3(0.f, 0.f, 0.f));
+            pForce[o] = make_float4(f.x + 0.0f, f.y + 0.0f, f.z + 0.0f, f.w + 0.0f);
+            pTorque[o] = make_float4(q.x + tq.x, q.y + tq.y, q.z + tq.z, q.w + 0.0f);
+        }
+    }
+    __syncthreads();
+    const int count = sCount, gl = t / kCoopLanes, l = t & (kCoopLanes - 1);
+    // (a wave's four groups stay together: the bound is the wave's, not the group's)
+    for (int k0 = (t >> 6) * (64 / kCoopLanes); k0 < count; k0 += kStaticBlock / kCoopLanes) {
+        const int k = k0 + (gl & (64 / kCoopLanes - 1));
+        const bool valid = k < count;
+        const int i = sList[valid ? k : k0];
+        const f3 pa = xyz(sPos[i]), va = xyz(sVel[i]);
+        int gx, gy, gz;
+        grid_pos(pa, g, gx, gy, gz);
+        const float F = coop_cells(
+            sGroup[gl], valid,
+            [&](int c, unsigned &b, unsigned &e) {
+                const unsigned h = grid_hash(gx + c % 3 - 1, gy + (c / 3) % 3 - 1, gz + c / 9 - 1, g);
+                b = cs[h];
+                e = REF ? ce[h] : cs[h + 1];
+                if (REF && (b == kEmpty || e < b)) b = e = 0u;   // an empty cell's end is not defined
+            },
+            [&](unsigned j, f3 &f) {
+                const f3 ps = xyz(stPos[j]);
+                if (!in_contact(pa, ps, ph)) return false;
+                return static_force(pa, ps, xyz(stNorm[REF ? stIdx[j] : j]), va, ph, f);
+            });
+        const f3 F3 = mk3(__shfl(F, 0, kCoopLanes), __shfl(F, 1, kCoopLanes), __shfl(F, 2, kCoopLanes));
+        if (!valid || l > 3) continue;
+        const unsigned o = sIdx[i];
+        auto pick = [l](f3 v) { return l == 0 ? v.x : l == 1 ? v.y : l == 2 ? v.z : 0.0f; };
+        float *pf = reinterpret_cast<float *>(pForce + o) + l;
+        *pf = *pf + pick(F3);
+        if (REF) {
+            float *pt = reinterpret_cast<float *>(pTorque + o) + l;
+            *pt = *pt + pick(cross3(xyz(relPos[o]), F3));
+        }
     }
 }
 
@@ -171,13 +206,19 @@ void launch_dem_static(const float4 *sPos, const float4 *sVel, const unsigned *s
                        const DevPhys &ph, const SceneGeom &g, float4 *pForce, float4 *pTorque,
                        const float4 *relPos, bool refLayout, hipStream_t st) {
     if (n <= 0) return;
-    const dim3 grid((n + 127) / 128);
+    // particles per workgroup: one per group of 16 lanes up to 8,192 workgroups (32 a CU: the particles near a
+    // surface, few and together, spread over the chip), then more, up to one per thread
+    const int groups = kStaticBlock / kCoopLanes;
+    int perBlock = (n + 8191) / 8192;
+    if (perBlock < groups) perBlock = groups;
+    if (perBlock > kStaticBlock) perBlock = kStaticBlock;
+    const dim3 grid((n + perBlock - 1) / perBlock);
     if (refLayout)
-        hipLaunchKernelGGL(k_dem_static<true>, grid, dim3(128), 0, st, sPos, sVel, sIdx, n, stPos, stNorm, stIdx, cs,
-                           ce, ph, g, pForce, pTorque, relPos);
+        hipLaunchKernelGGL(k_dem_static<true>, grid, dim3(kStaticBlock), 0, st, sPos, sVel, sIdx, n, perBlock, stPos,
+                           stNorm, stIdx, cs, ce, ph, g, pForce, pTorque, relPos);
     else
-        hipLaunchKernelGGL(k_dem_static<false>, grid, dim3(128), 0, st, sPos, sVel, sIdx, n, stPos, stNorm, stIdx,
-                           cs, ce, ph, g, pForce, pTorque, relPos);
+        hipLaunchKernelGGL(k_dem_static<false>, grid, dim3(kStaticBlock), 0, st, sPos, sVel, sIdx, n, perBlock, stPos,
+                           stNorm, stIdx, cs, ce, ph, g, pForce, pTorque, relPos);
 }
 
 }  // namespace arsim
