@@ -68,7 +68,7 @@ def parse():
                     help="only step the 512-scene batch (default tuning, no autotune): for profilers")
     ap.add_argument("--traversal-stats", action="store_true",
                     help="LBVH packet traversal statistics of the 2^20-particle scene (nodes visited per wave, leaf "
-                         "tests per particle, stack depth) from the counting build libarsim_traversal_stats.so")
+                         "tests per particle, list length) from the counting build libarsim_traversal_stats.so")
     ap.add_argument("--scene", choices=["small", "pile", "sis"], default=None,
                     help="time another plain scene instead of the headline one: 'small' = 256 cubes (16,384 "
                          "particles, 64^3 grid), 'pile' = the dense ellipsoid pile (~4.2 M particles), 'sis' = the "
@@ -126,17 +126,17 @@ def traversal_stats(args):
         e.step(args.steps)
         e.sync()
         capi.check(fn(capi.ptr(out), 1), "stats")
-    waves, visits, lanes, leaf_tests, interest, max_sp, done, contacts, packets, iters = (int(x) for x in out)
+    waves, visits, lanes, leaf_tests, reach, max_size, done, contacts, packets, iters = (int(x) for x in out)
     width = 64 * waves / max(packets, 1)   # lanes per packet
     print(json.dumps({"traversal_stats": True, "method": "lbvh30" if method == capi.METHOD_LBVH30 else "lbvh63",
                       "particles": sc.n, "steps": args.steps, "waves": waves, "packets": packets,
                       "lanes_per_packet": width,
-                      "nodes_visited_per_packet": visits / max(packets, 1),
-                      "node_loop_iterations_per_wave": iters / max(waves, 1),
+                      "nodes_expanded_per_packet": visits / max(packets, 1),
+                      "steps_per_wave": iters / max(waves, 1),
                       "leaf_tests_per_particle": leaf_tests / max(lanes, 1),
                       "contacts_per_particle": contacts / max(lanes, 1),
-                      "packet_efficiency": interest / max(visits * width, 1),
-                      "max_stack_depth": max_sp, "completed_lanes": done, "valid_lanes": lanes}))
+                      "candidates_in_reach": reach / max(leaf_tests, 1),
+                      "most_list_entries": max_size, "completed_lanes": done, "valid_lanes": lanes}))
 
 
 def batched_only(args):

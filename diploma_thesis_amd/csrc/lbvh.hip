@@ -8,14 +8,13 @@ namespace arsim {
 
 namespace {
 
-constexpr int kStackDepth = 64;   // per-thread LDS stack entries (the reference's int stack[64], RB_BVHKernels.cu:129)
-constexpr int kWaveStackDepth = 64;   // per-wave LDS stack entries of the packet traversal
+constexpr int kStackDepth = 64;   // the reference's int stack[64] (RB_BVHKernels.cu:129)
 
 #ifdef ARSIM_TRAVERSAL_STATS
 // Counting build only: totals of the packet traversal.
-//   [0] waves  [1] internal nodes visited, summed over packets  [2] valid lanes  [3] lane-leaf tests
-//   [4] lanes whose box overlaps an entered node, summed over entered nodes  [5] largest stack depth
-//   [6] lanes that completed  [7] contacts found  [8] packets  [9] iterations of the waves' node loops
+//   [0] waves  [1] nodes expanded  [2] valid lanes  [3] candidates tested, summed over lanes
+//   [4] of those in reach of the lane's particle  [5] most entries of a packet's list  [6] lanes that
+//   completed  [7] contacts found  [8] packets  [9] steps of the waves' loops
 constexpr int kTravStats = 10;
 __device__ unsigned long long g_travStats[kTravStats];
 #endif
@@ -529,299 +528,348 @@ __device__ __forceinline__ bool overlap(float4 aMin, float4 aMax, float4 bMin, f
            (aMin.z <= bMax.z) & (aMax.z >= bMin.z);
 }
 
-// collideBVHSoARigidBody (Kernels/RB_BVHKernels.cu:100-244): per sorted leaf, traversal from the
-// root (or the leaf's scene root), left child before right, the right child pushed when both
-// are entered.  Leaves are the nodes < n.  The stack lives in LDS, one column per thread.
+// ---------------------------------------------------------------- traversal
+// collideBVHSoARigidBody (Kernels/RB_BVHKernels.cu:100-244): per sorted leaf the contacts met by a traversal
+// from the root (or the leaf's scene root): a node's leaf children (left before right), then its inner
+// children (left before right).  Leaves are the nodes < n.  A lane's force is the sum over its contacts
+// in that order.
+
+// Where a node's children come from: the engine's packed 64-byte record, or the reference's arrays.
+struct PackedNodes {
+    const float4 *packed;
+    int n;
+    __device__ __forceinline__ void load(int node, int &L, int &R, float4 &a0, float4 &a1, float4 &b0, float4 &b1) const {
+        const float4 *q = packed + 4 * (size_t)(node - n);
+        a0 = q[0]; a1 = q[1]; b0 = q[2]; b1 = q[3];
+        L = __float_as_int(a0.w);
+        R = __float_as_int(a1.w);
+    }
+};
+struct RefNodes {
+    const int *left, *right;
+    const float4 *bounds;
+    __device__ __forceinline__ void load(int node, int &L, int &R, float4 &a0, float4 &a1, float4 &b0, float4 &b1) const {
+        L = left[node];
+        R = right[node];
+        a0 = bounds[2 * (size_t)L]; a1 = bounds[2 * (size_t)L + 1];
+        b0 = bounds[2 * (size_t)R]; b1 = bounds[2 * (size_t)R + 1];
+    }
+};
+
+constexpr int kPacketLanes = 16;
+constexpr int kCandCap = 64;                               // candidate leaves a packet holds before it tests them
+constexpr int kCandRound = 32;                             // of them tested per round,
+constexpr int kCandStep = 4;                               // read from LDS this many at a time
+constexpr int kFrontCap = 192;                           // entries of a packet's list of nodes to expand
+constexpr int kFrontWide = kFrontCap - kStackDepth;        // up to here 16 entries are expanded at once, then one
+// LDS of a packet in float4: centres, list, candidates, and 64 bytes that put the four packets of a wave,
+// which read their centres together, on different banks
+constexpr int kPacketLds = kCandRound + (kFrontCap + kCandCap) / 4 + 4;
+
+// One particle's side of the contact tests.
+struct LeafQuery {
+    int i, ra;
+    f3 pa, va;
+    float4 qMin, qMax;              // its box
+};
+struct LeafSum {
+    f3 F;
+    int cnt;
+};
+// Leaf j (centre Q) against the lane's particle: the force added, or the pair listed (EMIT).
 template <bool EMIT>
-__global__ void k_dem_lbvh(const int *__restrict__ sIdx, Lbvh t, int n, DevPhys ph, SceneView sv, int sceneInVelW,
-                           DemOut o, int *overflow) {
-    extern __shared__ int sStack[];
-    const int lb = xcd_block((int)blockIdx.x, (int)gridDim.x);
-    const int i = lb * (int)blockDim.x + (int)threadIdx.x;
-    if (i >= n) return;
-    const int bd = (int)blockDim.x, tid = (int)threadIdx.x;
-    const float4 C = t.cms[i];
-    const float4 Vq = t.sortedVel[i];
-    const int ra = __float_as_int(C.w);
-    const int s = sceneInVelW ? __float_as_int(Vq.w) : 0;
-    const float4 qMin = t.bounds[2 * (size_t)i], qMax = t.bounds[2 * (size_t)i + 1];
-    const f3 pa = xyz(C), va = xyz(Vq);
-    const int orig = sIdx[i];
-    int node = t.sceneRoot ? t.sceneRoot[s] : (n >= 2 ? n : -1);
-    f3 F = mk3(0.f, 0.f, 0.f);
-    int cnt = 0, sp = 0;
-    bool ovf = false;   // stack overflow: the traversal is incomplete and nothing is written
-    while (node >= n) {
-        int L, R;
-        bool oL, oR;
-        if (t.packed) {
-            // one 64-byte node: both children's boxes and ids
-            const float4 *q = t.packed + 4 * (size_t)(node - n);
-            const float4 a0 = q[0], a1 = q[1], b0 = q[2], b1 = q[3];
-            L = __float_as_int(a0.w);
-            R = __float_as_int(a1.w);
-            oL = L != i && overlap(qMin, qMax, a0, a1);
-            oR = R != i && overlap(qMin, qMax, b0, b1);
-        } else {
-            L = t.left[node];
-            R = t.right[node];
-            oL = L != i && overlap(qMin, qMax, t.bounds[2 * (size_t)L], t.bounds[2 * (size_t)L + 1]);
-            oR = R != i && overlap(qMin, qMax, t.bounds[2 * (size_t)R], t.bounds[2 * (size_t)R + 1]);
-        }
-        const bool lL = L < n, lR = R < n;
-        if (oL && lL) {
-            float4 CL = t.cms[L];
-            if (candidate(CL, pa, ra, false, ph)) {
-                if (EMIT) {
-                    if (in_contact(pa, xyz(CL), ph)) {
-                        if (cnt < o.maxPer) o.pairs[(size_t)orig * o.maxPer + cnt] = sIdx[L];
-                        ++cnt;
-                    }
-                } else {
-                    f3 fj;
-                    if (pair_force(pa, xyz(CL), va, xyz(t.sortedVel[L]), ph, fj)) F = add3(F, fj);
-                }
-            }
-        }
-        if (oR && lR) {
-            float4 CR = t.cms[R];
-            if (candidate(CR, pa, ra, false, ph)) {
-                if (EMIT) {
-                    if (in_contact(pa, xyz(CR), ph)) {
-                        if (cnt < o.maxPer) o.pairs[(size_t)orig * o.maxPer + cnt] = sIdx[R];
-                        ++cnt;
-                    }
-                } else {
-                    f3 fj;
-                    if (pair_force(pa, xyz(CR), va, xyz(t.sortedVel[R]), ph, fj)) F = add3(F, fj);
-                }
-            }
-        }
-        const bool tL = oL && !lL, tR = oR && !lR;
-        if (!tL && !tR) {
-            if (sp == 0) break;
-            --sp;
-            node = sStack[sp * bd + tid];
-        } else {
-            node = tL ? L : R;
-            if (tL && tR) {
-                if (sp == kStackDepth) {
-                    atomicOr(overflow, 1);
-                    ovf = true;
-                    break;
-                }
-                sStack[sp * bd + tid] = R;
-                ++sp;
-            }
-        }
-    }
-    if (ovf) return;
+__device__ __forceinline__ void leaf_contact(int j, const float4 &Q, const float4 &V, const LeafQuery &q,
+                                             const DevPhys &ph, const DemOut &o, const int *__restrict__ sIdx, int orig,
+                                             LeafSum &acc) {
     if (EMIT) {
-        o.counts[orig] = cnt;
-        return;
-    }
-    SceneGeom g;
-    load_geom(sv, s, g);
-    if (!((ph.flags & kGrainClamp) && ra < 0)) F = add3(F, wall_force(pa, va, ph, g));
-    if (ra >= 0) {
-        o.pForce[orig] = f4(F, 0.0f);
-        if (o.pTorque) o.pTorque[orig] = f4(cross3(xyz(o.relPos[orig]), F), 0.0f);
+        if (in_contact(q.pa, xyz(Q), ph)) {
+            if (acc.cnt < o.maxPer) o.pairs[(size_t)orig * o.maxPer + acc.cnt] = sIdx[j];
+            ++acc.cnt;
+        }
     } else {
-        const float fs = (ph.flags & kRefUnits) ? 1.0f : ph.dt;
-        o.vel[orig] = make_float4(va.x + F.x * fs, va.y + F.y * fs, va.z + F.z * fs, 0.0f);
+        f3 fj;
+        if (pair_force(q.pa, xyz(Q), q.va, xyz(V), ph, fj)) acc.F = add3(acc.F, fj);
     }
 }
 
-// Packet form of the same traversal: 16 consecutive leaves in Morton order (four packets per wave)
-// walk the tree together, with the packet's own node, LDS stack (kWaveStackDepth entries) and depth.
-// The packet visits a node when any of its lanes' boxes overlaps it.  A lane handles a leaf only when
-// its own box overlaps the leaf's, and every ancestor's box contains the leaf's box, so each lane meets
-// exactly the leaves of its own traversal, in the same depth-first order (left before right): the
-// per-lane force sums are bit-identical.  A smaller packet's lanes are closer together, so it enters
-// fewer nodes that none of its lanes overlaps (at the 2^20-particle scene a 64-lane packet enters 157
-// nodes, a 16-lane packet 78, and the wave, which runs as long as its slowest packet, 95).  A visit
-// loads the packet's 64-byte node record as one dword per lane and passes the words round the packet
-// by DPP row broadcasts.
-constexpr int kPacketLanes = 16;
-// Word K of each 16-lane row (DPP row_newbcast: every lane of a row receives lane K's value), as a float.
-template <int K>
-__device__ __forceinline__ float row_word(unsigned w) {
-    return __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, (int)w, 0x150 + K, 0xf, 0xf, false));
+// Inclusive minimum of the row's lanes before (SHR) or after this one, NaN ignored.
+template <bool SHR>
+__device__ __forceinline__ float row_scan_min(float v) {
+    const int inf = 0x7f800000;
+#define ARSIM_ROW_STEP(d) \
+    v = fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(inf, __float_as_int(v), (SHR ? 0x110 : 0x100) + d, 0xf, 0xf, false)))
+    ARSIM_ROW_STEP(1);
+    ARSIM_ROW_STEP(2);
+    ARSIM_ROW_STEP(4);
+    ARSIM_ROW_STEP(8);
+#undef ARSIM_ROW_STEP
+    return v;
 }
+struct Box6 { float v[6]; };        // min xyz, -max xyz
+__device__ __forceinline__ bool box_meets(const Box6 &b, const float4 &mn, const float4 &mx) {
+    return (b.v[0] <= mx.x) & (b.v[1] <= mx.y) & (b.v[2] <= mx.z) & (-b.v[3] >= mn.x) & (-b.v[4] >= mn.y) &
+           (-b.v[5] >= mn.z);
+}
+
+// Lanes of this lane's 16-lane row for which p holds.
+__device__ __forceinline__ unsigned row_ballot(bool p) {
+    const unsigned long long m = __ballot(p);
+    const unsigned lane = threadIdx.x & 63u;
+    const unsigned w = lane & 32u ? (unsigned)(m >> 32) : (unsigned)m;
+    return (w >> (lane & 16u)) & 0xffffu;
+}
+
+// A packet of 16 consecutive leaves traverses the tree together.  Its nodes to expand are a list in LDS
+// in the order a traversal meets them, the next one on top; a step takes up to 16 entries off the
+// top, one per lane, tests both children of each against the packet's reach and puts the children met
+// back in their place.  A walk node by node is bound by its chain of dependent record loads and by the
+// instructions of every visit (87 nodes a packet at the 2^20-particle scene); a step has 16 loads in
+// flight and there are 30 steps a wave.  Leaves that come up at the top of the list are the packet's next
+// candidates (40 there); the lanes test them 32 at a time from LDS and add their contacts in order.
+// Against 16-lane packets that walk node by node: 256 -> 152 us at the 2^20-particle scene, 103 -> 38 us at
+// 50,021 particles, 289 -> 111 us for a forest of 48 scenes (744,535 particles); against one thread per
+// leaf, 278 -> 117 us on the reference's arrays at a pile of 100,003.
+// The packet's reach is two boxes, the joint boxes of its leaves before and after the split that makes
+// them smallest: the 16 leaves of a Morton run often lie on both sides of a split of the tree, far
+// apart, where one box would take in everything between.  (With one box a packet in five overran a list
+// twice as long.  Every box that a lane's own box meets meets
+// one of them, and the contact test rejects what only the packet reaches.)
+// A packet's LDS: a list of 128 entries before the narrow steps made the pile's 262 us frame 362; registers are
+// held to five waves per SIMD, the most without spills (six and seven: within 2 %).
+// Past kFrontWide entries a step expands the top entry alone, which adds at most one entry per level,
+// so only trees deeper than kStackDepth levels can run out of room: that sets *overflow and
+// writes nothing for the packet.
 // FOREST: scenes' trees under their own roots (scene id in sortedVel.w); a packet whose lanes start at
-// different roots walks them one root after another, the lanes of the current root taking part.
-template <bool EMIT, bool FOREST>
-__global__ __attribute__((amdgpu_waves_per_eu(8))) void k_dem_lbvh_packets(const int *__restrict__ sIdx,
-                                                                           const float4 *__restrict__ packed,
-                                   const float4 *__restrict__ cms, const float4 *__restrict__ sVel,
-                                   const int *__restrict__ sceneRoot, int n,
-                                   DevPhys ph, SceneView sv, DemOut o, int *overflow) {
-    extern __shared__ int pStack[];
+// different roots walks them one after another, the lanes of the current root taking part.
+template <bool EMIT, bool FOREST, class NODES>
+__global__ __attribute__((amdgpu_waves_per_eu(5))) void k_dem_lbvh(
+    const int *__restrict__ sIdx, NODES nodes, const float4 *__restrict__ cms, const float4 *__restrict__ sVel,
+    const float4 *__restrict__ leafBounds, const int *__restrict__ sceneRoot, int n, DevPhys ph, SceneView sv, DemOut o,
+    int *overflow) {
+    extern __shared__ float4 pFront[];
     const int lb = xcd_block((int)blockIdx.x, (int)gridDim.x);
     const int i = lb * (int)blockDim.x + (int)threadIdx.x;
     const bool valid = i < n;
     const int ii = valid ? i : n - 1;
-    const int lane = (int)(threadIdx.x & 63);
-    const int pl = lane & (kPacketLanes - 1);
-    const unsigned long long pmask = 0xffffull << (lane & ~(kPacketLanes - 1));
-    int *stack = pStack + ((int)threadIdx.x / kPacketLanes) * kWaveStackDepth;
+    const int pl = (int)threadIdx.x & (kPacketLanes - 1);
+    const unsigned lower = (1u << pl) - 1u;
+    float4 *stage = pFront + ((int)threadIdx.x / kPacketLanes) * kPacketLds;
+    int *list = reinterpret_cast<int *>(stage + kCandRound), *cand = list + kFrontCap;
     const float4 C = cms[ii];
     const float4 Vq = sVel[ii];
-    const int ra = __float_as_int(C.w);
-    // the leaf's box, centre -/+ r as the refit forms it
-    const float4 qMin = make_float4(C.x - ph.r, C.y - ph.r, C.z - ph.r, 0.0f);
-    const float4 qMax = make_float4(C.x + ph.r, C.y + ph.r, C.z + ph.r, 0.0f);
-    const f3 pa = xyz(C), va = xyz(Vq);
-    const int orig = sIdx[ii];
-    f3 F = mk3(0.f, 0.f, 0.f);
-    int cnt = 0;
-    bool ovf = false;   // this lane's packet hit the stack bound: nothing is written for it
-    const int s = FOREST ? __float_as_int(Vq.w) : 0;
-    const int myRoot = FOREST ? sceneRoot[s] : (n >= 2 ? n : -1);
-    // the packet's lanes whose root has not been walked yet; node < 0: no walk under way
-    unsigned long long pending = __ballot(valid && myRoot >= n) & pmask;
-    int root = -1, node = -1, sp = 0;
-    if (!FOREST && pending != 0ull) {
-        root = node = n;
-        pending = 0ull;
+    LeafQuery q;
+    q.i = i;
+    q.ra = __float_as_int(C.w);
+    q.pa = xyz(C);
+    q.va = xyz(Vq);
+    if (leafBounds) {
+        q.qMin = leafBounds[2 * (size_t)ii];
+        q.qMax = leafBounds[2 * (size_t)ii + 1];
+    } else {   // centre -/+ r as the refit forms it
+        q.qMin = make_float4(C.x - ph.r, C.y - ph.r, C.z - ph.r, 0.0f);
+        q.qMax = make_float4(C.x + ph.r, C.y + ph.r, C.z + ph.r, 0.0f);
     }
-    const unsigned *words = reinterpret_cast<const unsigned *>(packed);
-    // The next node's record is requested as soon as the next node is known (from the overlap tests and
-    // the stack), before this node's leaf children are tested, so that its load overlaps theirs.
-    unsigned wn = node >= 0 ? words[16 * (size_t)(node - n) + pl] : 0u;
+    const int orig = sIdx[ii];
+    const int s = FOREST ? __float_as_int(Vq.w) : 0;
+    const int myRoot = !valid ? -1 : FOREST ? sceneRoot[s] : (n >= 2 ? n : -1);
+    LeafSum acc{mk3(0.f, 0.f, 0.f), 0};
+    bool ovf = false;
+
 #ifdef ARSIM_TRAVERSAL_STATS
-    const bool packetUsed = pending != 0ull || node >= 0;
-    unsigned long long stVisits = 0, stLeafTests = 0, stInterest = 0, stContacts = 0, stIters = 0;
-    int stMaxSp = 0;
+    unsigned long long stNodes = 0, stTests = 0, stReach = 0, stContacts = 0, stSteps = 0;
+    int stMaxSize = 0;
+    const bool packetUsed = row_ballot(myRoot >= n) != 0u;
 #endif
-    while (true) {
-        bool fresh = false;   // a walk that starts here: its root's record is not requested yet
-        if (FOREST) {
-            // a packet without a walk starts the next pending root (all lanes take part in the exchange)
-            const bool needRoot = node < 0 && pending != 0ull;
-            const int first = needRoot ? __builtin_ctzll(pending) : lane;
-            const int cand = __shfl(myRoot, first, 64);
-            if (needRoot) {
-                root = cand;
-                node = cand;
-                sp = 0;
-                fresh = true;
+    unsigned pending = row_ballot(myRoot >= n);   // the packet's lanes whose root has not been walked yet
+    while (__any(pending != 0u)) {
+        const int root = __shfl(myRoot, pending ? __builtin_ctz(pending) : 0, kPacketLanes);
+        const bool act = pending != 0u && valid && myRoot == root;
+        int size = pending != 0u ? 1 : 0, ncand = 0;
+        pending &= ~row_ballot(act);
+        if (pl == 0) list[0] = root;
+
+        Box6 A, Bx;   // the packet's two boxes
+        {
+            const float e[6] = {q.qMin.x, q.qMin.y, q.qMin.z, -q.qMax.x, -q.qMax.y, -q.qMax.z};
+            const float inf = __int_as_float(0x7f800000);
+            float pre[6], suf[6], cost = 1.f, costB = 1.f;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+                const float x = act ? e[k] : inf;
+                pre[k] = row_scan_min<true>(x);
+                suf[k] = __int_as_float(__builtin_amdgcn_update_dpp(
+                    0x7f800000, __float_as_int(row_scan_min<false>(x)), 0x101, 0xf, 0xf, false));   // of the lanes after
             }
-            pending &= ~(__ballot(needRoot && valid && myRoot == cand) & pmask);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                cost *= fmaxf(-pre[k + 3] - pre[k], 0.f) + 2.f * ph.r;
+                costB *= fmaxf(-suf[k + 3] - suf[k], 0.f) + 2.f * ph.r;
+            }
+            if (pl < kPacketLanes - 1) cost += costB;
+            float best = cost;
+#pragma unroll
+            for (int d = 1; d < kPacketLanes; d <<= 1) best = fminf(best, __shfl_xor(best, d, kPacketLanes));
+            const unsigned at = row_ballot(cost == best);
+            const int k0 = at ? __builtin_ctz(at) : kPacketLanes - 1;   // (no lane: NaN costs)
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+                A.v[k] = __shfl(pre[k], k0, kPacketLanes);
+                Bx.v[k] = __shfl(suf[k], k0, kPacketLanes);
+            }
         }
-        if (__ballot(node >= 0) == 0ull) break;
-        const bool live = node >= 0;
+
+        // the candidates, 32 per round: their centres into LDS, a bit per candidate in the lane's reach, then
+        // the lane's contacts two at a time
+        auto test_candidates = [&]() {
+            for (int b = 0; __any(b < ncand); b += kCandRound) {
+                const int left = ncand - b < kCandRound ? ncand - b : kCandRound;   // (negative: none)
+                __builtin_amdgcn_wave_barrier();
+                if (pl < left) stage[pl] = cms[cand[b + pl]];
+                if (pl + kPacketLanes < left) stage[pl + kPacketLanes] = cms[cand[b + pl + kPacketLanes]];
+                __builtin_amdgcn_wave_barrier();
+                unsigned hits = 0u;
+                for (int k = 0; __any(k < left); k += kCandStep) {
+#pragma unroll
+                    for (int u = 0; u < kCandStep; ++u)   // (past the end: old centres, masked below)
+                        hits |= candidate(stage[k + u], q.pa, q.ra, false, ph) ? 1u << (k + u) : 0u;
+                }
+                if (left < kCandRound) hits &= left > 0 ? (1u << left) - 1u : 0u;
+                if (!act) hits = 0u;
 #ifdef ARSIM_TRAVERSAL_STATS
-        ++stIters;
-        if (live) ++stVisits;
+                if (act && left > 0) {
+                    stTests += (unsigned long long)left;
+                    stReach += (unsigned long long)__popc(hits);
+                    for (int k = 0; k < left; ++k)
+                        if ((hits >> k & 1u) && cand[b + k] != i && in_contact(q.pa, xyz(stage[k]), ph)) ++stContacts;
+                }
 #endif
-        const unsigned w = fresh ? words[16 * (size_t)(node - n) + pl] : wn;
-        const float4 a0 = make_float4(row_word<0>(w), row_word<1>(w), row_word<2>(w), 0.f);
-        const float4 a1 = make_float4(row_word<4>(w), row_word<5>(w), row_word<6>(w), 0.f);
-        const float4 b0 = make_float4(row_word<8>(w), row_word<9>(w), row_word<10>(w), 0.f);
-        const float4 b1 = make_float4(row_word<12>(w), row_word<13>(w), row_word<14>(w), 0.f);
-        const int L = __float_as_int(row_word<3>(w)), R = __float_as_int(row_word<7>(w));
-        const bool act = live && valid && myRoot == root;
-        const bool oL = act & (L != i) & overlap(qMin, qMax, a0, a1);
-        const bool oR = act & (R != i) & overlap(qMin, qMax, b0, b1);
-        const bool tL = L >= n && (__ballot(oL) & pmask) != 0ull;
-        const bool tR = R >= n && (__ballot(oR) & pmask) != 0ull;
-#ifdef ARSIM_TRAVERSAL_STATS
-        stLeafTests += (L < n && oL ? 1 : 0) + (R < n && oR ? 1 : 0);
-        if (L < n && oL && in_contact(pa, xyz(cms[L]), ph)) ++stContacts;
-        if (R < n && oR && in_contact(pa, xyz(cms[R]), ph)) ++stContacts;
-        if (L >= n) stInterest += (unsigned long long)__popcll(__ballot(oL) & pmask);
-        if (R >= n) stInterest += (unsigned long long)__popcll(__ballot(oR) & pmask);
-        if (live && tL && tR) stMaxSp = sp + 1 > stMaxSp ? sp + 1 : stMaxSp;
-#endif
-        // next node: the left child entered (the right one pushed when both are), else the right one,
-        // else the top of the stack; selects rather than branches (every value is uniform in a packet)
-        const bool both = tL && tR, full = both && sp == kWaveStackDepth;
-        const int top = stack[sp > 0 ? sp - 1 : 0];
-        if (live && full && act) {
-            atomicOr(overflow, 1);
-            ovf = true;
-        }
-        if (live && both && !full && pl == 0) stack[sp] = R;
-        const int next = full ? -1 : (tL ? L : (tR ? R : (sp > 0 ? top : -1)));
-        const int dsp = (both && !full) ? 1 : ((!tL && !tR && sp > 0) ? -1 : 0);
-        node = live ? next : node;
-        sp = live ? sp + dsp : sp;
-        wn = node >= 0 ? words[16 * (size_t)(node - n) + pl] : 0u;
-        // both leaf children's centres requested before either is tested (one round trip, not two)
-        const bool hL = L < n && oL, hR = R < n && oR;
-        float4 CL, CR;
-        if (hL) CL = cms[L];
-        if (hR) CR = cms[R];
-        if (hL) {
-            if (candidate(CL, pa, ra, false, ph)) {
-                if (EMIT) {
-                    if (in_contact(pa, xyz(CL), ph)) {
-                        if (cnt < o.maxPer) o.pairs[(size_t)orig * o.maxPer + cnt] = sIdx[L];
-                        ++cnt;
+                while (hits) {
+                    const int k0 = __builtin_ctz(hits);
+                    hits &= hits - 1u;
+                    const bool two = hits != 0u;
+                    const int k1 = two ? __builtin_ctz(hits) : k0;
+                    hits &= hits - 1u;
+                    const int ja = cand[b + k0], jb = cand[b + k1];
+                    const float4 Va = EMIT ? stage[k0] : sVel[ja], Vb = EMIT ? stage[k1] : sVel[jb];
+                    bool oka = ja != i, okb = two && jb != i;
+                    if (leafBounds) {   // the caller's boxes need not be centre -/+ this radius
+                        oka = oka && overlap(q.qMin, q.qMax, leafBounds[2 * (size_t)ja], leafBounds[2 * (size_t)ja + 1]);
+                        okb = okb && overlap(q.qMin, q.qMax, leafBounds[2 * (size_t)jb], leafBounds[2 * (size_t)jb + 1]);
                     }
-                } else {
-                    f3 fj;
-                    if (pair_force(pa, xyz(CL), va, xyz(sVel[L]), ph, fj)) F = add3(F, fj);
+                    if (oka) leaf_contact<EMIT>(ja, stage[k0], Va, q, ph, o, sIdx, orig, acc);
+                    if (okb) leaf_contact<EMIT>(jb, stage[k1], Vb, q, ph, o, sIdx, orig, acc);
                 }
             }
-        }
-        if (hR) {
-            if (candidate(CR, pa, ra, false, ph)) {
-                if (EMIT) {
-                    if (in_contact(pa, xyz(CR), ph)) {
-                        if (cnt < o.maxPer) o.pairs[(size_t)orig * o.maxPer + cnt] = sIdx[R];
-                        ++cnt;
+            ncand = 0;
+        };
+
+        while (true) {
+            const bool more = __any(size > 0);
+            if (more) {
+                __builtin_amdgcn_wave_barrier();
+                const int most = size + kPacketLanes <= kFrontWide ? kPacketLanes : 1;
+                const int k = size < most ? size : most;
+#ifdef ARSIM_TRAVERSAL_STATS
+                ++stSteps;
+                stMaxSize = size > stMaxSize ? size : stMaxSize;
+                stNodes += (unsigned long long)__popc(row_ballot(pl < k && list[size - 1 - (pl < k ? pl : 0)] >= n));
+#endif
+                int L = -1, R = -1;
+                if (pl < k) {
+                    const int e = list[size - 1 - pl];
+                    L = e;
+                    if (e >= n) {
+                        float4 a0, a1, b0, b1;
+                        nodes.load(e, L, R, a0, a1, b0, b1);
+                        const bool lA = box_meets(A, a0, a1), lB = box_meets(Bx, a0, a1);
+                        const bool rA = box_meets(A, b0, b1), rB = box_meets(Bx, b0, b1);
+                        if (!(lA || lB)) L = -1;
+                        if (!(rA || rB)) R = -1;
+                        if (L >= n && R >= 0 && R < n) {   // a leaf is met before the inner child is entered
+                            const int x = L;
+                            L = R;
+                            R = x;
+                        }
                     }
+                }
+                // the children met, in order: out entries, the first `lead` of them leaves before any inner node
+                const unsigned mL = row_ballot(L >= 0), mR = row_ballot(R >= 0);
+                const unsigned mIn = row_ballot(L >= n || R >= n), mLeaf = row_ballot(L >= 0 && L < n);
+                const int at = __popc(mL & lower) + __popc(mR & lower);
+                const int out = __popc(mL) + __popc(mR);
+                int lead = out;
+                if (mIn) {
+                    const int f = __builtin_ctz(mIn);
+                    const unsigned below = (1u << f) - 1u;
+                    lead = __popc(mL & below) + __popc(mR & below) + (int)((mLeaf >> f) & 1u);
+                }
+                const int left = size - k + out - lead;
+                const bool full = left > kFrontCap;
+                if (!full) {
+                    auto put = [&](int r, int node) {
+                        if (r < lead) cand[ncand + r] = node;
+                        else list[left - 1 - (r - lead)] = node;
+                    };
+                    if (L >= 0) put(at, L);
+                    if (R >= 0) put(at + (L >= 0 ? 1 : 0), R);
+                    size = left;
+                    ncand += lead;
                 } else {
-                    f3 fj;
-                    if (pair_force(pa, xyz(CR), va, xyz(sVel[R]), ph, fj)) F = add3(F, fj);
+                    if (act) {
+                        atomicOr(overflow, 1);
+                        ovf = true;
+                    }
+                    size = 0;
                 }
             }
+            if (!more || __any(ncand > kCandCap - 2 * kPacketLanes)) test_candidates();
+            if (!more) break;
         }
     }
 #ifdef ARSIM_TRAVERSAL_STATS
     {
-        // per-lane leaf tests and contacts summed over the wave; the packet counts from each packet's
-        // first lane, the wave counts from lane 0 (stInterest and stVisits are packet-uniform)
-        unsigned long long lt = stLeafTests, ct = stContacts;
+        // per-lane counts summed over the wave; the packet counts from each packet's first lane (they are
+        // uniform in a packet), the wave counts from lane 0
+        unsigned long long lt = stTests, rt = stReach, ct = stContacts;
         for (int off = 32; off >= 1; off >>= 1) {
             lt += __shfl_xor(lt, off, 64);
+            rt += __shfl_xor(rt, off, 64);
             ct += __shfl_xor(ct, off, 64);
         }
         const unsigned long long lanes = (unsigned long long)__popcll(__ballot(valid));
         const unsigned long long done = (unsigned long long)__popcll(__ballot(valid && !ovf));
         if (pl == 0 && packetUsed) {
-            atomicAdd(&g_travStats[1], stVisits);
-            atomicAdd(&g_travStats[4], stInterest);
-            atomicMax(&g_travStats[5], (unsigned long long)stMaxSp);
+            atomicAdd(&g_travStats[1], stNodes);
+            atomicMax(&g_travStats[5], (unsigned long long)stMaxSize);
             atomicAdd(&g_travStats[8], 1ull);
         }
-        if (lane == 0) {
+        if ((threadIdx.x & 63u) == 0u) {
             atomicAdd(&g_travStats[0], 1ull);
             atomicAdd(&g_travStats[2], lanes);
             atomicAdd(&g_travStats[3], lt);
+            atomicAdd(&g_travStats[4], rt);
             atomicAdd(&g_travStats[6], done);
             atomicAdd(&g_travStats[7], ct);
-            atomicAdd(&g_travStats[9], stIters);
+            atomicAdd(&g_travStats[9], stSteps);
         }
     }
 #endif
     if (!valid || ovf) return;
     if (EMIT) {
-        o.counts[orig] = cnt;
+        o.counts[orig] = acc.cnt;
         return;
     }
     SceneGeom g;
     if (FOREST) g = sv.table[s];
     else g = sv.single;
-    if (!((ph.flags & kGrainClamp) && ra < 0)) F = add3(F, wall_force(pa, va, ph, g));
-    if (ra >= 0) {
+    f3 F = acc.F;
+    if (!((ph.flags & kGrainClamp) && q.ra < 0)) F = add3(F, wall_force(q.pa, q.va, ph, g));
+    if (q.ra >= 0) {
         o.pForce[orig] = f4(F, 0.0f);
         if (o.pTorque) o.pTorque[orig] = f4(cross3(xyz(o.relPos[orig]), F), 0.0f);
     } else {
         const float fs = (ph.flags & kRefUnits) ? 1.0f : ph.dt;
-        o.vel[orig] = make_float4(va.x + F.x * fs, va.y + F.y * fs, va.z + F.z * fs, 0.0f);
+        o.vel[orig] = make_float4(q.va.x + F.x * fs, q.va.y + F.y * fs, q.va.z + F.z * fs, 0.0f);
     }
 }
 
@@ -906,34 +954,31 @@ void launch_lbvh_bounds(const Lbvh &t, int n, float radius, hipStream_t st) {
 
 void launch_dem_lbvh(const int *sortedIdx, const Lbvh &t, int n, const DevPhys &ph, const SceneView &sv,
                      bool sceneInVelW, const DemOut &o, int block, hipStream_t st, int *overflow) {
+    (void)sceneInVelW;
     if (n <= 0) return;
     if (block <= 0) block = 128;
-    dim3 grid((n + block - 1) / block);
-    if (t.packed) {
-        // packets of 16 lanes, one scene or a forest (whose scene ids ride in sortedVel.w)
-        block = (block + 63) & ~63;
-        grid = dim3((n + block - 1) / block);
-        const size_t pl = (size_t)kWaveStackDepth * (block / kPacketLanes) * sizeof(int);
-        auto run = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, grid, dim3(block), pl, st, sortedIdx, t.packed, t.cms, t.sortedVel, t.sceneRoot, n,
-                               ph, sv, o, overflow);
-        };
-        if (t.sceneRoot) {
-            if (o.pairs) run(k_dem_lbvh_packets<true, true>);
-            else run(k_dem_lbvh_packets<false, true>);
-        } else {
-            if (o.pairs) run(k_dem_lbvh_packets<true, false>);
-            else run(k_dem_lbvh_packets<false, false>);
-        }
+    block = (block + 63) & ~63;
+    const dim3 grid((n + block - 1) / block);
+    const size_t lds = (size_t)(block / kPacketLanes) * kPacketLds * sizeof(float4);
+    const float4 *leafBounds = t.packed ? nullptr : t.bounds;
+    auto run = [&](auto kernel, auto nodes) {
+        hipLaunchKernelGGL(kernel, grid, dim3(block), lds, st, sortedIdx, nodes, t.cms, t.sortedVel, leafBounds, t.sceneRoot,
+                           n, ph, sv, o, overflow);
+    };
+    if (!t.packed) {
+        const RefNodes nodes{t.left, t.right, t.bounds};
+        if (o.pairs) run(k_dem_lbvh<true, false, RefNodes>, nodes);
+        else run(k_dem_lbvh<false, false, RefNodes>, nodes);
         return;
     }
-    size_t lds = (size_t)kStackDepth * block * sizeof(int);
-    if (o.pairs)
-        hipLaunchKernelGGL(k_dem_lbvh<true>, grid, dim3(block), lds, st, sortedIdx, t, n, ph, sv, sceneInVelW ? 1 : 0,
-                           o, overflow);
-    else
-        hipLaunchKernelGGL(k_dem_lbvh<false>, grid, dim3(block), lds, st, sortedIdx, t, n, ph, sv,
-                           sceneInVelW ? 1 : 0, o, overflow);
+    const PackedNodes nodes{t.packed, n};
+    if (t.sceneRoot) {
+        if (o.pairs) run(k_dem_lbvh<true, true, PackedNodes>, nodes);
+        else run(k_dem_lbvh<false, true, PackedNodes>, nodes);
+    } else {
+        if (o.pairs) run(k_dem_lbvh<true, false, PackedNodes>, nodes);
+        else run(k_dem_lbvh<false, false, PackedNodes>, nodes);
+    }
 }
 
 }  // namespace arsim
