@@ -1,5 +1,7 @@
 // body.hip -- rigid-body integration, particle pose / grain integration with key generation,
 // the segmented per-body reduction, and small utility kernels.
+#include <algorithm>
+
 #include "kernels.hpp"
 #include "reduce_apply.hpp"
 
@@ -593,6 +595,21 @@ __global__ void k_iota_ranges(const int4 *__restrict__ ranges, int numRanges, in
     }
 }
 
+// One range per blockIdx.y, 16 bytes a lane where the range allows it.  Writes host memory over PCIe: a scene's
+// state in one launch and one wait, where a copy call per array costs about 18 us whatever its size.
+__global__ __launch_bounds__(256) void k_fetch(FetchJobs jobs, unsigned *__restrict__ dst) {
+    const int k = (int)blockIdx.y;
+    const unsigned *src = jobs.src[k];
+    unsigned *out = dst + jobs.at[k];
+    const unsigned words = jobs.words[k], t = blockIdx.x * 256u + threadIdx.x, stride = gridDim.x * 256u;
+    if ((reinterpret_cast<uintptr_t>(src) & 15u) == 0u && (words & 3u) == 0u) {
+        for (unsigned w = t; w < words / 4u; w += stride)
+            reinterpret_cast<uint4 *>(out)[w] = reinterpret_cast<const uint4 *>(src)[w];
+        return;
+    }
+    for (unsigned w = t; w < words; w += stride) out[w] = src[w];
+}
+
 __global__ void k_fill_u16(uint16_t *p, uint16_t v, size_t n) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -660,6 +677,13 @@ void launch_iota_ranges(const int4 *ranges, int numRanges, int *dst, hipStream_t
     if (numRanges <= 0) return;
     hipLaunchKernelGGL(k_iota_ranges, dim3((unsigned)(numRanges < 4096 ? numRanges : 4096)), dim3(256), 0, st, ranges, numRanges,
                        dst);
+}
+
+void launch_fetch(const FetchJobs &jobs, unsigned *dst, hipStream_t st) {
+    unsigned most = 1u;
+    for (int k = 0; k < jobs.n; ++k) most = std::max(most, jobs.words[k]);
+    const unsigned blocks = std::min((most + 1023u) / 1024u, 256u);
+    hipLaunchKernelGGL(k_fetch, dim3(blocks, (unsigned)jobs.n), dim3(256), 0, st, jobs, dst);
 }
 
 void launch_fill_u16(uint16_t *p, uint16_t value, size_t count, hipStream_t st) {

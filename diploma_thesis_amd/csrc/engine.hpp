@@ -109,6 +109,16 @@ struct Engine {
     hipGraphExec_t gexec = nullptr;
     bool graphReady = false;
 
+    // pinned host memory that small reads of the state come through (allocated at the first one)
+    unsigned *fetchBuf = nullptr;
+    struct Fetch {
+        void *dst;
+        const void *src;
+        size_t bytes;           // a multiple of 4
+    };
+    // Waits for the steps enqueued so far and copies the device ranges to host memory.
+    int fetch(const std::vector<Fetch> &what);
+
     ~Engine();
     int build(const std::vector<SceneSource> &src, const ArSimTuning *tuning, int dev, hipStream_t stream);
     int enqueue_step(hipEvent_t *ev, int *numStages);

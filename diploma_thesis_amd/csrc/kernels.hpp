@@ -103,6 +103,14 @@ int  aabb_max_partials();
 void launch_check_finite(const float4 *a, int n, int *flag, hipStream_t st);
 // dst[i] = src[i] + delta for src[i] >= 0, else src[i] (rebases body indices when scenes move).
 void launch_copy_offset(int *dst, const int *src, int n, int delta, hipStream_t st);
+// Several device ranges copied into one host-visible buffer (4-byte words, each range at a multiple of 4 words).
+constexpr int kFetchMax = 12;
+struct FetchJobs {
+    const unsigned *src[kFetchMax];
+    unsigned words[kFetchMax], at[kFetchMax];
+    int n;
+};
+void launch_fetch(const FetchJobs &jobs, unsigned *dst, hipStream_t st);
 void launch_fill_u16(uint16_t *p, uint16_t value, size_t count, hipStream_t st);
 // dst[r.x + k] = r.y + k for every range r = (first destination, first value, count).
 void launch_iota_ranges(const int4 *ranges, int numRanges, int *dst, hipStream_t st);
