@@ -631,8 +631,7 @@ __device__ __forceinline__ unsigned row_ballot(bool p) {
 // leaf, 278 -> 117 us on the reference's arrays at a pile of 100,003.
 // The packet's reach is two boxes, the joint boxes of its leaves before and after the split that makes
 // them smallest: the 16 leaves of a Morton run often lie on both sides of a split of the tree, far
-// apart, where one box would take in everything between.  (With one box a packet in five overran a list
-// twice as long.  Every box that a lane's own box meets meets
+// apart, where one box would take in everything between.  (Every box that a lane's own box meets meets
 // one of them, and the contact test rejects what only the packet reaches.)
 // A packet's LDS: a list of 128 entries before the narrow steps made the pile's 262 us frame 362; registers are
 // held to five waves per SIMD, the most without spills (six and seven: within 2 %).
