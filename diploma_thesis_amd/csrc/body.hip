@@ -1,6 +1,7 @@
 // body.hip -- rigid-body integration, particle pose / grain integration with key generation,
 // the segmented per-body reduction, and small utility kernels.
 #include <algorithm>
+#include <type_traits>
 
 #include "kernels.hpp"
 #include "reduce_apply.hpp"
@@ -752,28 +753,19 @@ void launch_pose_key_tiles(const PartBufs &p, const BodyBufs &b, int numParticle
     if (numParticles <= 0) return;
     const int g = grainVelDead ? 1 : 0;
     const dim3 grid(to.numTiles);
-    if (to.morton == 2) {   // 63-bit Morton codes: tiles ranked by the top 10 bits
-        hipLaunchKernelGGL((k_pose_key_tiles<kKeyMorton63, 1024, 10>), grid, dim3(1024), 0, st, p, b, numParticles, ph,
-                           sv, to, g);
-        return;
-    }
-    if (to.morton) {   // 30-bit Morton keys, buckets of their top 10 bits
-        hipLaunchKernelGGL((k_pose_key_tiles<kKeyMorton30, 1024, 10>), grid, dim3(1024), 0, st, p, b, numParticles, ph,
-                           sv, to, g);
-        return;
-    }
-    if (to.tileKeys == 1024)
-        hipLaunchKernelGGL((k_pose_key_tiles<kKeyGrid, 256, 8>), grid, dim3(256), 0, st, p, b, numParticles, ph, sv, to,
-                           g);
-    else if (to.bucketBits <= 8)
-        hipLaunchKernelGGL((k_pose_key_tiles<kKeyGrid, 1024, 8>), grid, dim3(1024), 0, st, p, b, numParticles, ph, sv,
-                           to, g);
-    else if (to.bucketBits == 9)
-        hipLaunchKernelGGL((k_pose_key_tiles<kKeyGrid, 1024, 9>), grid, dim3(1024), 0, st, p, b, numParticles, ph, sv,
-                           to, g);
-    else
-        hipLaunchKernelGGL((k_pose_key_tiles<kKeyGrid, 1024, 10>), grid, dim3(1024), 0, st, p, b, numParticles, ph, sv,
-                           to, g);
+    auto run = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, st, p, b, numParticles, ph, sv, to, g);
+    };
+    auto of_mode = [&](auto mode) {
+        constexpr int M = decltype(mode)::value;
+        if (to.tileKeys == 1024) run(k_pose_key_tiles<M, 256, 8>, 256);
+        else if (to.bucketBits <= 8) run(k_pose_key_tiles<M, 1024, 8>, 1024);
+        else if (to.bucketBits == 9) run(k_pose_key_tiles<M, 1024, 9>, 1024);
+        else run(k_pose_key_tiles<M, 1024, 10>, 1024);
+    };
+    if (to.morton == 2) of_mode(std::integral_constant<int, kKeyMorton63>{});
+    else if (to.morton) of_mode(std::integral_constant<int, kKeyMorton30>{});
+    else of_mode(std::integral_constant<int, kKeyGrid>{});
 }
 
 void launch_reduce_apply(const float4 *pForce, const float4 *pTorque, const float4 *relPos, const BodyBufs &b,

@@ -80,6 +80,16 @@ struct LdsItems {
     __device__ unsigned digit(int i, int shift, unsigned mask) const { return (a[i] >> shift) & mask; }
     __device__ void move_to(const LdsItems &dst, int pos, int i) const { dst.a[pos] = a[i]; }
 };
+// Keys wider than a packed word's offset: the key and its position in the bucket in two arrays.
+struct LdsPairs {
+    unsigned *k;
+    unsigned short *p;
+    __device__ unsigned digit(int i, int shift, unsigned mask) const { return (k[i] >> shift) & mask; }
+    __device__ void move_to(const LdsPairs &dst, int pos, int i) const {
+        dst.k[pos] = k[i];
+        dst.p[pos] = p[i];
+    }
+};
 struct GlobalItems {
     unsigned *k, *v;
     __device__ unsigned digit(int i, int shift, unsigned mask) const { return (k[i] >> shift) & mask; }
@@ -157,14 +167,21 @@ __device__ __forceinline__ void block_fill(unsigned *table, unsigned long long a
 // POSBITS: bits of a bucket position in the packed LDS words (the offset from c0 takes the other 32 -
 // POSBITS; a bucket sorted in LDS holds at most 2^POSBITS keys).  REORDER: also the gathered sorted
 // copies and the cell table (grid keys); without it only the sorted keys and indices (Morton keys,
-// whose sorted-copy arrays are then only the global fallback's second buffer).
+// whose sorted-copy arrays are then only the global fallback's second buffer).  WIDE (Morton keys of scenes
+// with few particles, whose buckets span more than 2^(32 - POSBITS) codes, and 2^20 keys in 512 buckets
+// instead of 1,024: the LBVH30 step 342 -> 328 us): key and position apart.
+// kOut64 (a forest's Morton keys): the sorted keys as scene << 30 | code there instead of in kOut.
 // Eight waves per SIMD (two workgroups per CU): registers are held to that occupancy.
-template <int POSBITS, bool REORDER>
+template <int POSBITS, bool REORDER, bool WIDE>
 __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_bucket_sort(
     TileKeyOut to, int split, unsigned *__restrict__ kOut, unsigned *__restrict__ vOut,
     const float4 *__restrict__ rec, float4 *__restrict__ sPos, float4 *__restrict__ sVel,
-    unsigned *__restrict__ table, unsigned numCells) {
-    __shared__ unsigned sA[kBkCap], sB[kBkCap];
+    unsigned *__restrict__ table, unsigned numCells, uint64_t *__restrict__ kOut64) {
+    constexpr int kCap = kBkCap < (1 << POSBITS) ? kBkCap : (1 << POSBITS);
+    constexpr int kLds = WIDE ? kCap : kBkCap;
+    static_assert(!(WIDE && REORDER), "grid keys fit the packed words");
+    __shared__ unsigned sA[kLds], sB[kLds];
+    __shared__ unsigned short sPosA[WIDE ? kCap : 1], sPosB[WIDE ? kCap : 1];
     __shared__ unsigned sCur[kBkWaves][256];
     __shared__ unsigned sWave[kBkWaves];
     __shared__ unsigned sOff[kBkMaxTiles], sSrc[kBkMaxTiles];   // tile map: bucket offset and source slot
@@ -184,7 +201,6 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
     const unsigned tileWord = t < numTiles ? to.info[(size_t)bs.infoBase + (size_t)j * numTiles + t] : 0u;
     const unsigned start = bs.pStart + block_sum(hPrev, sWave);
     const int cnt = (int)hist[j];
-    constexpr int kCap = kBkCap < (1 << POSBITS) ? kBkCap : (1 << POSBITS);
     constexpr unsigned kPosMask = (1u << POSBITS) - 1u;
     const bool inLds = cnt <= kCap;
     // a bucket too large for LDS is sorted in global memory by its first workgroup alone
@@ -242,6 +258,11 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
         }
     };
     const unsigned base = (unsigned)c0;
+    const uint64_t sceneKey = (uint64_t)(unsigned)to.bucketScene[g] << 30;
+    auto store_key = [&](int i, unsigned key) {
+        if (!REORDER && kOut64) kOut64[start + i] = sceneKey | key;
+        else kOut[start + i] = key;
+    };
     if (inLds) {
         // every slot found first (LDS only), then every key and value load in flight at once; the
         // values wait in registers while the keys are sorted, then go to the buffer the sort left free,
@@ -262,17 +283,30 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
             const int i = t + q * kBkThreads;
-            if (i < cnt) sA[i] = ((kv[q] - base) << POSBITS) | (unsigned)i;
+            if (i < cnt) {
+                if (WIDE) {
+                    sA[i] = kv[q] - base;
+                    sPosA[i] = (unsigned short)i;
+                } else {
+                    sA[i] = ((kv[q] - base) << POSBITS) | (unsigned)i;
+                }
+            }
         }
         __syncthreads();
         unsigned *src = sA, *dst = sB;
+        unsigned short *srcP = sPosA, *dstP = sPosB;
         for (int sh = 0; sh < lowBits; sh += 8) {
-            stable_pass(LdsItems{src}, LdsItems{dst}, cnt, POSBITS + sh, min(8, lowBits - sh), sCur, sWave);
+            const int bits = min(8, lowBits - sh);
+            if (WIDE) stable_pass(LdsPairs{src, srcP}, LdsPairs{dst, dstP}, cnt, sh, bits, sCur, sWave);
+            else stable_pass(LdsItems{src}, LdsItems{dst}, cnt, POSBITS + sh, bits, sCur, sWave);
             unsigned *x = src;
             src = dst;
             dst = x;
+            unsigned short *y = srcP;
+            srcP = dstP;
+            dstP = y;
         }
-        const unsigned *sorted = src;   // packed words in sorted order
+        const unsigned *sorted = src;   // packed words (WIDE: offsets from c0) in sorted order
         unsigned *valAt = dst;          // valAt[i]: the value of the bucket's i-th key in gather order
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
@@ -280,6 +314,13 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
             if (i < cnt) valAt[i] = vv[q];
         }
         __syncthreads();
+        if (WIDE) {
+            for (int i = i0 + t; i < i1; i += kBkThreads) {
+                store_key(i, base + sorted[i]);
+                vOut[start + i] = valAt[srcP[i]];
+            }
+            return;
+        }
         // the gathers of the first two rounds of positions are issued before the table is filled, so
         // that their latency overlaps the table's stores; a lane past the part's end loads sorted
         // position 0 (the bucket is not empty) and stores nothing, so the loads need no branch
@@ -296,7 +337,7 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
             fill_table([&](int i) -> unsigned { return sorted[i] >> POSBITS; });
         }
         if (ha) {
-            kOut[start + ia] = base + (wa >> POSBITS);
+            store_key(ia, base + (wa >> POSBITS));
             vOut[start + ia] = va;
             if (REORDER) {
                 sPos[start + ia] = pa;
@@ -304,7 +345,7 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
             }
         }
         if (hb) {
-            kOut[start + ib] = base + (wb >> POSBITS);
+            store_key(ib, base + (wb >> POSBITS));
             vOut[start + ib] = vb;
             if (REORDER) {
                 sPos[start + ib] = pb;
@@ -325,14 +366,14 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
                 P2 = rec[2 * (size_t)val2];
                 Q2 = rec[2 * (size_t)val2 + 1];
             }
-            kOut[start + i] = base + (w >> POSBITS);
+            store_key(i, base + (w >> POSBITS));
             vOut[start + i] = val;
             if (REORDER) {
                 sPos[start + i] = P;
                 sVel[start + i] = Q;
             }
             if (h2) {
-                kOut[start + i2] = base + (w2 >> POSBITS);
+                store_key(i2, base + (w2 >> POSBITS));
                 vOut[start + i2] = val2;
                 if (REORDER) {
                     sPos[start + i2] = P2;
@@ -375,7 +416,7 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
             fill_table([&](int i) -> unsigned { return kOut[start + i]; });
             __syncthreads();
         }
-        for (int i = t; i < cnt; i += kBkThreads) kOut[start + i] += base;
+        for (int i = t; i < cnt; i += kBkThreads) store_key(i, kOut[start + i] + base);
     }
 }
 
@@ -417,7 +458,8 @@ void launch_morton63_ties(const unsigned *k30, const unsigned *vIn, const uint64
     hipLaunchKernelGGL(k_morton63_ties, dim3((n + 255) / 256), dim3(256), 0, st, k30, vIn, code63, n, kOut, vOut);
 }
 
-bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *out, int maxShift, int capKeys) {
+bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *out, int maxShift, int capKeys,
+                      bool sharedCells) {
     const size_t S = shapes.size();
     long long nTot = 0, tiles4k = 0;
     for (const auto &sh : shapes) {
@@ -491,7 +533,7 @@ bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *o
         for (int k = 0; k < b.tiles; ++k) p.tileScene.push_back((int)s);
         for (int k = 0; k < b.buckets; ++k) p.bucketScene.push_back((int)s);
         pBase += n;
-        cBase += c;
+        if (!sharedCells) cBase += c;
         bBase += b.buckets;
         tBase += b.tiles;
         info += (long long)b.buckets * tiles;
@@ -506,15 +548,19 @@ bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *o
 void launch_bucket_sort(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, const float4 *rec, float4 *sortedPos,
                         float4 *sortedVel, unsigned *table, unsigned numCells, int split, hipStream_t st) {
     if (to.numBuckets <= 0) return;
-    hipLaunchKernelGGL((k_bucket_sort<16, true>), dim3(to.numBuckets * split), dim3(kBkThreads), 0, st, to, split, kOut,
-                       vOut, rec, sortedPos, sortedVel, table, numCells);
+    hipLaunchKernelGGL((k_bucket_sort<16, true, false>), dim3(to.numBuckets * split), dim3(kBkThreads), 0, st, to, split,
+                       kOut, vOut, rec, sortedPos, sortedVel, table, numCells, nullptr);
 }
 
 void launch_bucket_sort_morton(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, float4 *scratchA,
-                               float4 *scratchB, hipStream_t st) {
+                               float4 *scratchB, uint64_t *kOut64, int maxShift, hipStream_t st) {
     if (to.numBuckets <= 0) return;
-    hipLaunchKernelGGL((k_bucket_sort<12, false>), dim3(to.numBuckets), dim3(kBkThreads), 0, st, to, 1, kOut, vOut,
-                       nullptr, scratchA, scratchB, nullptr, 0u);
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(to.numBuckets), dim3(kBkThreads), 0, st, to, 1, kOut, vOut, nullptr, scratchA,
+                           scratchB, nullptr, 0u, kOut64);
+    };
+    if (maxShift <= 32 - 12) run(k_bucket_sort<12, false, false>);
+    else run(k_bucket_sort<12, false, true>);
 }
 
 }  // namespace arsim

@@ -369,16 +369,16 @@ std::vector<unsigned> bucket_peaks(const float *pos4, int n, const SceneGeom &g)
     return peak;
 }
 
-// The fullest bucket of a scene's 30-bit Morton codes by their top 10 bits (1,024 buckets), at index 20 of
-// the plan's per-shift peaks (other widths: UINT_MAX), from host positions normalised as the device does
-// (for planning only).
+// The fullest bucket of a scene's 30-bit Morton codes for every bucket width of 2^20 codes (1,024 buckets) to
+// 2^30 (one), at index b of the plan's per-shift peaks (narrower ones: UINT_MAX), from host positions
+// normalised as the device does (for planning only).
 std::vector<unsigned> morton_peaks(const float *pos4, int n, const SceneGeom &g) {
     auto spread = [](unsigned v) {   // bit k of v to bit 3k
         unsigned r = 0u;
         for (int k = 0; k < 10; ++k) r |= ((v >> k) & 1u) << (3 * k);
         return r;
     };
-    std::vector<unsigned> peak(21, 0xffffffffu), hist(1024, 0u);
+    std::vector<unsigned> peak(31, 0xffffffffu), hist(1024, 0u);
     for (int i = 0; i < n; ++i) {
         unsigned q[3];
         for (int a = 0; a < 3; ++a) {
@@ -389,8 +389,12 @@ std::vector<unsigned> morton_peaks(const float *pos4, int n, const SceneGeom &g)
         const unsigned code = spread(q[0]) * 4u + spread(q[1]) * 2u + spread(q[2]);
         ++hist[code >> 20];
     }
-    peak[20] = *std::max_element(hist.begin(), hist.end());
-    return peak;
+    for (int b = 20;; ++b) {
+        peak[b] = *std::max_element(hist.begin(), hist.end());
+        if (b == 30) return peak;
+        for (size_t k = 0; k < hist.size() / 2; ++k) hist[k] = hist[2 * k] + hist[2 * k + 1];
+        hist.resize(hist.size() / 2);
+    }
 }
 
 }  // namespace
@@ -534,22 +538,27 @@ int Engine::build(const std::vector<SceneSource> &src, const ArSimTuning *tuning
     } else if ((method == ARSIM_METHOD_LBVH30 || method == ARSIM_METHOD_LBVH63) && S == 1) {
         const bool m63 = method == ARSIM_METHOD_LBVH63;
         keyBits = m63 ? 63 : 30; keyBytes = m63 ? 8 : 4;
-        // the codes sorted per bucket of their top 10 bits (tiles of 4096, fixed Morton box): 1,024 buckets
-        // of 2^20 codes, a bucket's positions in 12 bits of an LDS word.  63-bit codes: the same sort of
-        // their top 30 bits (the 30-bit code), then the ties among equal top bits ranked by the full code
-        if (!(flags & ARSIM_DYNAMIC_AABB) && N > 65536) {
-            std::vector<BucketSceneShape> shapes(1);
-            shapes[0].particles = N;
-            shapes[0].grid[0] = shapes[0].grid[1] = shapes[0].grid[2] = 1024u;
-            if (src[0].host) shapes[0].peak = morton_peaks(src[0].host->pos, N, geoms[0]);
-            else if (src[0].from && src[0].from->mortonBucket) shapes[0].shift = 20;
-            mortonBucket = plan_bucket_sort(shapes, &bkPlan, 20, 4096) && bkPlan.scenes[0].shift == 20 &&
-                           bkPlan.tileKeys == kTileKeys;
-        }
     } else if (method == ARSIM_METHOD_LBVH63) {
         keyBits = 63; keyBytes = 8;   // a forest of 63-bit codes
     } else {
         keyBits = 30 + sceneBits; keyBytes = 8;
+    }
+    if ((method == ARSIM_METHOD_LBVH30 || (method == ARSIM_METHOD_LBVH63 && S == 1)) && !(flags & ARSIM_DYNAMIC_AABB)) {
+        // the codes (in each scene's fixed Morton box) sorted per bucket of 2^shift of them, at most 1,024
+        // buckets a scene.  63-bit codes: the same sort of their top 30 bits (the 30-bit code), then the
+        // ties among equal top bits ranked by the full code
+        // (against the onesweep passes, each a chain of tiles of about 11 us however few the keys: 50,021
+        // particles' 63-bit codes 90 -> 17 us and their step 198 -> 116, a forest of 48 scenes 93 -> 38 us
+        // and its step 334 -> 269, the body integration's launch among it)
+        std::vector<BucketSceneShape> shapes(S);
+        for (int s = 0; s < S; ++s) {
+            shapes[s].particles = pCount[s];
+            shapes[s].grid[0] = shapes[s].grid[1] = shapes[s].grid[2] = 1024u;
+            if (src[s].host) shapes[s].peak = morton_peaks(src[s].host->pos, pCount[s], geoms[s]);
+            else if (src[s].from && src[s].from->mortonBucket)
+                shapes[s].shift = src[s].from->bkPlan.scenes[src[s].fromScene].shift;
+        }
+        mortonBucket = plan_bucket_sort(shapes, &bkPlan, 30, 4096, true);
     }
 
     // ---- allocation (everything a step touches, once)
@@ -893,7 +902,7 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
         lastKeys = kA;
         lastIdx = vA;
     } else if (mortonBucket) {
-        // Morton codes ranked per tile by their top 10 bits in the pose kernel, then sorted per bucket
+        // Morton codes ranked per tile by bucket in the pose kernel, then sorted per bucket
         if (!ahead) {
             launch_body_integrate(bb, B, ph, &zHist, st);
             rec();
@@ -907,7 +916,14 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
         rec();
         // (the tree's leaf arrays are the second buffer of a bucket sorted in global memory; the refit
         // writes them afterwards)
-        launch_bucket_sort_morton(to, (unsigned *)keysA, valsA, tree.cms, tree.sortedVel, st);
+        int maxShift = 0;
+        for (const BucketScene &b : bkPlan.scenes) maxShift = std::max(maxShift, b.shift);
+        // a forest's keys are 64 bits wide: the tile keys fill half of keysB, the other half is the u32 scratch
+        if (S > 1)
+            launch_bucket_sort_morton(to, (unsigned *)keysB + N, valsA, tree.cms, tree.sortedVel, (uint64_t *)keysA,
+                                      maxShift, st);
+        else
+            launch_bucket_sort_morton(to, (unsigned *)keysA, valsA, tree.cms, tree.sortedVel, nullptr, maxShift, st);
         // 63-bit codes: sorted codes and indices into (keysB, valsB), the tile arrays being free now
         void *kS = keysA;
         unsigned *vS = valsA;
@@ -917,13 +933,13 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
             vS = valsB;
         }
         rec();
-        launch_lbvh_build(kS, keyBytes, N, 0, sceneStartD, sceneCountD, S, tree, st);
+        launch_lbvh_build(kS, keyBytes, N, S > 1 ? 30 : 0, sceneStartD, sceneCountD, S, tree, st);
         rec();
-        launch_lbvh_refit((const int *)vS, pos, vel, rb, nullptr, gatherRec, ph.r, N, tree, st);
+        launch_lbvh_refit((const int *)vS, pos, vel, rb, S > 1 ? scene : nullptr, gatherRec, ph.r, N, tree, st);
         rec();
         DemOut o{};
         o.pForce = pForce; o.vel = vel; o.relPos = relPos;
-        launch_dem_lbvh((const int *)vS, tree, N, ph, sv, false, o, tu.demBlock, st, overflowD);
+        launch_dem_lbvh((const int *)vS, tree, N, ph, sv, S > 1, o, tu.demBlock, st, overflowD);
         if (numStatic)
             launch_dem_static(tree.cms, tree.sortedVel, vS, N, stPos, stNorm, nullptr, stTable, nullptr, ph,
                               geoms[0], pForce, nullptr, relPos, false, st);

@@ -180,8 +180,9 @@ struct TileKeyOut {
     const int *tileScene, *bucketScene;   // scene of each tile and of each bucket
     int numTiles, numBuckets, tileKeys;
     int bucketBits;                       // a scene has at most 2^bucketBits buckets (8, 9 or 10)
-    // Morton keys (one scene, 1,024 buckets of 2^20 codes): 1 = 30-bit codes; 2 = 63-bit codes, whose
-    // top 30 bits (the 30-bit code) are the tile keys while the full codes go to code63 in particle order
+    // Morton keys (each scene's codes cut into buckets of 2^shift, 20 <= shift <= 30): 1 = 30-bit codes;
+    // 2 = 63-bit codes, whose top 30 bits (the 30-bit code) are the tile keys while the full codes go to
+    // code63 in particle order
     int morton = 0;
     uint64_t *code63 = nullptr;
 };
@@ -210,26 +211,28 @@ struct BucketPlan {
     int bucketBits = 8;   // the most buckets of one scene, rounded up to a power of two (at least 2^8)
 };
 // maxShift / capKeys: the widest bucket (2^maxShift cells) and the most keys a bucket sorted in LDS holds
-// (grid keys: 2^16 and 7,776; Morton keys: 2^20 and 4,096, bucket positions taking 12 bits of a word).
+// (grid keys: 2^16 and 7,776; Morton keys: 2^30 and 4,096).  sharedCells: every scene's keys lie in the same range (Morton codes) instead of one
+// scene's after another's.
 bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *out, int maxShift = 16,
-                      int capKeys = 7776);
+                      int capKeys = 7776, bool sharedCells = false);
 // The grid sort finished per bucket (bucket.hip): each bucket gathers its keys from its scene's
 // tiles' runs (tile order keeps the sort stable), `split` workgroups (1 or 2) sort it by the low bits,
 // each writing its share of the sorted keys / indices to (kOut, vOut), of the gathered sorted copies
 // and of the bucket's range of the exact cell table (whose last entry, numCells, the last bucket writes).
 void launch_bucket_sort(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, const float4 *rec, float4 *sortedPos,
                         float4 *sortedVel, unsigned *table, unsigned numCells, int split, hipStream_t st);
-// The same for 30-bit Morton keys ranked by their top 10 bits (TileKeyOut.morton): each bucket of up to
-// 4,096 keys sorted by its low 20 bits in LDS, written as sorted keys and indices only; a larger bucket is
-// sorted in global memory with scratchA / scratchB (16 B per key, N entries) as its second buffer.
 // The 63-bit order from the stable sort by the codes' top 30 bits: code63 is in particle order, k30 /
 // vIn the sorted top 30 bits and particle indices.  Writes the sorted 63-bit codes and indices; within
 // a run of equal top bits the members are ranked by their full codes, equal codes keeping the run's
 // (particle) order, so the result is the stable sort by the 63-bit code.
 void launch_morton63_ties(const unsigned *k30, const unsigned *vIn, const uint64_t *code63, int n, uint64_t *kOut,
                           unsigned *vOut, hipStream_t st);
+// The same for 30-bit Morton keys ranked per tile by bucket (TileKeyOut.morton): each bucket of up to 4,096
+// keys sorted by its low bits in LDS (maxShift: the widest scene's), written as sorted keys and indices
+// only; a larger bucket is sorted in global memory with scratchA / scratchB (16 B per key, N entries) as
+// its second buffer.  kOut64 (a forest): the keys as scene << 30 | code there, kOut being scratch.
 void launch_bucket_sort_morton(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, float4 *scratchA,
-                               float4 *scratchB, hipStream_t st);
+                               float4 *scratchB, uint64_t *kOut64, int maxShift, hipStream_t st);
 // Capacity of the long-run list of a table of tableSize entries (runs are disjoint and longer than
 // kLongRange), and the launch that fills the listed runs.
 unsigned fill_long_capacity(unsigned long long tableSize);

@@ -1,7 +1,8 @@
-"""The packet traversal of the LBVH contact kernel, bit for bit against the oracle: leaf counts around a packet and a
+"""The packet traversal of the LBVH contact kernel and the bucket sort of its codes, bit for bit against the oracle: leaf counts around a packet and a
 wave, crowds in which every particle reaches every other (the packet's list outgrows what it expands at once, and
 candidates are tested in many rounds), leaves that lie on both sides of a split, and packets that hold the leaves of
-several small scenes."""
+several small scenes; codes in one tile and many, in tiles of 1,024 and 4,096, in buckets of every width and in one
+bucket too large for LDS, alone and in a forest."""
 import numpy as np
 import pytest
 
@@ -67,3 +68,35 @@ def test_forest_of_small_scenes():
             st = oracle.State(sc, np.float32)
             st.step(2)
             assert_state_equal(e.download(k), st, f"scene {k}")
+
+
+def packed(n, seed, method, box):
+    """n grains, about eight per unit cube, in a corner of a box of the given edge."""
+    sc = crowd(n, seed, method, (n / 8.0) ** (1.0 / 3.0))
+    sc.cfg.boxMax[:] = [box] * 3
+    return sc
+
+
+@pytest.mark.parametrize("method", [capi.METHOD_LBVH30, capi.METHOD_LBVH63])
+@pytest.mark.parametrize("n,box", [(1023, 16.0), (1025, 30.0), (4097, 16.0), (30000, 26.0), (66001, 30.0), (9000, 2000.0)])
+def test_code_buckets(n, box, method):
+    print(f"lbvh codes: {n} in a box of {box}, method {method}", flush=True)
+    check(packed(n, n, method, box), 1)
+
+
+def test_forest_code_buckets():
+    print("lbvh codes: forest", flush=True)
+    mix = [packed(n, k, capi.METHOD_LBVH30, box)
+           for k, (n, box) in enumerate([(700, 16.0), (6000, 2000.0), (1, 16.0), (3000, 20.0), (12000, 24.0)])]
+    with Engine(mix) as e, Engine(mix[:1]) as other:
+        e.step(1)
+        for k, sc in enumerate(mix):
+            st = oracle.State(sc, np.float32)
+            st.step(1)
+            assert_state_equal(e.download(k), st, f"scene {k}")
+        other.rebuild(e, keep=(1, 4, 2), added=[mix[3]])     # the scenes carried over keep their bucket widths
+        other.step(1)
+        for k, (src, steps) in enumerate([(1, 2), (4, 2), (2, 2), (3, 1)]):
+            st = oracle.State(mix[src], np.float32)
+            st.step(steps)
+            assert_state_equal(other.download(k), st, f"carried {k}")
