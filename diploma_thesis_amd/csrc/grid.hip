@@ -1,4 +1,5 @@
 // grid.hip -- uniform-grid broadphase: cell bounds + reorder, and the 27-cell DEM kernel.
+#include "coop_cells.hpp"
 #include "csr_fill.hpp"
 #include "kernels.hpp"
 #include "reduce_apply.hpp"
@@ -395,6 +396,59 @@ __global__ void k_dem_grid_seg(const float4 *__restrict__ sPos, const float4 *__
     }
 }
 
+// The contact kernel with 16 lanes per particle (coop_cells): cells of the reference's cellStart / cellEnd (REF)
+// or of the exact table (cs = segStart); sceneTable: each particle's scene (its id in sortedVel.w), else the one
+// scene g.  Up to kCoopMax particles there are too few waves to hide a thread's chain of lookups and
+// candidate loads: 16,384 particles of c0's cubes 15.2 -> 9.6 us, 50,021 mixed ones 25 -> 17, piles of 65,536
+// and 131,072 61 -> 28 and 60 -> 47; at 200,003 58.8 -> 57.7, and a pile of 300,007 is slower (86 -> 93): there
+// the lanes' shared steps (slots, ranks, the ordered adds) cost more than the chains.
+constexpr int kCoopBlock = 128;
+constexpr int kCoopMax = 3 << 16;
+template <bool REF>
+__global__ __launch_bounds__(kCoopBlock) void k_dem_grid_coop(const float4 *__restrict__ sPos,
+                                                              const float4 *__restrict__ sVel,
+                                                              const unsigned *__restrict__ sIdx,
+                                                              const unsigned *__restrict__ cs,
+                                                              const unsigned *__restrict__ ce, int n, DevPhys ph,
+                                                              SceneGeom g, const SceneGeom *__restrict__ sceneTable,
+                                                              DemOut o) {
+    __shared__ CoopGroupLds sGroup[kCoopBlock / kCoopLanes];
+    const int gl = (int)threadIdx.x / kCoopLanes, l = (int)threadIdx.x & (kCoopLanes - 1);
+    const int i = xcd_block((int)blockIdx.x, (int)gridDim.x) * (kCoopBlock / kCoopLanes) + gl;
+    const bool valid = i < n;
+    const float4 P = sPos[valid ? i : n - 1], Vq = sVel[valid ? i : n - 1];
+    const unsigned orig = sIdx[valid ? i : n - 1];
+    const int ra = __float_as_int(P.w);
+    const f3 pa = xyz(P), va = xyz(Vq);
+    if (sceneTable) g = sceneTable[__float_as_int(Vq.w)];
+    int gx, gy, gz;
+    grid_pos(pa, g, gx, gy, gz);
+    const float Fc = coop_cells(
+        sGroup[gl], valid,
+        [&](int c, unsigned &b, unsigned &e) {
+            const unsigned h = g.cellBase + grid_hash(gx + c % 3 - 1, gy + (c / 3) % 3 - 1, gz + c / 9 - 1, g);
+            b = cs[h];
+            e = REF ? ce[h] : cs[h + 1];
+            if (REF && (b == kEmpty || e < b)) b = e = 0u;   // an empty cell's end is not defined
+        },
+        [&](unsigned j, f3 &f) {
+            const float4 Q = sPos[j];
+            if (!candidate(Q, pa, ra, (int)j == i, ph)) return false;
+            return pair_force(pa, xyz(Q), va, xyz(sVel[j]), ph, f);
+        });
+    f3 F = mk3(__shfl(Fc, 0, kCoopLanes), __shfl(Fc, 1, kCoopLanes), __shfl(Fc, 2, kCoopLanes));
+    if (!valid || l > 3) return;
+    if (!((ph.flags & kGrainClamp) && ra < 0)) F = add3(F, wall_force(pa, va, ph, g));
+    auto pick = [l](f3 v) { return l == 0 ? v.x : l == 1 ? v.y : l == 2 ? v.z : 0.0f; };
+    if (ra >= 0) {
+        reinterpret_cast<float *>(o.pForce + orig)[l] = pick(F);
+        if (o.pTorque) reinterpret_cast<float *>(o.pTorque + orig)[l] = pick(cross3(xyz(o.relPos[orig]), F));
+    } else {
+        const float fs = (ph.flags & kRefUnits) ? 1.0f : ph.dt;
+        reinterpret_cast<float *>(o.vel + orig)[l] = pick(mk3(va.x + F.x * fs, va.y + F.y * fs, va.z + F.z * fs));
+    }
+}
+
 // Grid DEM fused with the per-body reduction and apply (engine, exact cell table, no static set):
 // one launch in place of k_dem_grid_seg + k_reduce_apply, with no per-particle force round trip
 // through memory.  Waves [0, B) take one body each: lane l walks the body's particles l, l+64, ... in
@@ -478,6 +532,13 @@ void launch_dem_grid_seg(const float4 *sortedPos, const float4 *sortedVel, const
                          const SceneView &sv, bool sceneInVelW, const DemOut &o, int block, hipStream_t st) {
     if (n <= 0) return;
     if (block <= 0) block = 128;
+    if (!o.pairs && segBits == 0 && n <= kCoopMax) {
+        const int per = kCoopBlock / kCoopLanes;
+        hipLaunchKernelGGL(k_dem_grid_coop<false>, dim3((n + per - 1) / per), dim3(kCoopBlock), 0, st, sortedPos,
+                           sortedVel, sortedIdx, segStart, nullptr, n, ph, sv.single, sceneInVelW ? sv.table : nullptr,
+                           o);
+        return;
+    }
     dim3 grid((n + block - 1) / block);
     auto run = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(block), 0, st, sortedPos, sortedVel, sortedKeys, sortedIdx, segStart,
@@ -527,6 +588,12 @@ void launch_dem_grid(const float4 *sortedPos, const float4 *sortedVel, const uns
                      const SceneView &sv, bool sceneInVelW, const DemOut &o, int block, hipStream_t st) {
     if (n <= 0) return;
     if (block <= 0) block = 128;
+    if (!o.pairs && !sceneInVelW && n <= kCoopMax) {
+        const int per = kCoopBlock / kCoopLanes;
+        hipLaunchKernelGGL(k_dem_grid_coop<true>, dim3((n + per - 1) / per), dim3(kCoopBlock), 0, st, sortedPos,
+                           sortedVel, sortedIdx, cellStart, cellEnd, n, ph, sv.single, nullptr, o);
+        return;
+    }
     dim3 grid((n + block - 1) / block);
     if (o.pairs)
         hipLaunchKernelGGL(k_dem_grid<true>, grid, dim3(block), 0, st, sortedPos, sortedVel, sortedIdx, cellStart,

@@ -7,8 +7,9 @@ import numpy as np
 import pytest
 
 import oracle
-from diploma_thesis_amd import capi, scenes
+from diploma_thesis_amd import Engine, capi, scenes
 from gpu_util import Dev, sync
+from test_gpu_engine import assert_state_equal
 
 pytestmark = pytest.mark.gpu
 L = capi.lib
@@ -51,3 +52,42 @@ def test_static_contacts_many_candidates(n, points):
     assert np.array_equal(dF.get(), st.force) and np.array_equal(dT.get(), st.torque)
     if points >= 900:
         assert np.abs(st.force).max() > 0
+
+
+def crowd(n, seed, edge, method=capi.METHOD_GRID):
+    """A mixed scene whose particles all lie in a cube of the given edge."""
+    sc = scenes.mix_scene(n, seed, method).copy()
+    rng = np.random.default_rng(seed)
+    grains = sc.rb < 0
+    sc.pos[grains, :3] = 5.0 + rng.uniform(0, edge, (int(grains.sum()), 3))
+    shift = 5.0 + rng.uniform(0, edge, (sc.b, 3)) - sc.rb_pos[:, :3]
+    sc.rb_pos[:, :3] += shift.astype(np.float32)
+    sc.rb_vel[:, :3] = rng.normal(size=(sc.b, 3))
+    sc.vel[:, :3] = rng.normal(size=(sc.n, 3))
+    return sc
+
+
+@pytest.mark.parametrize("n,edge", [(1, 1.0), (7, 1.0), (9, 1.5), (500, 3.0), (2001, 4.0), (196608, 55.0), (196609, 55.0)])
+def test_engine_crowd_vs_oracle(n, edge):
+    """Hundreds of candidates a particle, particle counts around a workgroup, both sides of the 16-lane form's limit."""
+    print(f"grid contacts: crowd of {n}", flush=True)
+    sc = crowd(n, n, edge)
+    with Engine(sc) as e:
+        e.step(2)
+        e.sync()
+        g = e.download()
+    st = oracle.State(sc, np.float32)
+    st.step(2)
+    assert_state_equal(g, st, f"crowd of {n}")
+
+
+def test_engine_small_batch_vs_oracle():
+    print("grid contacts: batch of crowds", flush=True)
+    mix = [crowd(n, 70 + n, edge) for n, edge in ((3, 1.0), (500, 3.0), (1, 1.0), (129, 2.0), (2000, 5.0))]
+    with Engine(mix) as e:
+        e.step(2)
+        e.sync()
+        for k, sc in enumerate(mix):
+            st = oracle.State(sc, np.float32)
+            st.step(2)
+            assert_state_equal(e.download(k), st, f"scene {k}")
