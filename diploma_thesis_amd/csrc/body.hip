@@ -639,6 +639,7 @@ __global__ void k_carry_particles(const CarryRange *__restrict__ tab, int R, int
     dst.pos[i] = src.pos[j];
     dst.vel[i] = src.vel[j];
     dst.bodyFrame[i] = src.bodyFrame[j];
+    dst.relPos[i] = src.relPos[j];   // (a grain's stays zero: no step writes it)
     const int v = src.rb[j];
     dst.rb[i] = v >= 0 ? v - r.srcB + r.dstB : v;
     dst.scene[i] = (uint16_t)r.scene;

@@ -237,7 +237,7 @@ SceneView Engine::scene_view() const {
 
 StateBufs Engine::state_bufs() const {
     StateBufs b{};
-    b.pos = pos; b.vel = vel; b.bodyFrame = bodyFrame; b.rb = rb; b.scene = scene;
+    b.pos = pos; b.vel = vel; b.relPos = relPos; b.bodyFrame = bodyFrame; b.rb = rb; b.scene = scene;
     b.rbPos = rbPos; b.rbVel = rbVel; b.rbAng = rbAng; b.qinc = qinc; b.qcum = qcum;
     b.Ib = Ib; b.Iw = Iw; b.mass = mass; b.model = model; b.pstart = pstartD; b.pcount = pcountD;
     return b;

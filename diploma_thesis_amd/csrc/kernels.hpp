@@ -122,6 +122,7 @@ struct CarryRange {
     int dstP, srcP, n, dstB, srcB, b, scene;
 };
 struct StateBufs {
+    float4 *relPos;
     float4 *pos, *vel, *bodyFrame;
     int *rb;
     uint16_t *scene;

@@ -36,3 +36,17 @@ def test_arrays_together_equal_arrays_alone(n):
             assert np.array_equal(m[:, 12:15], alone["rb_pos"][:, :3])
             snap = e.snapshot(s)
             assert np.array_equal(snap.pos, alone["pos"]) and np.array_equal(snap.rb_vel, alone["rb_vel"])
+
+
+def test_relative_positions_survive_a_rebuild():
+    """Scenes carried over keep relativePos: zero for grains, whatever the engine's buffers held before."""
+    print("fetch: rebuild", flush=True)
+    bodies, grains = scenes.mix_scene(6400, 3), scenes.mix_scene(30, 4)   # 30 particles: grains only
+    assert grains.b == 0
+    with Engine([bodies]) as target, Engine([grains, bodies]) as source:
+        target.step(1)                                  # the target's buffers hold the cubes' offsets
+        source.step(1)
+        want = [read(source, s, ("rel",))["rel"] for s in (0, 1)]
+        target.rebuild(source, keep=(0, 1))
+        for s in (0, 1):
+            assert np.array_equal(read(target, s, ("rel",))["rel"], want[s]), s
