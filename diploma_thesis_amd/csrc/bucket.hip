@@ -164,19 +164,21 @@ __device__ __forceinline__ void block_fill(unsigned *table, unsigned long long a
         *reinterpret_cast<uint4 *>(table + k) = v4;
 }
 
+enum { kOutKeys = 0, kOutTable = 1, kOutIndex = 2 };
 // POSBITS: bits of a bucket position in the packed LDS words (the offset from c0 takes the other 32 -
-// POSBITS; a bucket sorted in LDS holds at most 2^POSBITS keys).  REORDER: also the gathered sorted
-// copies and the cell table (grid keys); without it only the sorted keys and indices (Morton keys,
+// POSBITS; a bucket sorted in LDS holds at most 2^POSBITS keys).  OUT: kOutTable, also the gathered sorted
+// copies and the cell table (grid keys); kOutIndex, the compact cell index in place of the table; kOutKeys, only the sorted keys and indices (Morton keys,
 // whose sorted-copy arrays are then only the global fallback's second buffer).  WIDE (Morton keys of scenes
 // with few particles, whose buckets span more than 2^(32 - POSBITS) codes, and 2^20 keys in 512 buckets
 // instead of 1,024: the LBVH30 step 342 -> 328 us): key and position apart.
 // kOut64 (a forest's Morton keys): the sorted keys as scene << 30 | code there instead of in kOut.
 // Eight waves per SIMD (two workgroups per CU): registers are held to that occupancy.
-template <int POSBITS, bool REORDER, bool WIDE>
+template <int POSBITS, int OUT, bool WIDE>
 __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_bucket_sort(
     TileKeyOut to, int split, unsigned *__restrict__ kOut, unsigned *__restrict__ vOut,
     const float4 *__restrict__ rec, float4 *__restrict__ sPos, float4 *__restrict__ sVel,
-    unsigned *__restrict__ table, unsigned numCells, uint64_t *__restrict__ kOut64) {
+    unsigned *__restrict__ table, unsigned numCells, uint64_t *__restrict__ kOut64, CellIndex ix) {
+    constexpr bool REORDER = OUT != kOutKeys;
     constexpr int kCap = kBkCap < (1 << POSBITS) ? kBkCap : (1 << POSBITS);
     constexpr int kLds = WIDE ? kCap : kBkCap;
     static_assert(!(WIDE && REORDER), "grid keys fit the packed words");
@@ -211,11 +213,14 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
     // also writes the table's closing entry, table[numCells]
     const unsigned long long c0 = (unsigned long long)bs.cellBase + ((unsigned long long)j << lowBits);
     const unsigned long long sceneEnd = (unsigned long long)bs.cellBase + bs.cells;
-    const unsigned long long c1 = g == to.numBuckets - 1 ? sceneEnd + 1ull
+    const unsigned long long c1 = g == to.numBuckets - 1 && OUT != kOutIndex ? sceneEnd + 1ull
                                   : c0 + (1ull << lowBits) < sceneEnd ? c0 + (1ull << lowBits) : sceneEnd;
     if (cnt == 0) {
         const unsigned long long n = c1 - c0;
-        if (REORDER) block_fill(table, c0 + n * part / split, c0 + n * (part + 1) / split, start);
+        if (OUT == kOutTable) block_fill(table, c0 + n * part / split, c0 + n * (part + 1) / split, start);
+        if (OUT == kOutIndex && part == 0)
+            for (unsigned w = t; w < (unsigned)(c1 - c0) >> 5; w += kBkThreads)
+                ix.words[(c0 >> 5) + w] = make_uint2(0u, 0u);
         return;
     }
     // The bucket's keys are the runs of bucket j in the scene's tiles, in tile order: tile k's run
@@ -256,6 +261,47 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
             const unsigned a = (unsigned)c0 + kp + 1u, b = (unsigned)c0 + ki + 1u;
             wave_fill(table, has, a, b, start + (unsigned)i);
         }
+    };
+    // the cell index of the bucket: a bit per occupied cell, the sorted positions where the occupied cells
+    // start listed from ix.starts[start] on, and per 32 cells the list slot of their first (in the cursor
+    // table, free once the passes are done).  The slot past the bucket's last cell closes it; where every
+    // key has a cell of its own that slot is the next bucket's first, which holds the same position.
+    auto fill_index = [&](auto low) {
+        unsigned *sBits = &sCur[0][0], *sBase = sBits + 2048;   // 2^16 cells at most
+        const unsigned words = (unsigned)(c1 - c0) >> 5;
+        const int lane = t & 63, wave = t >> 6;
+        const int seg = ((cnt + kBkThreads - 1) / kBkThreads) * 64;
+        const int s0 = min(wave * seg, cnt), s1 = min(s0 + seg, cnt);
+        for (unsigned w = t; w < words; w += kBkThreads) sBits[w] = 0u;
+        unsigned heads = 0u;
+        for (int g0 = s0; g0 < s1; g0 += 64) {
+            const int i = g0 + lane;
+            heads += (unsigned)__popcll(__ballot(i < s1 && (i == 0 || low(i) != low(i - 1))));
+        }
+        if (lane == 0) sWave[wave] = heads;
+        __syncthreads();
+        unsigned k = start, all = 0u;
+        for (int w = 0; w < kBkWaves; ++w) {
+            if (w < wave) k += sWave[w];
+            all += sWave[w];
+        }
+        for (int g0 = s0; g0 < s1; g0 += 64) {
+            const int i = g0 + lane;
+            const unsigned c = i < s1 ? low(i) : 0u, p = i > 0 && i < s1 ? low(i - 1) : 0u;
+            const bool head = i < s1 && (i == 0 || c != p);
+            const uint64_t m = __ballot(head);
+            const unsigned slot = k + (unsigned)__popcll(m & (lane == 0 ? 0ull : (~0ull >> (64 - lane))));
+            if (head) {
+                if (i >= i0 && i < i1) ix.starts[slot] = start + (unsigned)i;
+                atomicOr(&sBits[c >> 5], 1u << (c & 31u));
+                if (i == 0 || (c >> 5) != (p >> 5)) sBase[c >> 5] = slot;
+            }
+            k += (unsigned)__popcll(m);
+        }
+        if (part == nparts - 1 && t == 0) ix.starts[start + all] = start + (unsigned)cnt;
+        __syncthreads();
+        const unsigned wa = words * (unsigned)part / (unsigned)nparts, wb = words * (unsigned)(part + 1) / (unsigned)nparts;
+        for (unsigned w = wa + t; w < wb; w += kBkThreads) ix.words[(c0 >> 5) + w] = make_uint2(sBits[w], sBase[w]);
     };
     const unsigned base = (unsigned)c0;
     const uint64_t sceneKey = (uint64_t)(unsigned)to.bucketScene[g] << 30;
@@ -334,7 +380,8 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
             qa = rec[2 * (size_t)va + 1];
             pb = rec[2 * (size_t)vb];
             qb = rec[2 * (size_t)vb + 1];
-            fill_table([&](int i) -> unsigned { return sorted[i] >> POSBITS; });
+            if (OUT == kOutIndex) fill_index([&](int i) -> unsigned { return sorted[i] >> POSBITS; });
+            else fill_table([&](int i) -> unsigned { return sorted[i] >> POSBITS; });
         }
         if (ha) {
             store_key(ia, base + (wa >> POSBITS));
@@ -413,7 +460,8 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
                 sVel[start + i] = rec[2 * (size_t)val + 1];
             }
             __syncthreads();
-            fill_table([&](int i) -> unsigned { return kOut[start + i]; });
+            if (OUT == kOutIndex) fill_index([&](int i) -> unsigned { return kOut[start + i]; });
+            else fill_table([&](int i) -> unsigned { return kOut[start + i]; });
             __syncthreads();
         }
         for (int i = t; i < cnt; i += kBkThreads) store_key(i, kOut[start + i] + base);
@@ -546,10 +594,16 @@ bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *o
 }
 
 void launch_bucket_sort(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, const float4 *rec, float4 *sortedPos,
-                        float4 *sortedVel, unsigned *table, unsigned numCells, int split, hipStream_t st) {
+                        float4 *sortedVel, unsigned *table, unsigned numCells, int split, const CellIndex &ix,
+                        hipStream_t st) {
     if (to.numBuckets <= 0) return;
-    hipLaunchKernelGGL((k_bucket_sort<16, true, false>), dim3(to.numBuckets * split), dim3(kBkThreads), 0, st, to, split,
-                       kOut, vOut, rec, sortedPos, sortedVel, table, numCells, nullptr);
+    if (ix.words) {
+        hipLaunchKernelGGL((k_bucket_sort<16, kOutIndex, false>), dim3(to.numBuckets * split), dim3(kBkThreads), 0, st, to,
+                           split, kOut, vOut, rec, sortedPos, sortedVel, nullptr, numCells, nullptr, ix);
+        return;
+    }
+    hipLaunchKernelGGL((k_bucket_sort<16, kOutTable, false>), dim3(to.numBuckets * split), dim3(kBkThreads), 0, st, to, split,
+                       kOut, vOut, rec, sortedPos, sortedVel, table, numCells, nullptr, ix);
 }
 
 void launch_bucket_sort_morton(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, float4 *scratchA,
@@ -557,10 +611,10 @@ void launch_bucket_sort_morton(const TileKeyOut &to, unsigned *kOut, unsigned *v
     if (to.numBuckets <= 0) return;
     auto run = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(to.numBuckets), dim3(kBkThreads), 0, st, to, 1, kOut, vOut, nullptr, scratchA,
-                           scratchB, nullptr, 0u, kOut64);
+                           scratchB, nullptr, 0u, kOut64, CellIndex{});
     };
-    if (maxShift <= 32 - 12) run(k_bucket_sort<12, false, false>);
-    else run(k_bucket_sort<12, false, true>);
+    if (maxShift <= 32 - 12) run(k_bucket_sort<12, kOutKeys, false>);
+    else run(k_bucket_sort<12, kOutKeys, true>);
 }
 
 }  // namespace arsim

@@ -60,6 +60,10 @@ struct Engine {
     unsigned char *keyBufA = nullptr, *keyBufB = nullptr, *sortWsBuf = nullptr;
     unsigned *valsA = nullptr, *valsB = nullptr;
     unsigned *segStart = nullptr;           // grid: CSR offsets over segments of 2^segBits cells
+    bool useIndex = false;                  // grid, bucket sort: the compact cell index instead (kernels.hpp)
+    uint2 *cellWords = nullptr;
+    unsigned *cellStarts = nullptr;
+    CellIndex cell_index() const { return useIndex ? CellIndex{cellWords, cellStarts} : CellIndex{}; }
     unsigned *tileInfo = nullptr;           // grid, bucket sort: per-tile bucket runs (count << 16 | first)
     BucketScene *bkScenesD = nullptr;       // grid, bucket sort: the plan (bucket.hip)
     int *tileSceneD = nullptr, *bucketSceneD = nullptr;
@@ -140,6 +144,7 @@ struct Engine {
     // new dt or static set).
     bool integrate_ahead() const { return (bucketSort || mortonBucket) && !(flags & ARSIM_CONTACT_SIS) && !fused_dem(); }
     int prime();
+    int table_for_view();                   // fills segStart from the last step's sorted keys
     BodyBufs ahead_bufs() const;
     bool primed = false;
     // the grid DEM and the per-body reduction run as one kernel (on request; exact cell table, no static set)

@@ -291,6 +291,47 @@ __device__ __forceinline__ f3 dem_rows_exact(const float4 *__restrict__ sPos, co
 // the geometry is then read through scalar loads), or each lane's own entry (kGeomLane).  A batch runs
 // the kGeomBlock launch and then the kGeomLane launch, each doing the blocks the other skips.
 enum { kGeomSingle = 0, kGeomBlock = 1, kGeomLane = 2 };
+// The block of particles this workgroup takes (false: none).
+template <int GEOM>
+__device__ __forceinline__ bool dem_block(const SceneView &sv, int n, int &lb) {
+    if (GEOM == kGeomLane && sv.sceneStart) {
+        // one workgroup per boundary between scenes k - 1 and k: the block that holds it, if the boundary
+        // lies strictly inside a block and no earlier boundary lies strictly inside the same one
+        const int k = (int)blockIdx.x + 1, bs = (int)blockDim.x;
+        const int b = sv.sceneStart[k], pb = sv.sceneStart[k - 1];
+        lb = b / bs;
+        if (b % bs == 0 || b >= n) return false;
+        return !(k > 1 && pb / bs == lb && pb % bs != 0);
+    }
+    lb = xcd_block((int)blockIdx.x, (int)gridDim.x);
+    return true;
+}
+// The block's scene geometry, unless it is each lane's own (false: the block is another launch's).
+template <int GEOM>
+__device__ __forceinline__ bool dem_geom(const SceneView &sv, const float4 *__restrict__ sVel, int first, int n,
+                                         SceneGeom &g) {
+    if (GEOM == kGeomSingle) {
+        g = sv.single;
+        return true;
+    }
+    const int last = min(n, first + (int)blockDim.x) - 1;
+    const int sf = __float_as_int(sVel[first].w), sl = __float_as_int(sVel[last].w);
+    if ((sf == sl) != (GEOM == kGeomBlock)) return false;
+    if (GEOM == kGeomBlock) g = sv.table[sf];
+    return true;
+}
+// A particle's contact sum F, the walls added, to its body's force or to its velocity.
+__device__ __forceinline__ void dem_write(f3 F, int ra, f3 pa, f3 va, unsigned orig, const DevPhys &ph,
+                                          const SceneGeom &g, const DemOut &o) {
+    if (!((ph.flags & kGrainClamp) && ra < 0)) F = add3(F, wall_force(pa, va, ph, g));
+    if (ra >= 0) {
+        o.pForce[orig] = f4(F, 0.0f);
+        if (o.pTorque) o.pTorque[orig] = f4(cross3(xyz(o.relPos[orig]), F), 0.0f);
+    } else {
+        const float fs = (ph.flags & kRefUnits) ? 1.0f : ph.dt;
+        o.vel[orig] = make_float4(va.x + F.x * fs, va.y + F.y * fs, va.z + F.z * fs, 0.0f);
+    }
+}
 
 template <bool EMIT, bool EXACT, int GEOM>
 __global__ void k_dem_grid_seg(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
@@ -298,27 +339,10 @@ __global__ void k_dem_grid_seg(const float4 *__restrict__ sPos, const float4 *__
                                const unsigned *__restrict__ segStart, int segBits, int n, DevPhys ph, SceneView sv,
                                DemOut o) {
     int lb;
-    if (GEOM == kGeomLane && sv.sceneStart) {
-        // one workgroup per boundary between scenes k - 1 and k: the block that holds it, if the boundary
-        // lies strictly inside a block and no earlier boundary lies strictly inside the same one
-        const int k = (int)blockIdx.x + 1, bs = (int)blockDim.x;
-        const int b = sv.sceneStart[k], pb = sv.sceneStart[k - 1];
-        lb = b / bs;
-        if (b % bs == 0 || b >= n) return;
-        if (k > 1 && pb / bs == lb && pb % bs != 0) return;
-    } else {
-        lb = xcd_block((int)blockIdx.x, (int)gridDim.x);
-    }
+    if (!dem_block<GEOM>(sv, n, lb)) return;
     const int first = lb * (int)blockDim.x;
     SceneGeom g;
-    if (GEOM == kGeomSingle) {
-        g = sv.single;
-    } else {
-        const int last = min(n, first + (int)blockDim.x) - 1;
-        const int sf = __float_as_int(sVel[first].w), sl = __float_as_int(sVel[last].w);
-        if ((sf == sl) != (GEOM == kGeomBlock)) return;
-        if (GEOM == kGeomBlock) g = sv.table[sf];
-    }
+    if (!dem_geom<GEOM>(sv, sVel, first, n, g)) return;
     const int i = first + (int)threadIdx.x;
     if (i >= n) return;
     const float4 P = sPos[i];
@@ -386,14 +410,91 @@ __global__ void k_dem_grid_seg(const float4 *__restrict__ sPos, const float4 *__
         o.counts[orig] = cnt;
         return;
     }
-    if (!((ph.flags & kGrainClamp) && ra < 0)) F = add3(F, wall_force(pa, va, ph, g));
-    if (ra >= 0) {
-        o.pForce[orig] = f4(F, 0.0f);
-        if (o.pTorque) o.pTorque[orig] = f4(cross3(xyz(o.relPos[orig]), F), 0.0f);
+    dem_write(F, ra, pa, va, orig, ph, g, o);
+}
+
+// The contact kernel over the compact cell index: the occupied cells of all nine rows first (nine loads in
+// flight, from an index of a quarter byte a cell where the table has four), then the rows that have any, each
+// lane its own next one.  At the 2^20-particle scene it takes as long as with the table (68 us: what it saves in
+// memory it spends in instructions), while the bucket sort, which wrote the table, goes from 45 to 31 us;
+// at 128 mixed scenes 148 -> 144 and 117 -> 72 us.
+template <int GEOM>
+__global__ void k_dem_grid_index(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
+                                 const unsigned *__restrict__ sIdx, CellIndex ix, int n, DevPhys ph, SceneView sv,
+                                 DemOut o) {
+    extern __shared__ unsigned sRank[];   // per row and thread: slot of the row's first occupied cell
+    int lb;
+    if (!dem_block<GEOM>(sv, n, lb)) return;
+    const int first = lb * (int)blockDim.x;
+    SceneGeom g;
+    if (!dem_geom<GEOM>(sv, sVel, first, n, g)) return;
+    const int i = first + (int)threadIdx.x;
+    if (i >= n) return;
+    const float4 P = sPos[i];
+    const float4 Vq = sVel[i];
+    const int ra = __float_as_int(P.w);
+    if (GEOM == kGeomLane) g = sv.table[__float_as_int(Vq.w)];
+    const f3 pa = xyz(P), va = xyz(Vq);
+    int gx, gy, gz;
+    grid_pos(pa, g, gx, gy, gz);
+    const unsigned orig = sIdx[i];
+    const unsigned x0 = (unsigned)(gx - 1) & g.gridMask[0], x1 = (unsigned)gx & g.gridMask[0],
+                   x2 = (unsigned)(gx + 1) & g.gridMask[0];
+    const bool contiguous = (x0 + 1u == x1) && (x1 + 1u == x2);
+    const int lgx = __ffs((int)g.gx) - 1, lgxy = __ffs((int)g.gxy) - 1;
+    f3 F = mk3(0.f, 0.f, 0.f);
+    int cnt = 0;
+    auto row_of = [&](int r) {
+        const unsigned uz = (unsigned)(gz + (r / 3) - 1) & g.gridMask[2];
+        const unsigned uy = (unsigned)(gy + (r % 3) - 1) & g.gridMask[1];
+        return g.cellBase + (uz << lgxy) + (uy << lgx);
+    };
+    if (contiguous) {
+        unsigned rows = 0u;   // three bits a row: its occupied cells
+#pragma unroll
+        for (int z = 0; z < 3; ++z) {
+            uint4 w[3];
+#pragma unroll
+            for (int y = 0; y < 3; ++y) __builtin_memcpy(&w[y], ix.words + ((row_of(3 * z + y) + x0) >> 5), sizeof(uint4));
+#pragma unroll
+            for (int y = 0; y < 3; ++y) {
+                const int r = 3 * z + y;
+                const unsigned sh = (row_of(r) + x0) & 31u;
+                const unsigned lowBits = w[y].x >> sh;
+                const unsigned bits = __builtin_amdgcn_alignbit(w[y].z, w[y].x, sh) & 7u;
+                sRank[r * blockDim.x + threadIdx.x] =
+                    lowBits ? w[y].y + __popc(w[y].x & ((1u << sh) - 1u)) : w[y].w;
+                rows |= bits << (3 * r);
+            }
+        }
+        while (rows) {
+            const unsigned r = (unsigned)__builtin_ctz(rows) / 3u;
+            const unsigned bits = (rows >> (3u * r)) & 7u;
+            rows &= ~(7u << (3u * r));
+            const unsigned slot = sRank[r * blockDim.x + threadIdx.x];
+            uint4 s;
+            __builtin_memcpy(&s, ix.starts + slot, sizeof(s));
+            const unsigned n0 = bits & 1u, n01 = n0 + ((bits >> 1) & 1u), n012 = n01 + (bits >> 2);
+            const unsigned b1 = n0 ? s.y : s.x;
+            const unsigned b2 = n01 == 0u ? s.x : n01 == 1u ? s.y : s.z;
+            const unsigned e = n012 == 1u ? s.y : n012 == 2u ? s.z : s.w;
+            scan_run<false>(sPos, sVel, sIdx, s.x, b1, b2, e, i, ra, pa, va, ph, F, cnt, orig, o);
+        }
     } else {
-        const float fs = (ph.flags & kRefUnits) ? 1.0f : ph.dt;
-        o.vel[orig] = make_float4(va.x + F.x * fs, va.y + F.y * fs, va.z + F.z * fs, 0.0f);
+        for (int r = 0; r < 9; ++r) {
+            const unsigned row = row_of(r);
+#pragma unroll 1
+            for (int k = 0; k < 3; ++k) {
+                const unsigned h = row + (k == 0 ? x0 : k == 1 ? x1 : x2);
+                const uint2 w = ix.words[h >> 5];
+                if (!((w.x >> (h & 31u)) & 1u)) continue;
+                const unsigned *st = ix.starts + w.y + __popc(w.x & ((1u << (h & 31u)) - 1u));
+                const unsigned e = st[1];
+                scan_run<false>(sPos, sVel, sIdx, st[0], e, e, e, i, ra, pa, va, ph, F, cnt, orig, o);
+            }
+        }
     }
+    dem_write(F, ra, pa, va, orig, ph, g, o);
 }
 
 // The contact kernel with 16 lanes per particle (coop_cells): cells of the reference's cellStart / cellEnd (REF)
@@ -403,7 +504,6 @@ __global__ void k_dem_grid_seg(const float4 *__restrict__ sPos, const float4 *__
 // and 131,072 61 -> 28 and 60 -> 47; at 200,003 58.8 -> 57.7, and a pile of 300,007 is slower (86 -> 93): there
 // the lanes' shared steps (slots, ranks, the ordered adds) cost more than the chains.
 constexpr int kCoopBlock = 128;
-constexpr int kCoopMax = 3 << 16;
 template <bool REF>
 __global__ __launch_bounds__(kCoopBlock) void k_dem_grid_coop(const float4 *__restrict__ sPos,
                                                               const float4 *__restrict__ sVel,
@@ -572,6 +672,26 @@ void launch_dem_grid_seg(const float4 *sortedPos, const float4 *sortedVel, const
             geoms(k_dem_grid_seg<false, false, kGeomSingle>, k_dem_grid_seg<false, false, kGeomBlock>,
                   k_dem_grid_seg<false, false, kGeomLane>);
     }
+}
+
+void launch_dem_grid_index(const float4 *sortedPos, const float4 *sortedVel, const unsigned *sortedIdx,
+                           const CellIndex &ix, int n, const DevPhys &ph, const SceneView &sv, bool sceneInVelW,
+                           const DemOut &o, int block, hipStream_t st) {
+    if (n <= 0) return;
+    if (block <= 0) block = 128;
+    const unsigned all = (unsigned)((n + block - 1) / block);
+    const size_t lds = (size_t)9 * block * sizeof(unsigned);
+    auto run = [&](auto kernel, unsigned blocks) {
+        if (blocks > 0u)
+            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(block), lds, st, sortedPos, sortedVel, sortedIdx, ix, n, ph, sv,
+                               o);
+    };
+    if (!sceneInVelW) {
+        run(k_dem_grid_index<kGeomSingle>, all);
+        return;
+    }
+    run(k_dem_grid_index<kGeomBlock>, all);
+    run(k_dem_grid_index<kGeomLane>, sv.sceneStart ? (unsigned)(sv.count - 1) : all);
 }
 
 void launch_reorder(const unsigned *sortedKeys, const unsigned *sortedIdx, const float4 *pos, const float4 *vel,

@@ -220,8 +220,18 @@ bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *o
 // tiles' runs (tile order keeps the sort stable), `split` workgroups (1 or 2) sort it by the low bits,
 // each writing its share of the sorted keys / indices to (kOut, vOut), of the gathered sorted copies
 // and of the bucket's range of the exact cell table (whose last entry, numCells, the last bucket writes).
+// ix (words set): the compact cell index instead of the table.
+// Compact cell index: words[c / 32] = (a bit per occupied cell of the 32, slot of the first of them in starts);
+// starts lists, per bucket from the bucket's first sorted position on, where its occupied cells start, and then
+// the bucket's end.  A row of three cells is one 16-byte load of two words and, unless it is empty, one of
+// starts.  Valid where a row of cells never spans two buckets (shift >= log2 of the grid's x size and >= 5).
+struct CellIndex {
+    uint2 *words = nullptr;      // cells / 32 entries and one more
+    unsigned *starts = nullptr;  // N + 4 entries
+};
 void launch_bucket_sort(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, const float4 *rec, float4 *sortedPos,
-                        float4 *sortedVel, unsigned *table, unsigned numCells, int split, hipStream_t st);
+                        float4 *sortedVel, unsigned *table, unsigned numCells, int split, const CellIndex &ix,
+                        hipStream_t st);
 // The 63-bit order from the stable sort by the codes' top 30 bits: code63 is in particle order, k30 /
 // vIn the sorted top 30 bits and particle indices.  Writes the sorted 63-bit codes and indices; within
 // a run of equal top bits the members are ranked by their full codes, equal codes keeping the run's
@@ -241,6 +251,12 @@ void launch_fill_long(unsigned *table, unsigned long long tableSize, const LongF
 void launch_dem_grid_seg(const float4 *sortedPos, const float4 *sortedVel, const unsigned *sortedKeys,
                          const unsigned *sortedIdx, const unsigned *segStart, int segBits, int n, const DevPhys &ph,
                          const SceneView &sv, bool sceneInVelW, const DemOut &o, int block, hipStream_t st);
+// The same with the compact cell index (forces only).
+void launch_dem_grid_index(const float4 *sortedPos, const float4 *sortedVel, const unsigned *sortedIdx,
+                           const CellIndex &ix, int n, const DevPhys &ph, const SceneView &sv, bool sceneInVelW,
+                           const DemOut &o, int block, hipStream_t st);
+// Up to this many particles the contact kernel takes 16 lanes per particle and the exact cell table.
+constexpr int kCoopMax = 3 << 16;
 // Grid DEM fused with the per-body reduction and apply (exact cell table, no static collider set):
 // bodies take one wave each, grains 64 per wave.  rec is the pose kernel's gather record in the
 // original order (pos.xyz + rbIndex bits, vel.xyz + scene id); grainIdx lists every grain's index.
