@@ -1,4 +1,6 @@
 // grid.hip -- uniform-grid broadphase: cell bounds + reorder, and the 27-cell DEM kernel.
+#include <type_traits>
+
 #include "coop_cells.hpp"
 #include "csr_fill.hpp"
 #include "kernels.hpp"
@@ -285,40 +287,45 @@ __device__ __forceinline__ f3 dem_rows_exact(const float4 *__restrict__ sPos, co
 // keys visit them in the order x-1, x, x+1.  EXACT (segments of one cell, segStart = cellStart
 // with numCells + 1 entries): a row is the run [segStart[h0], segStart[h0 + 3]) with its cell
 // boundaries read from the table, and the keys are not read at all.
-// Where the kernel takes a scene's geometry from: the one scene's, passed by value (kGeomSingle);
-// for several scenes (scene id in sortedVel.w), the table entry of the block's scene when all of the
-// block's particles belong to it (kGeomBlock: the block's first and last sorted particle tell, and
-// the geometry is then read through scalar loads), or each lane's own entry (kGeomLane).  A batch runs
-// the kGeomBlock launch and then the kGeomLane launch, each doing the blocks the other skips.
+// Where a block's scene geometry comes from: the one scene's, passed by value (kGeomSingle); for several
+// scenes (scene id in sortedVel.w), the table entry of the block's scene when all of the block's
+// particles belong to it (kGeomBlock: scalar loads), or each lane's own entry (kGeomLane).
 enum { kGeomSingle = 0, kGeomBlock = 1, kGeomLane = 2 };
-// The block of particles this workgroup takes (false: none).
-template <int GEOM>
-__device__ __forceinline__ bool dem_block(const SceneView &sv, int n, int &lb) {
-    if (GEOM == kGeomLane && sv.sceneStart) {
-        // one workgroup per boundary between scenes k - 1 and k: the block that holds it, if the boundary
-        // lies strictly inside a block and no earlier boundary lies strictly inside the same one
-        const int k = (int)blockIdx.x + 1, bs = (int)blockDim.x;
-        const int b = sv.sceneStart[k], pb = sv.sceneStart[k - 1];
-        lb = b / bs;
-        if (b % bs == 0 || b >= n) return false;
-        return !(k > 1 && pb / bs == lb && pb % bs != 0);
-    }
-    lb = xcd_block((int)blockIdx.x, (int)gridDim.x);
-    return true;
+// The blocks of a batch's launch: first one workgroup per boundary between scenes k - 1 and k, which takes the
+// block that holds the boundary with kGeomLane (if the boundary lies strictly inside a block and no
+// earlier boundary lies strictly inside the same one), then every block, those of one scene being
+// taken with kGeomBlock.  As a launch of their own after the others the boundary blocks were alone on the
+// chip for 27 to 37 us: 128 scenes' step 314 -> 289 us, 24 larger scenes' 50 steps 14.7 -> 13.5 ms.
+__device__ __forceinline__ bool boundary_block(const SceneView &sv, int n, int &lb) {
+    const int k = (int)blockIdx.x + 1, bs = (int)blockDim.x;
+    const int b = sv.sceneStart[k], pb = sv.sceneStart[k - 1];
+    lb = b / bs;
+    if (b % bs == 0 || b >= n) return false;
+    return !(k > 1 && pb / bs == lb && pb % bs != 0);
 }
-// The block's scene geometry, unless it is each lane's own (false: the block is another launch's).
-template <int GEOM>
-__device__ __forceinline__ bool dem_geom(const SceneView &sv, const float4 *__restrict__ sVel, int first, int n,
-                                         SceneGeom &g) {
-    if (GEOM == kGeomSingle) {
-        g = sv.single;
-        return true;
+// Whether block lb lies in one scene.
+__device__ __forceinline__ bool one_scene(const float4 *__restrict__ sVel, int lb, int n, int &scene) {
+    const int first = lb * (int)blockDim.x, last = min(n, first + (int)blockDim.x) - 1;
+    scene = __float_as_int(sVel[first].w);
+    return scene == __float_as_int(sVel[last].w);
+}
+// Runs body(lb, g, lanes) for this workgroup's block: g its scene's geometry, or none (lanes true).
+template <bool BATCH, class Body>
+__device__ __forceinline__ void for_dem_block(const SceneView &sv, const float4 *__restrict__ sVel, int n, Body body) {
+    if (!BATCH) {
+        body(xcd_block((int)blockIdx.x, (int)gridDim.x), sv.single, std::integral_constant<int, kGeomSingle>{});
+        return;
     }
-    const int last = min(n, first + (int)blockDim.x) - 1;
-    const int sf = __float_as_int(sVel[first].w), sl = __float_as_int(sVel[last].w);
-    if ((sf == sl) != (GEOM == kGeomBlock)) return false;
-    if (GEOM == kGeomBlock) g = sv.table[sf];
-    return true;
+    const int boundaries = sv.count - 1;
+    int lb, scene;
+    if ((int)blockIdx.x < boundaries) {
+        if (!boundary_block(sv, n, lb) || one_scene(sVel, lb, n, scene)) return;
+        body(lb, SceneGeom{}, std::integral_constant<int, kGeomLane>{});
+        return;
+    }
+    lb = xcd_block((int)blockIdx.x - boundaries, (int)gridDim.x - boundaries);
+    if (!one_scene(sVel, lb, n, scene)) return;
+    body(lb, sv.table[scene], std::integral_constant<int, kGeomBlock>{});
 }
 // A particle's contact sum F, the walls added, to its body's force or to its velocity.
 __device__ __forceinline__ void dem_write(f3 F, int ra, f3 pa, f3 va, unsigned orig, const DevPhys &ph,
@@ -334,15 +341,12 @@ __device__ __forceinline__ void dem_write(f3 F, int ra, f3 pa, f3 va, unsigned o
 }
 
 template <bool EMIT, bool EXACT, int GEOM>
-__global__ void k_dem_grid_seg(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
-                               const unsigned *__restrict__ keys, const unsigned *__restrict__ sIdx,
-                               const unsigned *__restrict__ segStart, int segBits, int n, DevPhys ph, SceneView sv,
-                               DemOut o) {
-    int lb;
-    if (!dem_block<GEOM>(sv, n, lb)) return;
+__device__ __forceinline__ void dem_seg_block(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
+                                              const unsigned *__restrict__ keys, const unsigned *__restrict__ sIdx,
+                                              const unsigned *__restrict__ segStart, int segBits, int n,
+                                              const DevPhys &ph, const SceneView &sv, const DemOut &o, int lb,
+                                              SceneGeom g) {
     const int first = lb * (int)blockDim.x;
-    SceneGeom g;
-    if (!dem_geom<GEOM>(sv, sVel, first, n, g)) return;
     const int i = first + (int)threadIdx.x;
     if (i >= n) return;
     const float4 P = sPos[i];
@@ -412,6 +416,15 @@ __global__ void k_dem_grid_seg(const float4 *__restrict__ sPos, const float4 *__
     }
     dem_write(F, ra, pa, va, orig, ph, g, o);
 }
+template <bool EMIT, bool EXACT, bool BATCH>
+__global__ void k_dem_grid_seg(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
+                               const unsigned *__restrict__ keys, const unsigned *__restrict__ sIdx,
+                               const unsigned *__restrict__ segStart, int segBits, int n, DevPhys ph, SceneView sv,
+                               DemOut o) {
+    for_dem_block<BATCH>(sv, sVel, n, [&](int lb, const SceneGeom &g, auto geom) {
+        dem_seg_block<EMIT, EXACT, decltype(geom)::value>(sPos, sVel, keys, sIdx, segStart, segBits, n, ph, sv, o, lb, g);
+    });
+}
 
 // The contact kernel over the compact cell index: the occupied cells of all nine rows first (nine loads in
 // flight, from an index of a quarter byte a cell where the table has four), then the rows that have any, each
@@ -419,15 +432,11 @@ __global__ void k_dem_grid_seg(const float4 *__restrict__ sPos, const float4 *__
 // memory it spends in instructions), while the bucket sort, which wrote the table, goes from 45 to 31 us;
 // at 128 mixed scenes 148 -> 144 and 117 -> 72 us.
 template <int GEOM>
-__global__ void k_dem_grid_index(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
-                                 const unsigned *__restrict__ sIdx, CellIndex ix, int n, DevPhys ph, SceneView sv,
-                                 DemOut o) {
-    extern __shared__ unsigned sRank[];   // per row and thread: slot of the row's first occupied cell
-    int lb;
-    if (!dem_block<GEOM>(sv, n, lb)) return;
+__device__ __forceinline__ void dem_index_block(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
+                                                const unsigned *__restrict__ sIdx, const CellIndex &ix, int n,
+                                                const DevPhys &ph, const SceneView &sv, const DemOut &o, int lb,
+                                                SceneGeom g, unsigned *sRank) {
     const int first = lb * (int)blockDim.x;
-    SceneGeom g;
-    if (!dem_geom<GEOM>(sv, sVel, first, n, g)) return;
     const int i = first + (int)threadIdx.x;
     if (i >= n) return;
     const float4 P = sPos[i];
@@ -495,6 +504,15 @@ __global__ void k_dem_grid_index(const float4 *__restrict__ sPos, const float4 *
         }
     }
     dem_write(F, ra, pa, va, orig, ph, g, o);
+}
+template <bool BATCH>
+__global__ void k_dem_grid_index(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
+                                 const unsigned *__restrict__ sIdx, CellIndex ix, int n, DevPhys ph, SceneView sv,
+                                 DemOut o) {
+    extern __shared__ unsigned sRank[];   // per row and thread: slot of the row's first occupied cell
+    for_dem_block<BATCH>(sv, sVel, n, [&](int lb, const SceneGeom &g, auto geom) {
+        dem_index_block<decltype(geom)::value>(sPos, sVel, sIdx, ix, n, ph, sv, o, lb, g, sRank);
+    });
 }
 
 // The contact kernel with 16 lanes per particle (coop_cells): cells of the reference's cellStart / cellEnd (REF)
@@ -640,37 +658,20 @@ void launch_dem_grid_seg(const float4 *sortedPos, const float4 *sortedVel, const
         return;
     }
     dim3 grid((n + block - 1) / block);
-    auto run = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(block), 0, st, sortedPos, sortedVel, sortedKeys, sortedIdx, segStart,
-                           segBits, n, ph, sv, o);
-    };
-    auto geoms = [&](auto single, auto perBlock, auto perLane) {
-        if (!sceneInVelW) {
-            run(single);
-        } else {
-            run(perBlock);
-            // the blocks that straddle two scenes: with the scenes' sorted ranges known, one workgroup
-            // per boundary instead of a full grid whose other blocks return at once
-            if (!sv.sceneStart) run(perLane);
-            else if (sv.count > 1)
-                hipLaunchKernelGGL(perLane, dim3((unsigned)(sv.count - 1)), dim3(block), 0, st, sortedPos, sortedVel,
-                                   sortedKeys, sortedIdx, segStart, segBits, n, ph, sv, o);
-        }
+    auto run = [&](auto single, auto batch) {
+        if (sceneInVelW)
+            hipLaunchKernelGGL(batch, dim3(grid.x + (unsigned)sv.count - 1u), dim3(block), 0, st, sortedPos, sortedVel,
+                               sortedKeys, sortedIdx, segStart, segBits, n, ph, sv, o);
+        else
+            hipLaunchKernelGGL(single, grid, dim3(block), 0, st, sortedPos, sortedVel, sortedKeys, sortedIdx, segStart,
+                               segBits, n, ph, sv, o);
     };
     if (o.pairs) {
-        if (segBits == 0)
-            geoms(k_dem_grid_seg<true, true, kGeomSingle>, k_dem_grid_seg<true, true, kGeomBlock>,
-                  k_dem_grid_seg<true, true, kGeomLane>);
-        else
-            geoms(k_dem_grid_seg<true, false, kGeomSingle>, k_dem_grid_seg<true, false, kGeomBlock>,
-                  k_dem_grid_seg<true, false, kGeomLane>);
+        if (segBits == 0) run(k_dem_grid_seg<true, true, false>, k_dem_grid_seg<true, true, true>);
+        else run(k_dem_grid_seg<true, false, false>, k_dem_grid_seg<true, false, true>);
     } else {
-        if (segBits == 0)
-            geoms(k_dem_grid_seg<false, true, kGeomSingle>, k_dem_grid_seg<false, true, kGeomBlock>,
-                  k_dem_grid_seg<false, true, kGeomLane>);
-        else
-            geoms(k_dem_grid_seg<false, false, kGeomSingle>, k_dem_grid_seg<false, false, kGeomBlock>,
-                  k_dem_grid_seg<false, false, kGeomLane>);
+        if (segBits == 0) run(k_dem_grid_seg<false, true, false>, k_dem_grid_seg<false, true, true>);
+        else run(k_dem_grid_seg<false, false, false>, k_dem_grid_seg<false, false, true>);
     }
 }
 
@@ -681,17 +682,12 @@ void launch_dem_grid_index(const float4 *sortedPos, const float4 *sortedVel, con
     if (block <= 0) block = 128;
     const unsigned all = (unsigned)((n + block - 1) / block);
     const size_t lds = (size_t)9 * block * sizeof(unsigned);
-    auto run = [&](auto kernel, unsigned blocks) {
-        if (blocks > 0u)
-            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(block), lds, st, sortedPos, sortedVel, sortedIdx, ix, n, ph, sv,
-                               o);
-    };
-    if (!sceneInVelW) {
-        run(k_dem_grid_index<kGeomSingle>, all);
-        return;
-    }
-    run(k_dem_grid_index<kGeomBlock>, all);
-    run(k_dem_grid_index<kGeomLane>, sv.sceneStart ? (unsigned)(sv.count - 1) : all);
+    if (sceneInVelW)
+        hipLaunchKernelGGL(k_dem_grid_index<true>, dim3(all + (unsigned)sv.count - 1u), dim3(block), lds, st, sortedPos,
+                           sortedVel, sortedIdx, ix, n, ph, sv, o);
+    else
+        hipLaunchKernelGGL(k_dem_grid_index<false>, dim3(all), dim3(block), lds, st, sortedPos, sortedVel, sortedIdx, ix,
+                           n, ph, sv, o);
 }
 
 void launch_reorder(const unsigned *sortedKeys, const unsigned *sortedIdx, const float4 *pos, const float4 *vel,
