@@ -25,7 +25,8 @@ bool sort_tuning_supported(int ipt, int rbits);
 // *keys / *vals hold the sorted data.  valsIota: the input values are 0..n-1 (not read).
 template <class K>
 int sort_pairs(K **keys, unsigned **vals, K **alt, unsigned **altVals, int n, int beginBit, int endBit,
-               bool valsIota, void *ws, size_t wsBytes, const SortTuning &tu, hipStream_t st, bool prepared = false);
+               bool valsIota, void *ws, size_t wsBytes, const SortTuning &tu, hipStream_t st, bool prepared = false,
+               const unsigned *gate = nullptr);
 // Where the sort keeps its digit histograms, tile counters and look-back words inside the workspace.
 // A caller may zero {hist, counters, statusA} and accumulate the histograms itself (for instance while
 // it generates the keys) and then call sort_pairs(..., prepared = true), which skips both steps; the
@@ -377,6 +378,13 @@ struct SisWork {
     float4 *prep;                  // the sweeps' records in level order (planes of cap float4)
     unsigned *blockCnt;
     int *numContacts;
+    // small islands (launch_sis_solve): gate[0] = some scene takes the levels, gate[1] = islands listed;
+    // each island's (first slot of islandList, contacts); the scenes' contact ranges left to the levels.  In
+    // the place of blockCnt, keysA, valsA and (one scene) sceneRange
+    unsigned *gate;
+    int2 *island;
+    int *islandList;
+    int2 *levelRange;
     size_t end;
 };
 // Deepest contact per sorted particle against other bodies' particles (engine layout: exact cell

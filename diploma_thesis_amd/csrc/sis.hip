@@ -5,7 +5,9 @@
 // contact before it that touches one of its bodies (its predecessors); level(c) = 1 + the larger
 // of its predecessors' levels.  Contacts of one level touch disjoint bodies and everything they
 // read was written by lower levels, so running a sweep level by level, with a barrier between
-// levels, reads and writes every body value exactly as the serial loop does.
+// levels, reads and writes every body value exactly as the serial loop does.  Where the contacts fall into many
+// small groups that share no body (islands), the groups run side by side, each in contact order, for the same
+// reason with the same results.
 #include <climits>
 
 #include "kernels.hpp"
@@ -289,7 +291,9 @@ __device__ __forceinline__ int2 scene_range(const int2 *sceneRange, const int *n
 // body contacts); the key is the body, or numBodies for an unused entry.  Sorted stably by key,
 // the entries of one body come in contact order.
 __global__ void k_sis_entries(const int2 *__restrict__ bodies, const int *__restrict__ numContacts, int cap,
-                              unsigned invalid, unsigned *__restrict__ keys, int *__restrict__ pred) {
+                              unsigned invalid, const unsigned *gate, unsigned *__restrict__ keys,
+                              int *__restrict__ pred) {
+    if (*gate == 0u) return;
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= 2 * cap) return;
     const int c = e >> 1, k = e & 1;
@@ -305,7 +309,8 @@ __global__ void k_sis_entries(const int2 *__restrict__ bodies, const int *__rest
 
 // pred[e] = the contact of the previous entry with the same body (-1 for the first).
 __global__ void k_sis_pred(const unsigned *__restrict__ keys, const unsigned *__restrict__ vals, int n,
-                           unsigned invalid, int *__restrict__ pred) {
+                           unsigned invalid, const unsigned *gate, int *__restrict__ pred) {
+    if (*gate == 0u) return;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const unsigned key = keys[i];
@@ -508,12 +513,9 @@ struct VelLds {
 // with coalesced loads (a level's positions are consecutive) instead of gathering by contact; the
 // bodies' inverse inertia, the same over the sweeps, comes from the bodies (in LDS when they fit).
 constexpr int kSisPlanes = 6;
-__global__ void k_sis_prep(SisContacts ct, SisBodies bd, SisSolvePhys ph, const int *__restrict__ numContacts,
-                           const int *__restrict__ order, int cap, float4 *__restrict__ rec) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= numContacts[0]) return;
-    const int c = order[q];
-    const size_t P = (size_t)cap;
+// Contact c's record at position q (bodies as l1, l2 in the record).
+__device__ __forceinline__ void sis_record(const SisContacts &ct, const SisBodies &bd, const SisSolvePhys &ph, int c,
+                                           int l1, int l2, float4 *rec, size_t P, size_t q) {
     const float4 n4 = ct.normal[c], pt = ct.point[c];
     const int2 bb = ct.bodies[c];
     const f3 n = xyz(n4);
@@ -538,7 +540,7 @@ __global__ void k_sis_prep(SisContacts ct, SisBodies bd, SisSolvePhys ph, const 
         rec[P + q] = f4(p1, mc);
         rec[2 * P + q] = f4(t, kt);
         rec[3 * P + q] = f4(t2, kt2);
-        rec[4 * P + q] = make_float4(__int_as_float(bb.x), __int_as_float(-1), m1, fb);
+        rec[4 * P + q] = make_float4(__int_as_float(l1), __int_as_float(-1), m1, fb);
         for (int k = 0; k < 9; ++k) I2[k] = 0.0f;
     } else {
         ld_mat(bd.Iw, bb.y, I2);
@@ -549,9 +551,18 @@ __global__ void k_sis_prep(SisContacts ct, SisBodies bd, SisSolvePhys ph, const 
         if (fabs((double)mc) < 0.00001) mc = 1.0f;
         rec[P + q] = f4(p1, mc);
         rec[2 * P + q] = f4(p2, 0.0f);
-        rec[4 * P + q] = make_float4(__int_as_float(bb.x), __int_as_float(bb.y), m1, m2);
+        rec[4 * P + q] = make_float4(__int_as_float(l1), __int_as_float(l2), m1, m2);
     }
     rec[5 * P + q] = ct.impulse[c];
+}
+__global__ void k_sis_prep(SisContacts ct, SisBodies bd, SisSolvePhys ph, const int *__restrict__ numContacts,
+                           const int *__restrict__ order, int cap, const unsigned *gate, float4 *__restrict__ rec) {
+    if (*gate == 0u) return;
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= numContacts[0]) return;
+    const int c = order[q];
+    const int2 b = ct.bodies[c];
+    sis_record(ct, bd, ph, c, b.x, b.y, rec, (size_t)cap, (size_t)q);
 }
 
 // One contact of one sweep, record q: SequentialImpulseSolver (Particles/updateFunctions.cpp:1580-1874).
@@ -562,7 +573,7 @@ __global__ void k_sis_prep(SisContacts ct, SisBodies bd, SisSolvePhys ph, const 
 //    signs (its friction impulses are not applied there, so they are not formed here).
 // Velocities are stored with w = 0.
 template <class VA>
-__device__ void sis_contact(size_t q, float4 *__restrict__ rec, size_t P, const VA &va) {
+__device__ __forceinline__ void sis_contact(size_t q, float4 *__restrict__ rec, size_t P, const VA &va) {
     const float4 r0 = rec[q], r1 = rec[P + q], r2 = rec[2 * P + q], r4 = rec[4 * P + q];
     float4 acc = rec[5 * P + q];
     const f3 n = xyz(r0);
@@ -638,6 +649,7 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_solve(float4 *__restrict__ re
     extern __shared__ float4 sVel[];
     const int s = blockIdx.x;
     const int2 rg = scene_range(sceneRange, numContacts, s);
+    if (rg.x == rg.y) return;
     const int levels = maxLvl[s] + 1;
     const int *off = offAll + rg.x + s;
     const size_t P = (size_t)cap;
@@ -668,6 +680,386 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_solve(float4 *__restrict__ re
             bd.ang[br.x + k] = sVel[2 * k + 1];
         }
     for (int k = rg.x + (int)threadIdx.x; k < rg.y; k += kSisBlock) impulse[order[k]] = rec[5 * P + k];
+}
+
+// ---- small islands.  Bodies that touch, directly or through others, form an island (the static points link
+// nothing), and the sweeps of one island read and write nothing of another's.  A scene whose islands are all
+// small (thrown objects on a scanned floor, stacks side by side) runs them side by side, each island's
+// contacts one after another in contact order with everything in LDS, instead of the whole scene level by
+// level in one workgroup.  A scene with a larger island keeps the levels as a whole: the levels advance with its
+// longest chain anyway, and the others' contacts fill them.
+constexpr int kIslandContacts = 128, kIslandBodies = 16;   // what one island may hold
+constexpr int kIslandSceneBodies = 4096;                   // bodies of a scene whose islands are looked for
+
+__device__ __forceinline__ int island_root(const int *parent, int b) {
+    while (true) {
+        const int p = __hip_atomic_load(parent + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (p == b) return b;
+        b = p;
+    }
+}
+
+// One workgroup per scene: the islands by union-find over the body contacts (a root always points at a
+// smaller body, so the links form no cycle), their contacts counted and, if all are small, listed (in any
+// order within an island).  Bound by the latency of its three passes over the contacts' bodies: 49,152 contacts
+// 58 us with a leader per run of equal pairs, 83 with every contact on its own.
+__global__ __launch_bounds__(kSisBlock) void k_sis_islands(const int2 *__restrict__ bodies,
+                                                           const int2 *__restrict__ sceneRange,
+                                                           const int *__restrict__ numContacts,
+                                                           const int2 *__restrict__ sceneBodies, int numBodies,
+                                                           int2 *__restrict__ levelRange, unsigned *__restrict__ gate,
+                                                           int2 *__restrict__ island, int *__restrict__ islandList,
+                                                           int *__restrict__ order) {
+    __shared__ int parent[kIslandSceneBodies], sCnt[kIslandSceneBodies], sBodies[kIslandSceneBodies];
+    __shared__ int sWaveN[kSisWaves], sWaveC[kSisWaves], sBase;
+    const int s = blockIdx.x, t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int2 rg = scene_range(sceneRange, numContacts, s);
+    const int2 br = sceneBodies ? sceneBodies[s] : make_int2(0, numBodies);
+    if (rg.x == rg.y || br.y > kIslandSceneBodies) {
+        if (t == 0) {
+            levelRange[s] = rg;
+            if (rg.x != rg.y) atomicOr(gate, 1u);
+        }
+        return;
+    }
+    for (int b = t; b < br.y; b += kSisBlock) {
+        parent[b] = b;
+        sCnt[b] = 0;
+        sBodies[b] = 0;
+    }
+    __syncthreads();
+    // The contacts in steps of kAhead per thread, their bodies loaded together.  A body's contacts with one partner
+    // are consecutive, so only the first of a run of equal pairs within a wave acts, for the whole run.
+    constexpr int kAhead = 4;
+    auto for_runs = [&](auto act) {   // act(contact, bodies, leads its run, the lane that does, run length of a leader)
+        for (int c0 = rg.x; c0 < rg.y; c0 += kAhead * kSisBlock) {
+            int2 bb[kAhead];
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                const int c = c0 + k * kSisBlock + t;
+                bb[k] = c < rg.y ? bodies[c] : make_int2(-1, -1);
+            }
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                const int c = c0 + k * kSisBlock + t;
+                const int px = __shfl_up(bb[k].x, 1, 64), py = __shfl_up(bb[k].y, 1, 64);
+                const bool head = c < rg.y && (lane == 0 || px != bb[k].x || py != bb[k].y);
+                const uint64_t m = __ballot(head), live = __ballot(c < rg.y);
+                const uint64_t upto = ~0ull >> (63 - lane);
+                const uint64_t later = m & ~upto;
+                const int end = later ? __ffsll((long long)later) - 1 : __popcll(live);
+                const int leader = (m & upto) ? 63 - __clzll((long long)(m & upto)) : 0;
+                act(c, bb[k], head, leader, end - lane);
+            }
+        }
+    };
+    bool big = false;
+    for_runs([&](int, int2 bb, bool head, int, int) {
+        if (!head) return;
+        if ((unsigned)(bb.x - br.x) >= (unsigned)br.y || (bb.y >= 0 && (unsigned)(bb.y - br.x) >= (unsigned)br.y) ||
+            bb.x == bb.y) {
+            big = true;   // (a caller's list that names a body it did not count, or one body twice)
+            return;
+        }
+        if (bb.y < 0) return;
+        int u = island_root(parent, bb.x - br.x), v = island_root(parent, bb.y - br.x);
+        while (u != v) {
+            if (u < v) {
+                const int x = u;
+                u = v;
+                v = x;
+            }
+            const int old = atomicCAS(&parent[u], u, v);   // u is the larger root: hang it under v
+            if (old == u) break;
+            u = island_root(parent, old);
+            v = island_root(parent, v);
+        }
+    });
+    if (!__syncthreads_or(big)) {
+        for (int b = t; b < br.y; b += kSisBlock) atomicAdd(&sBodies[island_root(parent, b)], 1);
+        for_runs([&](int, int2 bb, bool head, int, int len) {
+            if (head) atomicAdd(&sCnt[island_root(parent, bb.x - br.x)], len);
+        });
+        __syncthreads();
+    }
+    for (int b = t; b < br.y; b += kSisBlock)
+        big |= sCnt[b] > kIslandContacts || (sCnt[b] > 0 && sBodies[b] > kIslandBodies);
+    if (__syncthreads_or(big)) {
+        if (t == 0) {
+            levelRange[s] = rg;
+            atomicOr(gate, 1u);
+        }
+        return;
+    }
+    // islands numbered and their lists laid out in body order of their roots: four bodies a thread
+    constexpr int kPer = kIslandSceneBodies / kSisBlock;
+    int cnt[kPer], n = 0, contacts = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int b = t * kPer + k;
+        cnt[k] = b < br.y ? sCnt[b] : 0;
+        n += cnt[k] > 0 ? 1 : 0;
+        contacts += cnt[k];
+    }
+    int xn = n, xc = contacts;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int yn = __shfl_up(xn, d, 64), yc = __shfl_up(xc, d, 64);
+        if (lane >= d) {
+            xn += yn;
+            xc += yc;
+        }
+    }
+    if (lane == 63) {
+        sWaveN[wave] = xn;
+        sWaveC[wave] = xc;
+    }
+    __syncthreads();
+    int all = 0, at = xn - n, first = xc - contacts;
+    for (int w = 0; w < kSisWaves; ++w) {
+        at += w < wave ? sWaveN[w] : 0;
+        first += w < wave ? sWaveC[w] : 0;
+        all += sWaveN[w];
+    }
+    if (t == 0) {
+        sBase = (int)atomicAdd(gate + 1, (unsigned)all);
+        levelRange[s] = make_int2(rg.x, rg.x);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int b = t * kPer + k;
+        if (cnt[k] <= 0) continue;
+        island[sBase + at++] = make_int2(rg.x + first, cnt[k]);
+        sCnt[b] = first;
+        first += cnt[k];
+    }
+    __syncthreads();
+    for_runs([&](int c, int2 bb, bool head, int leader, int len) {
+        int slot = head ? atomicAdd(&sCnt[island_root(parent, bb.x - br.x)], len) : 0;
+        slot = __shfl(slot, leader, 64) + lane - leader;
+        if (c >= rg.y) return;
+        islandList[rg.x + slot] = c;
+        order[c] = c;   // (the level records of a scene without levels are formed, and not used)
+    });
+}
+
+// Lane K's or a rotated lane's value within each quad of lanes (DPP quad_perm).
+template <int CTRL>
+__device__ __forceinline__ float quad(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float q_next(float v) { return quad<0xC9>(v); }    // component c + 1
+__device__ __forceinline__ float q_after(float v) { return quad<0xD2>(v); }   // component c + 2
+__device__ __forceinline__ float q_0(float v) { return quad<0x00>(v); }
+__device__ __forceinline__ float q_1(float v) { return quad<0x55>(v); }
+__device__ __forceinline__ float q_2(float v) { return quad<0xAA>(v); }
+__device__ __forceinline__ float q_dot(float a, float b) {
+    const float m = a * b;
+    return (q_0(m) + q_1(m)) + q_2(m);
+}
+
+// The sweeps of the islands, eight lanes an island and up to four islands a wave.  An island's contacts are one
+// dependent chain (48 contacts for a stack of two cubes on the floor, 18 sweeps of them), so what counts is the
+// time of one contact: lane c of a quad holds component c of every vector, the first quad the contact's first
+// body and the second quad its partner; of a static contact's three impulses lane c divides and clamps its
+// own.  Every sum and product is that of sis_contact, in its order.  Contacts are taken in runs of one pair of
+// bodies, which stay in registers for the run, and the next contact's record is read while this one is worked on.
+// One wave a workgroup and islands added to a wave only when there are more than CUs: waves that share a CU slow
+// each other down about as much as they add, islands in one wave run in step.  The sweeps of the stacked-cubes
+// scene (1,024 islands of 48 contacts): the levels in one workgroup 1,672 us; one island a wave 580, with four waves a
+// workgroup 613; so 312.  64 islands, the whole solve: 295 us, with four waves a workgroup 606, the levels 719.
+constexpr int kWaveIslands = 4;   // islands a wave takes at most
+__device__ __forceinline__ void wave_sync() {   // LDS written by the wave's lanes, read by others of them
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+struct IslandLds {
+    float4 rec[kSisPlanes * kIslandContacts], vel[kIslandBodies * 2];
+    float inertia[kIslandBodies * 9];
+    int key[kIslandContacts], ord[kIslandContacts], body[2 * kIslandContacts], first[2 * kIslandContacts];
+    int2 count;                     // contacts, bodies
+    int ids[kIslandBodies], run[kIslandContacts + 1];   // run: first contacts of the runs of one pair
+};
+__global__ __launch_bounds__(64) void k_sis_solve_islands(SisContacts ct, SisBodies bd, SisSolvePhys ph,
+                                                          const unsigned *__restrict__ gate,
+                                                          const int2 *__restrict__ island,
+                                                          const int *__restrict__ islandList, int iterations) {
+    constexpr int kSlots = kIslandContacts;
+    __shared__ IslandLds sAll[kWaveIslands];
+    const int lane = (int)threadIdx.x;
+    const unsigned islands = gate[1];
+    int per = 1;   // islands of this wave: one a CU as long as there are CUs
+    while (per < kWaveIslands && (unsigned)per * 256u < islands) per *= 2;
+    const unsigned g0 = blockIdx.x * (unsigned)per;
+    if (g0 >= islands) return;
+    int myN = 0, myRuns = 0;   // of the island that this lane's eight lanes take
+    for (int q = 0; q < per; ++q) {
+        IslandLds &I = sAll[q];
+        float4 *sRec = I.rec, *sVel = I.vel;
+        float *sI = I.inertia;
+        int *sKey = I.key, *sOrd = I.ord, *sBody = I.body, *sFirst = I.first, *sIds = I.ids, *sRun = I.run;
+        const int2 is = g0 + (unsigned)q < islands ? island[g0 + (unsigned)q] : make_int2(0, 0);
+        const int n = is.y;
+        // the contacts in contact order: a contact's place is the number of smaller ones
+        for (int k = lane; k < n; k += 64) sKey[k] = islandList[is.x + k];
+        wave_sync();
+        for (int k = lane; k < n; k += 64) {
+            const int key = sKey[k];
+            int r = 0;
+            for (int j = 0; j < n; ++j) r += sKey[j] < key ? 1 : 0;
+            sOrd[r] = key;
+        }
+        wave_sync();
+        // the bodies, numbered by their first appearance among the contacts' (b1, b2)
+        for (int k = lane; k < n; k += 64) {
+            const int2 bb = ct.bodies[sOrd[k]];
+            sBody[2 * k] = bb.x;
+            sBody[2 * k + 1] = bb.y;
+        }
+        wave_sync();
+        int ids = 0;
+        for (int e0 = 0; e0 < 2 * n; e0 += 64) {
+            const int e = e0 + lane;
+            const int b = e < 2 * n ? sBody[e] : -1;
+            int f = e;
+            for (int j = 2 * n - 1; j >= 0; --j) f = sBody[j] == b && j < f ? j : f;
+            const uint64_t m = __ballot(b >= 0 && f == e);
+            if (b >= 0 && f == e) {
+                const int id = ids + (int)__popcll(m & (lane == 0 ? 0ull : (~0ull >> (64 - lane))));
+                sIds[id] = b;
+                sFirst[e] = id;
+            }
+            ids += (int)__popcll(m);
+            wave_sync();
+            if (b >= 0 && f != e) sFirst[e] = sFirst[f];
+        }
+        wave_sync();
+        for (int k = lane; k < ids; k += 64) {
+            const int b = sIds[k];
+            sVel[2 * k] = bd.vel[b];
+            sVel[2 * k + 1] = bd.ang[b];
+            for (int i = 0; i < 9; ++i) sI[9 * k + i] = bd.Iw[9 * (size_t)b + i];
+        }
+        for (int k = lane; k < n; k += 64)
+            sis_record(ct, bd, ph, sOrd[k], sFirst[2 * k], sFirst[2 * k + 1], sRec, kSlots, k);
+        wave_sync();
+        int runs = 0;
+        for (int e0 = 0; e0 < n; e0 += 64) {
+            const int k = e0 + lane;
+            const bool head = k < n && (k == 0 || sBody[2 * k] != sBody[2 * k - 2] || sBody[2 * k + 1] != sBody[2 * k - 1]);
+            const uint64_t m = __ballot(head);
+            if (head) sRun[runs + (int)__popcll(m & (lane == 0 ? 0ull : (~0ull >> (64 - lane))))] = k;
+            runs += (int)__popcll(m);
+        }
+        if (lane == 0) {
+            sRun[runs] = n;
+            I.count = make_int2(n, ids);
+        }
+        if ((lane >> 3) == q) {
+            myN = n;
+            myRuns = runs;
+        }
+        wave_sync();
+    }
+    if (myN > 0) {
+        IslandLds &I = sAll[lane >> 3];
+        float4 *sRec = I.rec, *sVel = I.vel;
+        const float *sI = I.inertia;
+        const int *sRun = I.run, runs = myRuns, sub = lane & 7;
+        const int c = lane & 3, c0 = c < 3 ? c : 0, cn = c0 == 2 ? 0 : c0 + 1, ca = c0 == 0 ? 2 : c0 - 1;
+        const bool second = sub >= 4;
+        float *R = reinterpret_cast<float *>(sRec), *V = reinterpret_cast<float *>(sVel);
+        auto word = [&](int plane, int k, int w) { return R[4 * (plane * kSlots + k) + w]; };
+        int at = -1, at1 = -1, at2 = -1;   // the quad's body (-1: none of its own), and the pair held
+        float v = 0.f, w = 0.f, i0 = 0.f, i3 = 0.f, i6 = 0.f, mass = 1.f;
+        auto put_back = [&]() {
+            if (at < 0) return;
+            V[8 * at + c] = c < 3 ? v : 0.0f;
+            V[8 * at + 4 + c] = c < 3 ? w : 0.0f;
+        };
+        // the impulse J moves the quad's body: v += J / m, w += I^-1 (p x J) (the partner: -=)
+        auto apply = [&](float J, float pn, float pa, bool minus) {
+            const float dv = J / mass;
+            const float pj = pn * q_after(J) - pa * q_next(J);
+            const float dw = i0 * q_0(pj) + i3 * q_1(pj) + i6 * q_2(pj);
+            v = minus ? v - dv : v + dv;
+            w = minus ? w - dw : w + dw;
+        };
+        for (int it = 0; it < iterations; ++it)
+            for (int r = 0; r < runs; ++r) {
+                const int k0 = sRun[r], k1 = sRun[r + 1];
+                const int b1 = __float_as_int(word(4, k0, 0)), b2 = __float_as_int(word(4, k0, 1));
+                if (b1 != at1 || b2 != at2) {
+                    put_back();
+                    wave_sync();
+                    at1 = b1;
+                    at2 = b2;
+                    at = second ? b2 : b1;
+                    const int b = at < 0 ? b1 : at;   // (a static contact's second quad works along with the first)
+                    v = V[8 * b + c];
+                    w = V[8 * b + 4 + c];
+                    i0 = sI[9 * b + c0];
+                    i3 = sI[9 * b + 3 + c0];
+                    i6 = sI[9 * b + 6 + c0];
+                    mass = word(4, k0, second && b2 >= 0 ? 3 : 2);   // (a body contact's word 3 is its partner's mass)
+                }
+                if (b2 < 0) {
+                    float pn = word(1, k0, cn), pa = word(1, k0, ca), nn = word(0, k0, c0), t = word(2, k0, c0),
+                          t2 = word(3, k0, c0), bias = word(0, k0, 3), den = word(1 + c0, k0, 3), fb = word(4, k0, 3),
+                          acc = word(5, k0, c0);
+                    for (int k = k0; k < k1; ++k) {
+                        const int kn = k + 1 < k1 ? k + 1 : k;
+                        const float pn_ = word(1, kn, cn), pa_ = word(1, kn, ca), nn_ = word(0, kn, c0),
+                                    t_ = word(2, kn, c0), t2_ = word(3, kn, c0), bias_ = word(0, kn, 3),
+                                    den_ = word(1 + c0, kn, 3), fb_ = word(4, kn, 3), acc_ = word(5, kn, c0);
+                        const float vp = v + (q_next(w) * pa - q_after(w) * pn);   // v + w x p
+                        const float d0 = q_dot(vp, nn), d1 = q_dot(vp, t), d2 = q_dot(vp, t2);
+                        const float num = c0 == 0 ? -(d0 + bias) : -(c0 == 1 ? d1 : d2);
+                        const float lo = c0 == 0 ? 0.0f : -fb, hi = c0 == 0 ? 100.0f : fb;
+                        float tmp = acc + num / den;
+                        tmp = tmp < lo ? lo : (tmp > hi ? hi : tmp);
+                        const float d = tmp - acc;
+                        if (sub < 3) R[4 * (5 * kSlots + k) + sub] = tmp;
+                        apply((q_0(d) * nn + q_1(d) * t) + q_2(d) * t2, pn, pa, false);
+                        pn = pn_; pa = pa_; nn = nn_; t = t_; t2 = t2_; bias = bias_; den = den_; fb = fb_; acc = acc_;
+                    }
+                } else {
+                    const int pp = second ? 2 : 1;
+                    float pn = word(pp, k0, cn), pa = word(pp, k0, ca), nn = word(0, k0, c0), bias = word(0, k0, 3),
+                          den = word(1, k0, 3), acc = word(5, k0, 0);
+                    for (int k = k0; k < k1; ++k) {
+                        const int kn = k + 1 < k1 ? k + 1 : k;
+                        const float pn_ = word(pp, kn, cn), pa_ = word(pp, kn, ca), nn_ = word(0, kn, c0),
+                                    bias_ = word(0, kn, 3), den_ = word(1, kn, 3), acc_ = word(5, kn, 0);
+                        const float vp = v + (q_next(w) * pa - q_after(w) * pn);
+                        const float s = q_dot(vp, nn);
+                        // the first body's minus the partner's, in both quads (DPP row_shl / row_shr by four lanes)
+                        const float up = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x104, 0xf, 0xf, true));
+                        const float dn = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x114, 0xf, 0xf, true));
+                        const float num = -((second ? dn - s : s - up) + bias);
+                        float tmp = acc + num / den;
+                        tmp = tmp < 0.0f ? 0.0f : (tmp > 100.0f ? 100.0f : tmp);
+                        const float d = tmp - acc;
+                        if (sub == 0) R[4 * (5 * kSlots + k)] = tmp;
+                        apply(d * nn, pn, pa, second);
+                        pn = pn_; pa = pa_; nn = nn_; bias = bias_; den = den_; acc = acc_;
+                    }
+                }
+            }
+        put_back();
+    }
+    wave_sync();
+    for (int q = 0; q < per; ++q) {
+        const IslandLds &I = sAll[q];
+        const int n = I.count.x, ids = I.count.y;
+        for (int k = lane; k < ids; k += 64) {
+            const int b = I.ids[k];
+            bd.vel[b] = I.vel[2 * k];
+            bd.ang[b] = I.vel[2 * k + 1];
+        }
+        for (int k = lane; k < n; k += 64) ct.impulse[I.ord[k]] = I.rec[5 * kSlots + k];
+    }
 }
 
 }  // namespace
@@ -739,6 +1131,11 @@ SisWork sis_work_layout(void *base, int cap, int numScenes, int numBodyParticles
     w.prep = (float4 *)take((size_t)kSisPlanes * cap * 16);
     w.blockCnt = (unsigned *)take(2 * (size_t)(nblk + 1) * 4);
     w.numContacts = (int *)take(4);
+    // the islands are found and swept after the gather's counts and before the levels' sort keys, in their place
+    w.gate = w.blockCnt;
+    w.island = (int2 *)w.keysA;
+    w.islandList = (int *)w.valsA;
+    w.levelRange = numScenes > 1 ? (int2 *)take((size_t)numScenes * 8) : w.sceneRange;   // (one scene's range is not stored)
     w.end = o;
     return w;
 }
@@ -762,19 +1159,29 @@ int launch_sis_solve(const SisContacts &ct, const SisBodies &bd, const SisSolveP
     const unsigned invalid = (unsigned)numBodies;
     int bits = 1;
     while (bits < 32 && (invalid >> bits) != 0u) ++bits;
+    launch_fill_u32(w.gate, 0u, 2, st);
+    hipLaunchKernelGGL(k_sis_islands, dim3(numScenes), dim3(kSisBlock), 0, st, ct.bodies,
+                       numScenes > 1 ? w.sceneRange : nullptr, w.numContacts, sceneBodies, numBodies, w.levelRange,
+                       w.gate, w.island, w.islandList, w.order);
+    const int most = cap < numBodies ? cap : numBodies;   // every island has a contact and a body
+    if (most > 0 && iterations > 0)
+        hipLaunchKernelGGL(k_sis_solve_islands, dim3(most), dim3(64), 0, st, ct, bd, ph, w.gate, w.island,
+                           w.islandList, iterations);
+    // the scenes left to the levels (none: these launches end at their gate)
     hipLaunchKernelGGL(k_sis_entries, dim3((ne + 255) / 256), dim3(256), 0, st, ct.bodies, w.numContacts, cap,
-                       invalid, w.keysA, w.pred);
+                       invalid, w.gate, w.keysA, w.pred);
     unsigned *kA = w.keysA, *kB = w.keysB, *vA = w.valsA, *vB = w.valsB;
-    if (sort_pairs<unsigned>(&kA, &vA, &kB, &vB, ne, 0, bits, true, w.sortWs, w.sortWsBytes, tu, st)) return 1;
-    hipLaunchKernelGGL(k_sis_pred, dim3((ne + 255) / 256), dim3(256), 0, st, kA, vA, ne, invalid, w.pred);
-    const int2 *rg = numScenes > 1 ? w.sceneRange : nullptr;
+    if (sort_pairs<unsigned>(&kA, &vA, &kB, &vB, ne, 0, bits, true, w.sortWs, w.sortWsBytes, tu, st, false, w.gate))
+        return 1;
+    hipLaunchKernelGGL(k_sis_pred, dim3((ne + 255) / 256), dim3(256), 0, st, kA, vA, ne, invalid, w.gate, w.pred);
+    const int2 *rg = w.levelRange;
     hipLaunchKernelGGL(k_sis_levels, dim3(numScenes), dim3(kSisBlock), 0, st, w.pred, rg, w.numContacts, w.lvl,
                        w.maxLvl);
     hipLaunchKernelGGL(k_sis_bucket, dim3(numScenes), dim3(kSisBlock), 0, st, w.lvl, rg, w.numContacts, w.maxLvl,
                        w.off, w.cur, w.order);
     if (iterations > 0) {
         hipLaunchKernelGGL(k_sis_prep, dim3((cap + 255) / 256), dim3(256), 0, st, ct, bd, ph, w.numContacts, w.order,
-                           cap, w.prep);
+                           cap, w.gate, w.prep);
         if (maxSceneBodies <= kSisLdsBodies)
             hipLaunchKernelGGL(k_sis_solve<true>, dim3(numScenes), dim3(kSisBlock),
                                (size_t)maxSceneBodies * (2 * sizeof(float4) + 9 * sizeof(float)), st, w.prep, cap,

@@ -47,8 +47,10 @@ __device__ __forceinline__ unsigned block_exclusive_scan(unsigned v, unsigned *s
     return waveOff + x - v;
 }
 
+// gate (of every kernel here): the sort does nothing when it is given and zero.
 __global__ void k_sort_init(unsigned *hist, int histWords, unsigned *counters, int numCounters,
-                            unsigned *status0, int statusWords) {
+                            unsigned *status0, int statusWords, const unsigned *gate) {
+    if (gate && *gate == 0u) return;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     int stride = gridDim.x * blockDim.x;
     for (int k = i; k < histWords; k += stride) hist[k] = 0u;
@@ -58,7 +60,9 @@ __global__ void k_sort_init(unsigned *hist, int histWords, unsigned *counters, i
 
 template <class K, int RBITS>
 __global__ __launch_bounds__(kBlock) void k_sort_hist(const K *__restrict__ keys, int n, int beginBit,
-                                                       int endBit, int passes, unsigned *__restrict__ hist) {
+                                                       int endBit, int passes, unsigned *__restrict__ hist,
+                                                       const unsigned *gate) {
+    if (gate && *gate == 0u) return;
     constexpr int RADIX = 1 << RBITS;
     constexpr int MAXP = (int)(sizeof(K) * 8 + RBITS - 1) / RBITS;
     __shared__ unsigned sh[MAXP * RADIX];
@@ -94,7 +98,8 @@ __global__ __launch_bounds__(kBlock) void k_onesweep(const K *__restrict__ kin, 
                                                       int shift, int bits, int valsIota,
                                                       const unsigned *__restrict__ histPass,
                                                       unsigned *tileCounter, unsigned *status,
-                                                      unsigned *statusNext) {
+                                                      unsigned *statusNext, const unsigned *gate) {
+    if (gate && *gate == 0u) return;
     constexpr int RADIX = 1 << RBITS;
     constexpr int TILE = kBlock * IPT;
     __shared__ K sKeys[TILE];
@@ -225,13 +230,13 @@ inline int num_passes(int beginBit, int endBit, int rbits) { return (endBit - be
 template <class K, int IPT, int RBITS>
 void launch_passes(K **keys, unsigned **vals, K **alt, unsigned **altVals, int n, int beginBit, int endBit,
                    bool valsIota, unsigned *hist, unsigned *counters, unsigned *statusA, unsigned *statusB,
-                   int numTiles, bool doHist, hipStream_t st) {
+                   int numTiles, bool doHist, const unsigned *gate, hipStream_t st) {
     const int passes = num_passes(beginBit, endBit, RBITS);
     if (doHist) {
         int histBlocks = (n + kBlock * 8 - 1) / (kBlock * 8);
         histBlocks = histBlocks < 1 ? 1 : (histBlocks > 4096 ? 4096 : histBlocks);
         hipLaunchKernelGGL((k_sort_hist<K, RBITS>), dim3(histBlocks), dim3(kBlock), 0, st, *keys, n, beginBit, endBit,
-                           passes, hist);
+                           passes, hist, gate);
     }
     for (int p = 0; p < passes; ++p) {
         int shift = beginBit + p * RBITS;
@@ -240,7 +245,7 @@ void launch_passes(K **keys, unsigned **vals, K **alt, unsigned **altVals, int n
         unsigned *nxt = (p + 1 < passes) ? ((p & 1) ? statusA : statusB) : nullptr;
         hipLaunchKernelGGL((k_onesweep<K, IPT, RBITS>), dim3(numTiles), dim3(kBlock), 0, st, *keys, *vals, *alt,
                            *altVals, n, shift, bits, (valsIota && p == 0) ? 1 : 0, hist + (size_t)p * 256,
-                           counters + p, cur, nxt);
+                           counters + p, cur, nxt, gate);
         K *tk = *keys; *keys = *alt; *alt = tk;
         unsigned *tv = *vals; *vals = *altVals; *altVals = tv;
     }
@@ -283,7 +288,8 @@ SortPlan sort_plan(void *ws, int n, int keyBytes, int beginBit, int endBit, cons
 
 template <class K>
 int sort_pairs(K **keys, unsigned **vals, K **alt, unsigned **altVals, int n, int beginBit, int endBit,
-               bool valsIota, void *ws, size_t wsBytes, const SortTuning &tu, hipStream_t st, bool prepared) {
+               bool valsIota, void *ws, size_t wsBytes, const SortTuning &tu, hipStream_t st, bool prepared,
+               const unsigned *gate) {
     if (n <= 0) return 0;
     if (n >= (1 << 30)) return -1;
     const int keyBits = (int)sizeof(K) * 8;
@@ -298,12 +304,12 @@ int sort_pairs(K **keys, unsigned **vals, K **alt, unsigned **altVals, int n, in
         int initBlocks = (initWords + kBlock - 1) / kBlock;
         initBlocks = initBlocks < 1 ? 1 : (initBlocks > 1024 ? 1024 : initBlocks);
         hipLaunchKernelGGL(k_sort_init, dim3(initBlocks), dim3(kBlock), 0, st, hist, (int)pl.histWords, counters,
-                           pl.passes, statusA, initWords);
+                           pl.passes, statusA, initWords, gate);
     }
 #define ARSIM_SORT_CASE(I, R)                                                                                 \
     if (ipt == I && rbits == R) {                                                                             \
         launch_passes<K, I, R>(keys, vals, alt, altVals, n, beginBit, endBit, valsIota, hist, counters,       \
-                               statusA, statusB, numTiles, !prepared, st);                                    \
+                               statusA, statusB, numTiles, !prepared, gate, st);                              \
         return 0;                                                                                             \
     }
     ARSIM_SORT_CASE(8, 8)
@@ -320,9 +326,9 @@ int sort_pairs(K **keys, unsigned **vals, K **alt, unsigned **altVals, int n, in
 }
 
 template int sort_pairs<unsigned>(unsigned **, unsigned **, unsigned **, unsigned **, int, int, int, bool, void *,
-                                  size_t, const SortTuning &, hipStream_t, bool);
+                                  size_t, const SortTuning &, hipStream_t, bool, const unsigned *);
 template int sort_pairs<uint64_t>(uint64_t **, unsigned **, uint64_t **, unsigned **, int, int, int, bool, void *,
-                                  size_t, const SortTuning &, hipStream_t, bool);
+                                  size_t, const SortTuning &, hipStream_t, bool, const unsigned *);
 
 // ---------------------------------------------------------------- sort without a caller workspace
 // The workspace of a u32-key sort of up to ARSIM_SORT_NOALLOC_MAX_ITEMS items lives in this
