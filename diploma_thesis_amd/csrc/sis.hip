@@ -315,7 +315,8 @@ __global__ void k_sis_pred(const unsigned *__restrict__ keys, const unsigned *__
     if (i >= n) return;
     const unsigned key = keys[i];
     if (key == invalid) return;
-    if (i > 0 && keys[i - 1] == key) pred[vals[i]] = (int)(vals[i - 1] >> 1);
+    // (a contact that names one body twice is not its own predecessor: the levels would never settle)
+    if (i > 0 && keys[i - 1] == key && vals[i - 1] >> 1 != vals[i] >> 1) pred[vals[i]] = (int)(vals[i - 1] >> 1);
 }
 
 __device__ __forceinline__ int block_max(int v, int *sRed) {

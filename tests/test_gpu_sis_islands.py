@@ -81,6 +81,13 @@ def test_solve_island_sizes_vs_oracle(islands, shuffle):
     solve_both(nb, pairs, 7 + len(islands))
 
 
+def test_solve_a_body_against_itself_vs_oracle():
+    print("sis islands: a contact that names one body twice", flush=True)
+    nb, pairs = contact_list([(3, 9), (2, 4)], True, np.random.default_rng(3))
+    pairs[5] = pairs[5, 0]
+    solve_both(nb, pairs, 11)
+
+
 def test_engine_scenes_with_and_without_small_islands():
     # sparse scenes (islands), a dense one (levels) and one without contacts in one batch, and each alone
     print("sis islands: batch of both kinds", flush=True)
