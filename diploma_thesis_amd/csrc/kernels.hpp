@@ -378,12 +378,12 @@ struct SisWork {
     float4 *prep;                  // the sweeps' records in level order (planes of cap float4)
     unsigned *blockCnt;
     int *numContacts;
-    // small islands (launch_sis_solve): gate[0] = some scene takes the levels, gate[1] = islands listed;
-    // each island's (first slot of islandList, contacts); the scenes' contact ranges left to the levels.  In
-    // the place of blockCnt, keysA, valsA and (one scene) sceneRange
+    // small islands (launch_sis_solve): gate[0] = some contacts take the levels, gate[1] = islands listed;
+    // each island's (first slot of islandList, contacts); the contacts left to the levels and the scenes' ranges of
+    // them.  In the place of blockCnt, keysA, valsA, prep and (one scene) sceneRange
     unsigned *gate;
     int2 *island;
-    int *islandList;
+    int *islandList, *levelList;
     int2 *levelRange;
     size_t end;
 };

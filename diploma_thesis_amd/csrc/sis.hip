@@ -287,18 +287,20 @@ __device__ __forceinline__ int2 scene_range(const int2 *sceneRange, const int *n
     return sceneRange ? sceneRange[s] : make_int2(0, numContacts[0]);
 }
 
-// Entries of the predecessor search: entry e = 2c + k names body k of contact c (k = 1 only for
+// The contacts that go through the levels, in contact order: entry j of a scene's range in list[] (-1: unused), which
+// is what the predecessors and levels speak of.
+// Entries of the predecessor search: entry e = 2j + k names body k of contact list[j] (k = 1 only for
 // body contacts); the key is the body, or numBodies for an unused entry.  Sorted stably by key,
 // the entries of one body come in contact order.
-__global__ void k_sis_entries(const int2 *__restrict__ bodies, const int *__restrict__ numContacts, int cap,
-                              unsigned invalid, const unsigned *gate, unsigned *__restrict__ keys,
-                              int *__restrict__ pred) {
+__global__ void k_sis_entries(const int2 *__restrict__ bodies, const int *__restrict__ list,
+                              const int *__restrict__ numContacts, int cap, unsigned invalid, const unsigned *gate,
+                              unsigned *__restrict__ keys, int *__restrict__ pred) {
     if (*gate == 0u) return;
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= 2 * cap) return;
-    const int c = e >> 1, k = e & 1;
+    const int k = e & 1, c = (e >> 1) < numContacts[0] ? list[e >> 1] : -1;
     unsigned key = invalid;
-    if (c < numContacts[0]) {
+    if (c >= 0) {
         const int2 b = bodies[c];
         const int body = k ? b.y : b.x;
         if (body >= 0) key = (unsigned)body;
@@ -408,11 +410,12 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_levels(const int *__restrict_
     if (threadIdx.x == 0) maxLvl[blockIdx.x] = mx;
 }
 
-// Contacts of one scene grouped by level: off[L] = first position of level L in order[], for
+// Contacts (list[j]) of one scene grouped by level: off[L] = first position of level L in order[], for
 // L = 0 .. maxLvl + 1; the scene's offsets start at off + range.x + scene.  The per-level counters
 // live in LDS when the levels fit, in global memory (cur) otherwise.
 constexpr int kBucketLds = 12288;
 __global__ __launch_bounds__(kSisBlock) void k_sis_bucket(const int *__restrict__ lvl,
+                                                          const int *__restrict__ list,
                                                           const int2 *__restrict__ sceneRange,
                                                           const int *__restrict__ numContacts,
                                                           const int *__restrict__ maxLvl, int *__restrict__ offAll,
@@ -459,7 +462,7 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_bucket(const int *__restrict_
         if (threadIdx.x == 0) sCarry = carry + (int)tot;
         __syncthreads();
     }
-    for (int c = rg.x + (int)threadIdx.x; c < rg.y; c += kSisBlock) order[rg.x + atomicAdd(&cnt[lvl[c]], 1)] = c;
+    for (int c = rg.x + (int)threadIdx.x; c < rg.y; c += kSisBlock) order[rg.x + atomicAdd(&cnt[lvl[c]], 1)] = list[c];
 }
 
 __device__ __forceinline__ void ld_mat(const float *__restrict__ Iw, int b, float m[9]) {
@@ -562,6 +565,7 @@ __global__ void k_sis_prep(SisContacts ct, SisBodies bd, SisSolvePhys ph, const 
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= numContacts[0]) return;
     const int c = order[q];
+    if (c < 0) return;   // (no contact of the levels)
     const int2 b = ct.bodies[c];
     sis_record(ct, bd, ph, c, b.x, b.y, rec, (size_t)cap, (size_t)q);
 }
@@ -684,11 +688,11 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_solve(float4 *__restrict__ re
 }
 
 // ---- small islands.  Bodies that touch, directly or through others, form an island (the static points link
-// nothing), and the sweeps of one island read and write nothing of another's.  A scene whose islands are all
-// small (thrown objects on a scanned floor, stacks side by side) runs them side by side, each island's
-// contacts one after another in contact order with everything in LDS, instead of the whole scene level by
-// level in one workgroup.  A scene with a larger island keeps the levels as a whole: the levels advance with its
-// longest chain anyway, and the others' contacts fill them.
+// nothing), and the sweeps of one island read and write nothing of another's.  Small islands (thrown objects on
+// a scanned floor, stacks side by side) run side by side, each one's contacts one after another in contact
+// order with everything in LDS, instead of level by level in one workgroup a scene.  The contacts of larger islands
+// keep the levels, which advance with the longest chain: the stacked cubes after 800 steps, when some have spread
+// into one large island, 2,636 us a step with all contacts in the levels and 2,177 so.
 constexpr int kIslandContacts = 128, kIslandBodies = 16;   // what one island may hold
 constexpr int kIslandSceneBodies = 4096;                   // bodies of a scene whose islands are looked for
 
@@ -701,8 +705,8 @@ __device__ __forceinline__ int island_root(const int *parent, int b) {
 }
 
 // One workgroup per scene: the islands by union-find over the body contacts (a root always points at a
-// smaller body, so the links form no cycle), their contacts counted and, if all are small, listed (in any
-// order within an island).  Bound by the latency of its three passes over the contacts' bodies: 49,152 contacts
+// smaller body, so the links form no cycle) and their contacts counted; the small ones listed (in any order within
+// an island), the others' contacts gathered in contact order for the levels.  Bound by the latency of its three passes over the contacts' bodies: 49,152 contacts
 // 58 us with a leader per run of equal pairs, 83 with every contact on its own.
 __global__ __launch_bounds__(kSisBlock) void k_sis_islands(const int2 *__restrict__ bodies,
                                                            const int2 *__restrict__ sceneRange,
@@ -710,17 +714,21 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_islands(const int2 *__restric
                                                            const int2 *__restrict__ sceneBodies, int numBodies,
                                                            int2 *__restrict__ levelRange, unsigned *__restrict__ gate,
                                                            int2 *__restrict__ island, int *__restrict__ islandList,
-                                                           int *__restrict__ order) {
+                                                           int *__restrict__ levelList, int *__restrict__ order) {
     __shared__ int parent[kIslandSceneBodies], sCnt[kIslandSceneBodies], sBodies[kIslandSceneBodies];
     __shared__ int sWaveN[kSisWaves], sWaveC[kSisWaves], sBase;
     const int s = blockIdx.x, t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
     const int2 rg = scene_range(sceneRange, numContacts, s);
     const int2 br = sceneBodies ? sceneBodies[s] : make_int2(0, numBodies);
-    if (rg.x == rg.y || br.y > kIslandSceneBodies) {
+    auto all_to_levels = [&]() {
+        for (int c = rg.x + t; c < rg.y; c += kSisBlock) levelList[c] = c;
         if (t == 0) {
             levelRange[s] = rg;
             if (rg.x != rg.y) atomicOr(gate, 1u);
         }
+    };
+    if (rg.x == rg.y || br.y > kIslandSceneBodies) {
+        all_to_levels();
         return;
     }
     for (int b = t; b < br.y; b += kSisBlock) {
@@ -754,12 +762,12 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_islands(const int2 *__restric
             }
         }
     };
-    bool big = false;
+    bool bad = false;
     for_runs([&](int, int2 bb, bool head, int, int) {
         if (!head) return;
         if ((unsigned)(bb.x - br.x) >= (unsigned)br.y || (bb.y >= 0 && (unsigned)(bb.y - br.x) >= (unsigned)br.y) ||
             bb.x == bb.y) {
-            big = true;   // (a caller's list that names a body it did not count, or one body twice)
+            bad = true;   // (a caller's list that names a body it did not count, or one body twice)
             return;
         }
         if (bb.y < 0) return;
@@ -776,29 +784,33 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_islands(const int2 *__restric
             v = island_root(parent, v);
         }
     });
-    if (!__syncthreads_or(big)) {
-        for (int b = t; b < br.y; b += kSisBlock) atomicAdd(&sBodies[island_root(parent, b)], 1);
-        for_runs([&](int, int2 bb, bool head, int, int len) {
-            if (head) atomicAdd(&sCnt[island_root(parent, bb.x - br.x)], len);
-        });
-        __syncthreads();
-    }
-    for (int b = t; b < br.y; b += kSisBlock)
-        big |= sCnt[b] > kIslandContacts || (sCnt[b] > 0 && sBodies[b] > kIslandBodies);
-    if (__syncthreads_or(big)) {
-        if (t == 0) {
-            levelRange[s] = rg;
-            atomicOr(gate, 1u);
-        }
+    if (__syncthreads_or(bad)) {
+        all_to_levels();
         return;
     }
+    for (int b = t; b < br.y; b += kSisBlock) atomicAdd(&sBodies[island_root(parent, b)], 1);
+    for_runs([&](int c, int2 bb, bool head, int, int len) {
+        if (head) atomicAdd(&sCnt[island_root(parent, bb.x - br.x)], len);
+        if (c >= rg.y) return;
+        levelList[c] = -1;
+        order[c] = -1;
+    });
+    __syncthreads();
+    // sBodies from here on: whether the root's island is small
+    bool large = false;
+    for (int b = t; b < br.y; b += kSisBlock) {
+        const bool fits = sCnt[b] <= kIslandContacts && sBodies[b] <= kIslandBodies;
+        large |= sCnt[b] > 0 && !fits;
+        sBodies[b] = fits ? 1 : 0;
+    }
+    large = __syncthreads_or(large);
     // islands numbered and their lists laid out in body order of their roots: four bodies a thread
     constexpr int kPer = kIslandSceneBodies / kSisBlock;
     int cnt[kPer], n = 0, contacts = 0;
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
         const int b = t * kPer + k;
-        cnt[k] = b < br.y ? sCnt[b] : 0;
+        cnt[k] = b < br.y && sBodies[b] ? sCnt[b] : 0;
         n += cnt[k] > 0 ? 1 : 0;
         contacts += cnt[k];
     }
@@ -824,7 +836,7 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_islands(const int2 *__restric
     }
     if (t == 0) {
         sBase = (int)atomicAdd(gate + 1, (unsigned)all);
-        levelRange[s] = make_int2(rg.x, rg.x);
+        if (!large) levelRange[s] = make_int2(rg.x, rg.x);
     }
     __syncthreads();
 #pragma unroll
@@ -837,12 +849,35 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_islands(const int2 *__restric
     }
     __syncthreads();
     for_runs([&](int c, int2 bb, bool head, int leader, int len) {
-        int slot = head ? atomicAdd(&sCnt[island_root(parent, bb.x - br.x)], len) : 0;
+        int slot = 0;
+        if (head) {
+            const int root = island_root(parent, bb.x - br.x);
+            slot = sBodies[root] ? atomicAdd(&sCnt[root], len) : -64;
+        }
         slot = __shfl(slot, leader, 64) + lane - leader;
-        if (c >= rg.y) return;
-        islandList[rg.x + slot] = c;
-        order[c] = c;   // (the level records of a scene without levels are formed, and not used)
+        if (c < rg.y && slot >= 0) islandList[rg.x + slot] = c;
     });
+    if (!large) return;
+    int kept = 0;
+    for (int c0 = rg.x; c0 < rg.y; c0 += kSisBlock) {
+        const int c = c0 + t;
+        const bool mine = c < rg.y && !sBodies[island_root(parent, bodies[c].x - br.x)];
+        const uint64_t m = __ballot(mine);
+        if (lane == 0) sWaveN[wave] = __popcll(m);
+        __syncthreads();
+        int before = 0, sum = 0;
+        for (int w = 0; w < kSisWaves; ++w) {
+            before += w < wave ? sWaveN[w] : 0;
+            sum += sWaveN[w];
+        }
+        if (mine) levelList[rg.x + kept + before + __popcll(m & ((1ull << lane) - 1))] = c;
+        kept += sum;
+        __syncthreads();
+    }
+    if (t == 0) {
+        levelRange[s] = make_int2(rg.x, rg.x + kept);
+        atomicOr(gate, 1u);
+    }
 }
 
 // Lane K's or a rotated lane's value within each quad of lanes (DPP quad_perm).
@@ -1132,10 +1167,12 @@ SisWork sis_work_layout(void *base, int cap, int numScenes, int numBodyParticles
     w.prep = (float4 *)take((size_t)kSisPlanes * cap * 16);
     w.blockCnt = (unsigned *)take(2 * (size_t)(nblk + 1) * 4);
     w.numContacts = (int *)take(4);
-    // the islands are found and swept after the gather's counts and before the levels' sort keys, in their place
+    // the islands are found and swept after the gather's counts and before the levels' sort keys, in their place; the
+    // levels' contacts are named until the records take theirs
     w.gate = w.blockCnt;
     w.island = (int2 *)w.keysA;
     w.islandList = (int *)w.valsA;
+    w.levelList = (int *)w.prep;
     w.levelRange = numScenes > 1 ? (int2 *)take((size_t)numScenes * 8) : w.sceneRange;   // (one scene's range is not stored)
     w.end = o;
     return w;
@@ -1163,14 +1200,14 @@ int launch_sis_solve(const SisContacts &ct, const SisBodies &bd, const SisSolveP
     launch_fill_u32(w.gate, 0u, 2, st);
     hipLaunchKernelGGL(k_sis_islands, dim3(numScenes), dim3(kSisBlock), 0, st, ct.bodies,
                        numScenes > 1 ? w.sceneRange : nullptr, w.numContacts, sceneBodies, numBodies, w.levelRange,
-                       w.gate, w.island, w.islandList, w.order);
+                       w.gate, w.island, w.islandList, w.levelList, w.order);
     const int most = cap < numBodies ? cap : numBodies;   // every island has a contact and a body
     if (most > 0 && iterations > 0)
         hipLaunchKernelGGL(k_sis_solve_islands, dim3(most), dim3(64), 0, st, ct, bd, ph, w.gate, w.island,
                            w.islandList, iterations);
-    // the scenes left to the levels (none: these launches end at their gate)
-    hipLaunchKernelGGL(k_sis_entries, dim3((ne + 255) / 256), dim3(256), 0, st, ct.bodies, w.numContacts, cap,
-                       invalid, w.gate, w.keysA, w.pred);
+    // what is left to the levels (nothing: these launches end at their gate)
+    hipLaunchKernelGGL(k_sis_entries, dim3((ne + 255) / 256), dim3(256), 0, st, ct.bodies, w.levelList,
+                       w.numContacts, cap, invalid, w.gate, w.keysA, w.pred);
     unsigned *kA = w.keysA, *kB = w.keysB, *vA = w.valsA, *vB = w.valsB;
     if (sort_pairs<unsigned>(&kA, &vA, &kB, &vB, ne, 0, bits, true, w.sortWs, w.sortWsBytes, tu, st, false, w.gate))
         return 1;
@@ -1178,7 +1215,7 @@ int launch_sis_solve(const SisContacts &ct, const SisBodies &bd, const SisSolveP
     const int2 *rg = w.levelRange;
     hipLaunchKernelGGL(k_sis_levels, dim3(numScenes), dim3(kSisBlock), 0, st, w.pred, rg, w.numContacts, w.lvl,
                        w.maxLvl);
-    hipLaunchKernelGGL(k_sis_bucket, dim3(numScenes), dim3(kSisBlock), 0, st, w.lvl, rg, w.numContacts, w.maxLvl,
+    hipLaunchKernelGGL(k_sis_bucket, dim3(numScenes), dim3(kSisBlock), 0, st, w.lvl, w.levelList, rg, w.numContacts, w.maxLvl,
                        w.off, w.cur, w.order);
     if (iterations > 0) {
         hipLaunchKernelGGL(k_sis_prep, dim3((cap + 255) / 256), dim3(256), 0, st, ct, bd, ph, w.numContacts, w.order,

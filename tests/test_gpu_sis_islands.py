@@ -1,6 +1,6 @@
 """Sequential-impulse sweeps of small islands (groups of contacts that share no body) against the oracle, bit
 for bit: contact lists at the edges of what an island may hold, interleaved in the list and with impulses
-already there, and engine scenes of which some take the islands and some the levels."""
+already there, beside larger ones that take the levels, and engine scenes of both kinds."""
 import ctypes as C
 
 import numpy as np
@@ -62,7 +62,7 @@ def solve_both(nb, pairs, seed, iterations=18):
     assert np.array_equal(con[4].get(), want["impulse"])
 
 
-# islands of (bodies, contacts); the last three have one that is too large, so the whole list takes the levels
+# islands of (bodies, contacts); the last five have some that are too large and take the levels
 @pytest.mark.parametrize("islands,shuffle", [
     ([(1, 1)], False),
     ([(2, 1), (1, 3), (2, 7)], True),
@@ -73,8 +73,11 @@ def solve_both(nb, pairs, seed, iterations=18):
     ([(1, 4)] * 4096, False),                   # the most bodies
     ([(16, 129), (2, 5)], True),
     ([(17, 40), (2, 5)], True),
+    ([(40, 500)] + [(2, 9)] * 300 + [(20, 33), (1, 1400)], True),
+    ([(2, 5)] * 150 + [(60, 2100)], False),
     ([(1, 2)] * 4097, False),
-], ids=["one", "three", "full", "seventy", "pairs", "quads", "bodies4096", "contacts129", "bodies17", "bodies4097"])
+], ids=["one", "three", "full", "seventy", "pairs", "quads", "bodies4096", "contacts129", "bodies17", "mixed",
+        "mixed_last", "bodies4097"])
 def test_solve_island_sizes_vs_oracle(islands, shuffle):
     print(f"sis islands: {len(islands)} groups, first {islands[0]}", flush=True)
     nb, pairs = contact_list(islands, shuffle, np.random.default_rng(len(islands)))
