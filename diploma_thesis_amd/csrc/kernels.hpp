@@ -378,8 +378,8 @@ struct SisWork {
     float4 *prep;                  // the sweeps' records in level order (planes of cap float4)
     unsigned *blockCnt;
     int *numContacts;
-    // small islands (launch_sis_solve): gate[0] = some contacts take the levels, gate[1] = islands listed;
-    // each island's (first slot of islandList, contacts); the contacts left to the levels and the scenes' ranges of
+    // islands (launch_sis_solve): gate[0] = some contacts take the levels, gate[1], gate[2] = small and medium ones
+    // listed; each one's (first slot of islandList, contacts); the contacts left to the levels and the scenes' ranges of
     // them.  In the place of blockCnt, keysA, valsA, prep and (one scene) sceneRange
     unsigned *gate;
     int2 *island;

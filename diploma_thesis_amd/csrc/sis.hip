@@ -687,13 +687,13 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_solve(float4 *__restrict__ re
     for (int k = rg.x + (int)threadIdx.x; k < rg.y; k += kSisBlock) impulse[order[k]] = rec[5 * P + k];
 }
 
-// ---- small islands.  Bodies that touch, directly or through others, form an island (the static points link
-// nothing), and the sweeps of one island read and write nothing of another's.  Small islands (thrown objects on
-// a scanned floor, stacks side by side) run side by side, each one's contacts one after another in contact
-// order with everything in LDS, instead of level by level in one workgroup a scene.  The contacts of larger islands
-// keep the levels, which advance with the longest chain: the stacked cubes after 800 steps, when some have spread
-// into one large island, 2,636 us a step with all contacts in the levels and 2,177 so.
-constexpr int kIslandContacts = 128, kIslandBodies = 16;   // what one island may hold
+// ---- islands.  Bodies that touch, directly or through others, form an island (the static points link
+// nothing), and the sweeps of one island read and write nothing of another's.  Islands of up to 1,024 contacts (thrown objects on
+// a scanned floor, stacks side by side) run side by side, each one's runs of contacts in the order they need
+// with everything in LDS, instead of level by level in one workgroup a scene.  The contacts of larger islands
+// keep the levels, which advance with the longest chain (864 levels at about 1.9 us in a step of the stacked cubes).
+constexpr int kIslandContacts = 128, kIslandBodies = 16;     // what one of a wave's islands may hold
+constexpr int kMediumContacts = 1024, kMediumBodies = 128;   // and one that takes a wave for itself
 constexpr int kIslandSceneBodies = 4096;                   // bodies of a scene whose islands are looked for
 
 __device__ __forceinline__ int island_root(const int *parent, int b) {
@@ -713,10 +713,11 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_islands(const int2 *__restric
                                                            const int *__restrict__ numContacts,
                                                            const int2 *__restrict__ sceneBodies, int numBodies,
                                                            int2 *__restrict__ levelRange, unsigned *__restrict__ gate,
-                                                           int2 *__restrict__ island, int *__restrict__ islandList,
-                                                           int *__restrict__ levelList, int *__restrict__ order) {
+                                                           int2 *__restrict__ island, int cap,
+                                                           int *__restrict__ islandList, int *__restrict__ levelList,
+                                                           int *__restrict__ order) {
     __shared__ int parent[kIslandSceneBodies], sCnt[kIslandSceneBodies], sBodies[kIslandSceneBodies];
-    __shared__ int sWaveN[kSisWaves], sWaveC[kSisWaves], sBase;
+    __shared__ int sWaveN[kSisWaves], sWaveC[kSisWaves], sBase, sMedium;
     const int s = blockIdx.x, t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
     const int2 rg = scene_range(sceneRange, numContacts, s);
     const int2 br = sceneBodies ? sceneBodies[s] : make_int2(0, numBodies);
@@ -796,22 +797,25 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_islands(const int2 *__restric
         order[c] = -1;
     });
     __syncthreads();
-    // sBodies from here on: whether the root's island is small
+    // sBodies from here on: the root's island takes the levels (0), a wave (1), a part of a wave (2)
     bool large = false;
     for (int b = t; b < br.y; b += kSisBlock) {
-        const bool fits = sCnt[b] <= kIslandContacts && sBodies[b] <= kIslandBodies;
-        large |= sCnt[b] > 0 && !fits;
-        sBodies[b] = fits ? 1 : 0;
+        const int n = sCnt[b], nb = sBodies[b];
+        const int cls = n <= kIslandContacts && nb <= kIslandBodies ? 2 : n <= kMediumContacts && nb <= kMediumBodies ? 1 : 0;
+        large |= n > 0 && cls == 0;
+        sBodies[b] = cls;
     }
     large = __syncthreads_or(large);
-    // islands numbered and their lists laid out in body order of their roots: four bodies a thread
+    // islands numbered (small ones from the list's front, the others from its back) and their contacts' places laid
+    // out in body order of their roots: four bodies a thread
     constexpr int kPer = kIslandSceneBodies / kSisBlock;
+    constexpr int kMediumOne = 1 << 16;   // n: small islands, and medium ones in the upper half
     int cnt[kPer], n = 0, contacts = 0;
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-        const int b = t * kPer + k;
-        cnt[k] = b < br.y && sBodies[b] ? sCnt[b] : 0;
-        n += cnt[k] > 0 ? 1 : 0;
+        const int b = t * kPer + k, cls = b < br.y ? sBodies[b] : 0;
+        cnt[k] = cls ? sCnt[b] : 0;
+        n += cnt[k] > 0 ? (cls == 2 ? 1 : kMediumOne) : 0;
         contacts += cnt[k];
     }
     int xn = n, xc = contacts;
@@ -835,7 +839,8 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_islands(const int2 *__restric
         all += sWaveN[w];
     }
     if (t == 0) {
-        sBase = (int)atomicAdd(gate + 1, (unsigned)all);
+        sBase = (int)atomicAdd(gate + 1, (unsigned)(all & (kMediumOne - 1)));
+        sMedium = all / kMediumOne ? (int)atomicAdd(gate + 2, (unsigned)(all / kMediumOne)) : 0;
         if (!large) levelRange[s] = make_int2(rg.x, rg.x);
     }
     __syncthreads();
@@ -843,7 +848,10 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_islands(const int2 *__restric
     for (int k = 0; k < kPer; ++k) {
         const int b = t * kPer + k;
         if (cnt[k] <= 0) continue;
-        island[sBase + at++] = make_int2(rg.x + first, cnt[k]);
+        const bool small = sBodies[b] == 2;
+        island[small ? sBase + (at & (kMediumOne - 1)) : cap - 1 - (sMedium + at / kMediumOne)] =
+            make_int2(rg.x + first, cnt[k]);
+        at += small ? 1 : kMediumOne;
         sCnt[b] = first;
         first += cnt[k];
     }
@@ -852,7 +860,7 @@ __global__ __launch_bounds__(kSisBlock) void k_sis_islands(const int2 *__restric
         int slot = 0;
         if (head) {
             const int root = island_root(parent, bb.x - br.x);
-            slot = sBodies[root] ? atomicAdd(&sCnt[root], len) : -64;
+            slot = sBodies[root] ? atomicAdd(&sCnt[root], len) : -64;   // (a run is no longer than 64)
         }
         slot = __shfl(slot, leader, 64) + lane - leader;
         if (c < rg.y && slot >= 0) islandList[rg.x + slot] = c;
@@ -895,207 +903,303 @@ __device__ __forceinline__ float q_dot(float a, float b) {
     return (q_0(m) + q_1(m)) + q_2(m);
 }
 
-// The sweeps of the islands, eight lanes an island and up to four islands a wave.  An island's contacts are one
-// dependent chain (48 contacts for a stack of two cubes on the floor, 18 sweeps of them), so what counts is the
-// time of one contact: lane c of a quad holds component c of every vector, the first quad the contact's first
-// body and the second quad its partner; of a static contact's three impulses lane c divides and clamps its
-// own.  Every sum and product is that of sis_contact, in its order.  Contacts are taken in runs of one pair of
-// bodies, which stay in registers for the run, and the next contact's record is read while this one is worked on.
+// The sweeps of the islands by single waves, eight lanes a contact: lane c of a quad holds component c of every
+// vector, the first quad the contact's first body and the second quad its partner; of a static contact's three
+// impulses lane c divides and clamps its own.  Every sum and product is that of sis_contact, in its order.
+// Contacts are taken in runs of one pair of bodies, which stay in registers for the run.  A run waits for the last
+// run before it that has one of its bodies; runs of one level of that order touch different bodies and go to
+// different lanes: the eight groups of a wave share its islands (one medium island, or up to eight small ones).
+// What counts is the time of one contact of a dependent chain (two stacked cubes on the floor have 48 contacts,
+// and there are 18 sweeps), so the words of the next contact are read one contact ahead, by addresses that only step.
 // One wave a workgroup and islands added to a wave only when there are more than CUs: waves that share a CU slow
 // each other down about as much as they add, islands in one wave run in step.  The sweeps of the stacked-cubes
 // scene (1,024 islands of 48 contacts): the levels in one workgroup 1,672 us; one island a wave 580, with four waves a
-// workgroup 613; so 312.  64 islands, the whole solve: 295 us, with four waves a workgroup 606, the levels 719.
-constexpr int kWaveIslands = 4;   // islands a wave takes at most
+// workgroup 613; four islands a wave 312; with stepping addresses 273; with the runs by level 231.  After 800 steps, when islands of
+// up to a few hundred contacts have formed, a step takes 585 us; 2,177 with those in the levels.
+constexpr int kWaveGroups = 8;   // of eight lanes
+constexpr int kIslandCus = 256;
 __device__ __forceinline__ void wave_sync() {   // LDS written by the wave's lanes, read by others of them
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 }
+template <int SLOTS, int BODIES>
 struct IslandLds {
-    float4 rec[kSisPlanes * kIslandContacts], vel[kIslandBodies * 2];
-    float inertia[kIslandBodies * 9];
-    int key[kIslandContacts], ord[kIslandContacts], body[2 * kIslandContacts], first[2 * kIslandContacts];
-    int2 count;                     // contacts, bodies
-    int ids[kIslandBodies], run[kIslandContacts + 1];   // run: first contacts of the runs of one pair
+    float4 rec[kSisPlanes * SLOTS], vel[2 * BODIES];
+    float inertia[9 * BODIES], dump;
+    int ord[SLOTS], pair[2 * SLOTS];   // the contacts in contact order, and their bodies as indices of ids (static: -1)
+    int ids[BODIES], bodyLevel[BODIES];
+    int run[SLOTS + 1], runLevel[SLOTS], runOrd[SLOTS], levelOff[SLOTS + 1];   // first contacts of the runs; by level
+    int key[SLOTS];
+    int contacts, bodies, levels;
 };
-__global__ __launch_bounds__(64) void k_sis_solve_islands(SisContacts ct, SisBodies bd, SisSolvePhys ph,
-                                                          const unsigned *__restrict__ gate,
-                                                          const int2 *__restrict__ island,
-                                                          const int *__restrict__ islandList, int iterations) {
-    constexpr int kSlots = kIslandContacts;
-    __shared__ IslandLds sAll[kWaveIslands];
-    const int lane = (int)threadIdx.x;
-    const unsigned islands = gate[1];
-    int per = 1;   // islands of this wave: one a CU as long as there are CUs
-    while (per < kWaveIslands && (unsigned)per * 256u < islands) per *= 2;
-    const unsigned g0 = blockIdx.x * (unsigned)per;
-    if (g0 >= islands) return;
-    int myN = 0, myRuns = 0;   // of the island that this lane's eight lanes take
-    for (int q = 0; q < per; ++q) {
-        IslandLds &I = sAll[q];
-        float4 *sRec = I.rec, *sVel = I.vel;
-        float *sI = I.inertia;
-        int *sKey = I.key, *sOrd = I.ord, *sBody = I.body, *sFirst = I.first, *sIds = I.ids, *sRun = I.run;
-        const int2 is = g0 + (unsigned)q < islands ? island[g0 + (unsigned)q] : make_int2(0, 0);
-        const int n = is.y;
-        // the contacts in contact order: a contact's place is the number of smaller ones
-        for (int k = lane; k < n; k += 64) sKey[k] = islandList[is.x + k];
-        wave_sync();
-        for (int k = lane; k < n; k += 64) {
-            const int key = sKey[k];
-            int r = 0;
-            for (int j = 0; j < n; ++j) r += sKey[j] < key ? 1 : 0;
-            sOrd[r] = key;
+
+// Loads one island (first slot of islandList, contacts) and lays out its runs.
+template <int SLOTS, int BODIES>
+__device__ __forceinline__ void island_load(IslandLds<SLOTS, BODIES> &I, int2 is, const SisContacts &ct,
+                                            const SisBodies &bd, const SisSolvePhys &ph,
+                                            const int *__restrict__ islandList) {
+    const int lane = (int)threadIdx.x, n = is.y;
+    const uint64_t below = (1ull << lane) - 1;
+    // the contacts in contact order: a contact's place is the number of smaller ones
+    for (int k = lane; k < n; k += 64) I.key[k] = islandList[is.x + k];
+    wave_sync();
+    for (int k = lane; k < n; k += 64) {
+        const int key = I.key[k];
+        int r = 0;
+#pragma unroll 4
+        for (int j = 0; j < n; ++j) r += I.key[j] < key ? 1 : 0;
+        I.ord[r] = key;
+    }
+    wave_sync();
+    // the bodies, numbered as they appear
+    int ids = 0;
+    for (int e0 = 0; e0 < 2 * n; e0 += 64) {
+        const int e = e0 + lane;
+        int b = -1, id = -1;
+        if (e < 2 * n) {
+            const int2 bb = ct.bodies[I.ord[e >> 1]];
+            b = e & 1 ? bb.y : bb.x;
         }
-        wave_sync();
-        // the bodies, numbered by their first appearance among the contacts' (b1, b2)
-        for (int k = lane; k < n; k += 64) {
-            const int2 bb = ct.bodies[sOrd[k]];
-            sBody[2 * k] = bb.x;
-            sBody[2 * k + 1] = bb.y;
+#pragma unroll 4
+        for (int j = 0; j < ids; ++j) id = I.ids[j] == b ? j : id;
+        uint64_t m = __ballot(b >= 0 && id < 0);
+        while (m) {
+            const int nb = __shfl(b, __ffsll((long long)m) - 1, 64);
+            if (b == nb) id = ids;
+            if (lane == 0) I.ids[ids] = nb;
+            ++ids;
+            m = __ballot(b >= 0 && id < 0);
         }
-        wave_sync();
-        int ids = 0;
-        for (int e0 = 0; e0 < 2 * n; e0 += 64) {
-            const int e = e0 + lane;
-            const int b = e < 2 * n ? sBody[e] : -1;
-            int f = e;
-            for (int j = 2 * n - 1; j >= 0; --j) f = sBody[j] == b && j < f ? j : f;
-            const uint64_t m = __ballot(b >= 0 && f == e);
-            if (b >= 0 && f == e) {
-                const int id = ids + (int)__popcll(m & (lane == 0 ? 0ull : (~0ull >> (64 - lane))));
-                sIds[id] = b;
-                sFirst[e] = id;
-            }
-            ids += (int)__popcll(m);
-            wave_sync();
-            if (b >= 0 && f != e) sFirst[e] = sFirst[f];
-        }
-        wave_sync();
-        for (int k = lane; k < ids; k += 64) {
-            const int b = sIds[k];
-            sVel[2 * k] = bd.vel[b];
-            sVel[2 * k + 1] = bd.ang[b];
-            for (int i = 0; i < 9; ++i) sI[9 * k + i] = bd.Iw[9 * (size_t)b + i];
-        }
-        for (int k = lane; k < n; k += 64)
-            sis_record(ct, bd, ph, sOrd[k], sFirst[2 * k], sFirst[2 * k + 1], sRec, kSlots, k);
-        wave_sync();
-        int runs = 0;
-        for (int e0 = 0; e0 < n; e0 += 64) {
-            const int k = e0 + lane;
-            const bool head = k < n && (k == 0 || sBody[2 * k] != sBody[2 * k - 2] || sBody[2 * k + 1] != sBody[2 * k - 1]);
-            const uint64_t m = __ballot(head);
-            if (head) sRun[runs + (int)__popcll(m & (lane == 0 ? 0ull : (~0ull >> (64 - lane))))] = k;
-            runs += (int)__popcll(m);
-        }
-        if (lane == 0) {
-            sRun[runs] = n;
-            I.count = make_int2(n, ids);
-        }
-        if ((lane >> 3) == q) {
-            myN = n;
-            myRuns = runs;
-        }
+        if (e < 2 * n) I.pair[e] = id;
         wave_sync();
     }
-    if (myN > 0) {
-        IslandLds &I = sAll[lane >> 3];
-        float4 *sRec = I.rec, *sVel = I.vel;
-        const float *sI = I.inertia;
-        const int *sRun = I.run, runs = myRuns, sub = lane & 7;
-        const int c = lane & 3, c0 = c < 3 ? c : 0, cn = c0 == 2 ? 0 : c0 + 1, ca = c0 == 0 ? 2 : c0 - 1;
-        const bool second = sub >= 4;
-        float *R = reinterpret_cast<float *>(sRec), *V = reinterpret_cast<float *>(sVel);
-        auto word = [&](int plane, int k, int w) { return R[4 * (plane * kSlots + k) + w]; };
-        int at = -1, at1 = -1, at2 = -1;   // the quad's body (-1: none of its own), and the pair held
-        float v = 0.f, w = 0.f, i0 = 0.f, i3 = 0.f, i6 = 0.f, mass = 1.f;
-        auto put_back = [&]() {
-            if (at < 0) return;
-            V[8 * at + c] = c < 3 ? v : 0.0f;
-            V[8 * at + 4 + c] = c < 3 ? w : 0.0f;
-        };
-        // the impulse J moves the quad's body: v += J / m, w += I^-1 (p x J) (the partner: -=)
-        auto apply = [&](float J, float pn, float pa, bool minus) {
-            const float dv = J / mass;
-            const float pj = pn * q_after(J) - pa * q_next(J);
-            const float dw = i0 * q_0(pj) + i3 * q_1(pj) + i6 * q_2(pj);
-            v = minus ? v - dv : v + dv;
-            w = minus ? w - dw : w + dw;
-        };
-        for (int it = 0; it < iterations; ++it)
-            for (int r = 0; r < runs; ++r) {
-                const int k0 = sRun[r], k1 = sRun[r + 1];
+    for (int k = lane; k < ids; k += 64) {
+        const int b = I.ids[k];
+        I.vel[2 * k] = bd.vel[b];
+        I.vel[2 * k + 1] = bd.ang[b];
+        for (int i = 0; i < 9; ++i) I.inertia[9 * k + i] = bd.Iw[9 * (size_t)b + i];
+        I.bodyLevel[k] = 0;
+    }
+    for (int k = lane; k < n; k += 64)
+        sis_record(ct, bd, ph, I.ord[k], I.pair[2 * k], I.pair[2 * k + 1], I.rec, SLOTS, k);
+    int runs = 0;
+    for (int e0 = 0; e0 < n; e0 += 64) {
+        const int k = e0 + lane;
+        const bool head = k < n && (k == 0 || I.pair[2 * k] != I.pair[2 * k - 2] || I.pair[2 * k + 1] != I.pair[2 * k - 1]);
+        const uint64_t m = __ballot(head);
+        if (head) I.run[runs + (int)__popcll(m & below)] = k;
+        runs += (int)__popcll(m);
+    }
+    wave_sync();
+    int levels = 0;
+    if (lane == 0) {
+        I.run[runs] = n;
+        for (int r = 0; r < runs; ++r) {
+            const int k = I.run[r], b1 = I.pair[2 * k], b2 = I.pair[2 * k + 1];
+            int l = I.bodyLevel[b1];
+            if (b2 >= 0) {
+                l = max(l, I.bodyLevel[b2]);
+                I.bodyLevel[b2] = l + 1;
+            }
+            I.bodyLevel[b1] = l + 1;
+            I.runLevel[r] = l;
+            levels = max(levels, l + 1);
+        }
+        I.contacts = n;
+        I.bodies = ids;
+        I.levels = levels;
+        I.levelOff[levels] = runs;
+    }
+    wave_sync();
+    // the runs by level (every level up to the last has one)
+    for (int k = lane; k < runs; k += 64) {
+        const int l = I.runLevel[k];
+        int r = 0, first = 0;
+#pragma unroll 4
+        for (int j = 0; j < runs; ++j) {
+            const int lj = I.runLevel[j];
+            first += lj < l ? 1 : 0;
+            r += lj < l || (lj == l && j < k) ? 1 : 0;
+        }
+        I.runOrd[r] = k;
+        I.levelOff[l] = first;
+    }
+    wave_sync();
+}
+
+template <int SLOTS, int BODIES>
+__device__ __forceinline__ void island_store(const IslandLds<SLOTS, BODIES> &I, const SisContacts &ct,
+                                             const SisBodies &bd) {
+    const int lane = (int)threadIdx.x;
+    for (int k = lane; k < I.bodies; k += 64) {
+        const int b = I.ids[k];
+        bd.vel[b] = I.vel[2 * k];
+        bd.ang[b] = I.vel[2 * k + 1];
+    }
+    for (int k = lane; k < I.contacts; k += 64) ct.impulse[I.ord[k]] = I.rec[5 * SLOTS + k];
+}
+
+// The sweeps of an island by `groups` of the wave's groups, of which this lane's is the `group`-th.
+template <int SLOTS, int BODIES>
+__device__ __forceinline__ void island_sweep(IslandLds<SLOTS, BODIES> &I, int group, int groups, int iterations) {
+    constexpr int kSlots = SLOTS;
+    const int sub = (int)threadIdx.x & 7;
+    const int c = sub & 3, c0 = c < 3 ? c : 0, cn = c0 == 2 ? 0 : c0 + 1, ca = c0 == 0 ? 2 : c0 - 1;
+    const bool second = sub >= 4;
+    float *R = reinterpret_cast<float *>(I.rec), *V = reinterpret_cast<float *>(I.vel);
+    const float *sI = I.inertia;
+    auto word = [&](int plane, int k, int w) { return R[4 * (plane * kSlots + k) + w]; };
+    const int levels = I.levels;
+    for (int it = 0; it < iterations; ++it)
+        for (int L = 0; L < levels; ++L) {
+            const int last = I.levelOff[L + 1];
+            for (int r = I.levelOff[L] + group; r < last; r += groups) {
+                const int run = I.runOrd[r], k0 = I.run[run], k1 = I.run[run + 1];
                 const int b1 = __float_as_int(word(4, k0, 0)), b2 = __float_as_int(word(4, k0, 1));
-                if (b1 != at1 || b2 != at2) {
-                    put_back();
-                    wave_sync();
-                    at1 = b1;
-                    at2 = b2;
-                    at = second ? b2 : b1;
-                    const int b = at < 0 ? b1 : at;   // (a static contact's second quad works along with the first)
-                    v = V[8 * b + c];
-                    w = V[8 * b + 4 + c];
-                    i0 = sI[9 * b + c0];
-                    i3 = sI[9 * b + 3 + c0];
-                    i6 = sI[9 * b + 6 + c0];
-                    mass = word(4, k0, second && b2 >= 0 ? 3 : 2);   // (a body contact's word 3 is its partner's mass)
-                }
+                // the quad's body (a static contact's second quad works along with the first)
+                const bool own = !second || b2 >= 0;
+                const int b = second && b2 >= 0 ? b2 : b1;
+                float v = V[8 * b + c], w = V[8 * b + 4 + c];
+                const float i0 = sI[9 * b + c0], i3 = sI[9 * b + 3 + c0], i6 = sI[9 * b + 6 + c0];
+                const float mass = word(4, k0, second && b2 >= 0 ? 3 : 2);   // (a body contact's word 3 is its partner's)
+                // the impulse J moves the quad's body: v += J / m, w += I^-1 (p x J) (the partner: -=)
+                auto apply = [&](float J, float pn, float pa, bool minus) {
+                    const float dv = J / mass;
+                    const float pj = pn * q_after(J) - pa * q_next(J);
+                    const float dw = i0 * q_0(pj) + i3 * q_1(pj) + i6 * q_2(pj);
+                    v = minus ? v - dv : v + dv;
+                    w = minus ? w - dw : w + dw;
+                };
+                // The lane's words of contact k, and where it leaves its impulse (the lanes without one: a word nobody
+                // reads).  The next contact's words are read one contact ahead, past the run's end too.
+                const float *P = R + 4 * ((b2 >= 0 && second ? 2 : 1) * kSlots + k0), *N = R + 4 * k0;
+                const float *Pn = P + cn, *Pa = P + ca, *Nn = N + c0, *Nb = N + 3;
+                const bool writes = b2 < 0 ? sub < 3 : sub == 0;
+                float *Wr = writes ? R + 4 * (5 * kSlots + k0) + sub : &I.dump;
+                const int wStep = writes ? 4 : 0;
+                int left = k1 - k0;
                 if (b2 < 0) {
-                    float pn = word(1, k0, cn), pa = word(1, k0, ca), nn = word(0, k0, c0), t = word(2, k0, c0),
-                          t2 = word(3, k0, c0), bias = word(0, k0, 3), den = word(1 + c0, k0, 3), fb = word(4, k0, 3),
-                          acc = word(5, k0, c0);
-                    for (int k = k0; k < k1; ++k) {
-                        const int kn = k + 1 < k1 ? k + 1 : k;
-                        const float pn_ = word(1, kn, cn), pa_ = word(1, kn, ca), nn_ = word(0, kn, c0),
-                                    t_ = word(2, kn, c0), t2_ = word(3, kn, c0), bias_ = word(0, kn, 3),
-                                    den_ = word(1 + c0, kn, 3), fb_ = word(4, kn, 3), acc_ = word(5, kn, c0);
-                        const float vp = v + (q_next(w) * pa - q_after(w) * pn);   // v + w x p
-                        const float d0 = q_dot(vp, nn), d1 = q_dot(vp, t), d2 = q_dot(vp, t2);
-                        const float num = c0 == 0 ? -(d0 + bias) : -(c0 == 1 ? d1 : d2);
-                        const float lo = c0 == 0 ? 0.0f : -fb, hi = c0 == 0 ? 100.0f : fb;
-                        float tmp = acc + num / den;
+                    struct Words {
+                        float pn, pa, nn, t, t2, bias, den, fb, acc;
+                    } A, B;
+                    const float *Dn = R + 4 * ((1 + c0) * kSlots + k0) + 3;
+                    auto read = [&](Words &o, int i) {
+                        o.pn = Pn[4 * i];
+                        o.pa = Pa[4 * i];
+                        o.nn = Nn[4 * i];
+                        o.t = Nn[4 * (2 * kSlots + i)];
+                        o.t2 = Nn[4 * (3 * kSlots + i)];
+                        o.bias = Nb[4 * i];
+                        o.den = Dn[4 * i];
+                        o.fb = Nb[4 * (4 * kSlots + i)];
+                        o.acc = Nn[4 * (5 * kSlots + i)];
+                    };
+                    auto contact = [&](const Words &o) {
+                        const float vp = v + (q_next(w) * o.pa - q_after(w) * o.pn);   // v + w x p
+                        const float d0 = q_dot(vp, o.nn), d1 = q_dot(vp, o.t), d2 = q_dot(vp, o.t2);
+                        const float num = c0 == 0 ? -(d0 + o.bias) : -(c0 == 1 ? d1 : d2);
+                        const float lo = c0 == 0 ? 0.0f : -o.fb, hi = c0 == 0 ? 100.0f : o.fb;
+                        float tmp = o.acc + num / o.den;
                         tmp = tmp < lo ? lo : (tmp > hi ? hi : tmp);
-                        const float d = tmp - acc;
-                        if (sub < 3) R[4 * (5 * kSlots + k) + sub] = tmp;
-                        apply((q_0(d) * nn + q_1(d) * t) + q_2(d) * t2, pn, pa, false);
-                        pn = pn_; pa = pa_; nn = nn_; t = t_; t2 = t2_; bias = bias_; den = den_; fb = fb_; acc = acc_;
+                        const float d = tmp - o.acc;
+                        *Wr = tmp;
+                        Wr += wStep;
+                        apply((q_0(d) * o.nn + q_1(d) * o.t) + q_2(d) * o.t2, o.pn, o.pa, false);
+                    };
+                    read(A, 0);
+                    while (true) {
+                        read(B, 1);
+                        contact(A);
+                        if (--left == 0) break;
+                        read(A, 2);
+                        Pn += 8;
+                        Pa += 8;
+                        Nn += 8;
+                        Nb += 8;
+                        Dn += 8;
+                        contact(B);
+                        if (--left == 0) break;
                     }
                 } else {
-                    const int pp = second ? 2 : 1;
-                    float pn = word(pp, k0, cn), pa = word(pp, k0, ca), nn = word(0, k0, c0), bias = word(0, k0, 3),
-                          den = word(1, k0, 3), acc = word(5, k0, 0);
-                    for (int k = k0; k < k1; ++k) {
-                        const int kn = k + 1 < k1 ? k + 1 : k;
-                        const float pn_ = word(pp, kn, cn), pa_ = word(pp, kn, ca), nn_ = word(0, kn, c0),
-                                    bias_ = word(0, kn, 3), den_ = word(1, kn, 3), acc_ = word(5, kn, 0);
-                        const float vp = v + (q_next(w) * pa - q_after(w) * pn);
-                        const float s = q_dot(vp, nn);
+                    struct Words {
+                        float pn, pa, nn, bias, den, acc;
+                    } A, B;
+                    auto read = [&](Words &o, int i) {
+                        o.pn = Pn[4 * i];
+                        o.pa = Pa[4 * i];
+                        o.nn = Nn[4 * i];
+                        o.bias = Nb[4 * i];
+                        o.den = Nb[4 * (kSlots + i)];
+                        o.acc = Nb[4 * (5 * kSlots + i) - 3];
+                    };
+                    auto contact = [&](const Words &o) {
+                        const float vp = v + (q_next(w) * o.pa - q_after(w) * o.pn);
+                        const float s = q_dot(vp, o.nn);
                         // the first body's minus the partner's, in both quads (DPP row_shl / row_shr by four lanes)
                         const float up = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x104, 0xf, 0xf, true));
                         const float dn = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x114, 0xf, 0xf, true));
-                        const float num = -((second ? dn - s : s - up) + bias);
-                        float tmp = acc + num / den;
+                        const float num = -((second ? dn - s : s - up) + o.bias);
+                        float tmp = o.acc + num / o.den;
                         tmp = tmp < 0.0f ? 0.0f : (tmp > 100.0f ? 100.0f : tmp);
-                        const float d = tmp - acc;
-                        if (sub == 0) R[4 * (5 * kSlots + k)] = tmp;
-                        apply(d * nn, pn, pa, second);
-                        pn = pn_; pa = pa_; nn = nn_; bias = bias_; den = den_; acc = acc_;
+                        *Wr = tmp;
+                        Wr += wStep;
+                        apply((tmp - o.acc) * o.nn, o.pn, o.pa, second);
+                    };
+                    read(A, 0);
+                    while (true) {
+                        read(B, 1);
+                        contact(A);
+                        if (--left == 0) break;
+                        read(A, 2);
+                        Pn += 8;
+                        Pa += 8;
+                        Nn += 8;
+                        Nb += 8;
+                        contact(B);
+                        if (--left == 0) break;
                     }
                 }
+                if (own) {
+                    V[8 * b + c] = c < 3 ? v : 0.0f;
+                    V[8 * b + 4 + c] = c < 3 ? w : 0.0f;
+                }
             }
-        put_back();
-    }
-    wave_sync();
-    for (int q = 0; q < per; ++q) {
-        const IslandLds &I = sAll[q];
-        const int n = I.count.x, ids = I.count.y;
-        for (int k = lane; k < ids; k += 64) {
-            const int b = I.ids[k];
-            bd.vel[b] = I.vel[2 * k];
-            bd.ang[b] = I.vel[2 * k + 1];
+            wave_sync();
         }
-        for (int k = lane; k < n; k += 64) ct.impulse[I.ord[k]] = I.rec[5 * kSlots + k];
+}
+
+// The first blocks take the medium islands, the others up to eight small ones each.
+__global__ __launch_bounds__(64) void k_sis_solve_islands(SisContacts ct, SisBodies bd, SisSolvePhys ph,
+                                                          const unsigned *__restrict__ gate,
+                                                          const int2 *__restrict__ island, int cap, int mediumBlocks,
+                                                          const int *__restrict__ islandList, int iterations) {
+    __shared__ union {
+        IslandLds<kIslandContacts, kIslandBodies> small[kWaveGroups];
+        IslandLds<kMediumContacts, kMediumBodies> medium;
+    } lds;
+    const int lane = (int)threadIdx.x;
+    if ((int)blockIdx.x < mediumBlocks) {
+        for (int m = (int)blockIdx.x; m < (int)gate[2]; m += mediumBlocks) {
+            island_load(lds.medium, island[cap - 1 - m], ct, bd, ph, islandList);
+            island_sweep(lds.medium, lane >> 3, kWaveGroups, iterations);
+            wave_sync();
+            island_store(lds.medium, ct, bd);
+            wave_sync();
+        }
+        return;
     }
+    const unsigned islands = gate[1];
+    int per = 1;   // islands of this wave: one a CU as long as there are CUs
+    while (per < kWaveGroups && per * kIslandCus < (int)islands) per *= 2;
+    const unsigned g0 = (blockIdx.x - (unsigned)mediumBlocks) * (unsigned)per;
+    if (g0 >= islands) return;
+    for (int q = 0; q < per; ++q)
+        island_load(lds.small[q], g0 + (unsigned)q < islands ? island[g0 + (unsigned)q] : make_int2(0, 0), ct, bd, ph,
+                    islandList);
+    const int groups = kWaveGroups / per;
+    island_sweep(lds.small[(lane >> 3) / groups], (lane >> 3) % groups, groups, iterations);
+    wave_sync();
+    for (int q = 0; q < per; ++q) island_store(lds.small[q], ct, bd);
 }
 
 }  // namespace
@@ -1197,14 +1301,19 @@ int launch_sis_solve(const SisContacts &ct, const SisBodies &bd, const SisSolveP
     const unsigned invalid = (unsigned)numBodies;
     int bits = 1;
     while (bits < 32 && (invalid >> bits) != 0u) ++bits;
-    launch_fill_u32(w.gate, 0u, 2, st);
+    launch_fill_u32(w.gate, 0u, 3, st);
     hipLaunchKernelGGL(k_sis_islands, dim3(numScenes), dim3(kSisBlock), 0, st, ct.bodies,
                        numScenes > 1 ? w.sceneRange : nullptr, w.numContacts, sceneBodies, numBodies, w.levelRange,
-                       w.gate, w.island, w.islandList, w.levelList, w.order);
-    const int most = cap < numBodies ? cap : numBodies;   // every island has a contact and a body
-    if (most > 0 && iterations > 0)
-        hipLaunchKernelGGL(k_sis_solve_islands, dim3(most), dim3(64), 0, st, ct, bd, ph, w.gate, w.island,
-                           w.islandList, iterations);
+                       w.gate, w.island, cap, w.islandList, w.levelList, w.order);
+    // every island has a contact and a body, a medium one more of either than a small one may have; the small ones'
+    // blocks are no more than the CUs until each takes kWaveGroups
+    const int islands = cap < numBodies ? cap : numBodies, waves = (islands + kWaveGroups - 1) / kWaveGroups;
+    const int small = islands < kIslandCus ? islands : waves > kIslandCus ? waves : kIslandCus;
+    int medium = cap / (kIslandContacts + 1) + numBodies / (kIslandBodies + 1);
+    if (medium > kIslandCus) medium = kIslandCus;
+    if (small > 0 && iterations > 0)
+        hipLaunchKernelGGL(k_sis_solve_islands, dim3(medium + small), dim3(64), 0, st, ct, bd, ph, w.gate, w.island, cap,
+                           medium, w.islandList, iterations);
     // what is left to the levels (nothing: these launches end at their gate)
     hipLaunchKernelGGL(k_sis_entries, dim3((ne + 255) / 256), dim3(256), 0, st, ct.bodies, w.levelList,
                        w.numContacts, cap, invalid, w.gate, w.keysA, w.pred);

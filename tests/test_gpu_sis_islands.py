@@ -62,7 +62,7 @@ def solve_both(nb, pairs, seed, iterations=18):
     assert np.array_equal(con[4].get(), want["impulse"])
 
 
-# islands of (bodies, contacts); the last five have some that are too large and take the levels
+# islands of (bodies, contacts): up to 16 bodies and 128 contacts share a wave, up to 128 and 1,024 take one
 @pytest.mark.parametrize("islands,shuffle", [
     ([(1, 1)], False),
     ([(2, 1), (1, 3), (2, 7)], True),
@@ -75,9 +75,14 @@ def solve_both(nb, pairs, seed, iterations=18):
     ([(17, 40), (2, 5)], True),
     ([(40, 500)] + [(2, 9)] * 300 + [(20, 33), (1, 1400)], True),
     ([(2, 5)] * 150 + [(60, 2100)], False),
+    ([(128, 1024), (3, 7)], False),
+    ([(128, 1024), (100, 1024), (2, 3)], True),
+    ([(129, 600), (2, 5)], True),
+    ([(20, 1025), (5, 40)], True),
+    ([(17, 20)] * 230, True),
     ([(1, 2)] * 4097, False),
 ], ids=["one", "three", "full", "seventy", "pairs", "quads", "bodies4096", "contacts129", "bodies17", "mixed",
-        "mixed_last", "bodies4097"])
+        "mixed_last", "wave_full", "wave_two", "bodies129", "contacts1025", "waves230", "bodies4097"])
 def test_solve_island_sizes_vs_oracle(islands, shuffle):
     print(f"sis islands: {len(islands)} groups, first {islands[0]}", flush=True)
     nb, pairs = contact_list(islands, shuffle, np.random.default_rng(len(islands)))
