@@ -197,7 +197,8 @@ void launch_pose_key_tiles(const PartBufs &p, const BodyBufs &b, int numParticle
 // number of grid periods long the hashed cells are unevenly filled, and the plan then expects the
 // fullest bucket to hold ceil(r) / r times the average along each axis a bucket does not span,
 // r = extent / grid size.  A scene that kept its shift from an earlier plan (a rebuild) passes it.
-// False when a scene needs more buckets than its tiles can rank or more than 384 tiles.
+// False when a scene needs more buckets than its tiles can rank or more than 384 tiles, and for grid keys where
+// the fullest measured bucket is too full at every width.
 struct BucketSceneShape {
     long long particles = 0;
     unsigned grid[3] = {1, 1, 1};
