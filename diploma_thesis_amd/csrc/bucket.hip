@@ -563,12 +563,14 @@ bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *o
             }
         }
         // No width fits a scene whose particles crowd into few of its cells (a settled pile in a tall box: at 250,000
-        // particles 78 of 1,024 buckets have any, and 6,900 keys each).  Alone on the chip such buckets take
-        // longer than the digit passes and the reorder (sort 94 against 73 us; at 10^6 240 against 98, where they no longer
-        // fit in LDS); six piles of 210,000 whose buckets do fit fill it, and take 117 against 180 us.
+        // particles 78 of 1,024 buckets have any, up to 6,900 keys each, a key's bucket 5,000 on average).  Alone on
+        // the chip such buckets take longer than the digit passes and the reorder (97 us against 73; at 10^6 240
+        // against 98; a scene of 120,000 in one layer 228 against 86), but not a scene of 20,000 (54 against 75) nor
+        // buckets of which only a few are so full.  Other scenes beside it fill the chip unless its fullest bucket
+        // does not fit in LDS (a pile of 10^6 and 40 mixed scenes 373 against 188, at 190,000 particles 90 against 93).
         // Morton buckets of a pile of 50,000 that exceed the LDS: 15 us against 48.
-        if (shift < 0 && measured && !sharedCells &&
-            (S == 1 || (narrowest >= 0 && sc.peak[narrowest] > (unsigned)capKeys)))
+        if (shift < 0 && measured && !sharedCells && sc.load > 0.5 * capKeys &&
+            (S == 1 ? nTot > 65536 : nTot > (3 << 16) && narrowest >= 0 && sc.peak[narrowest] > (unsigned)capKeys))
             return false;
         if (shift < 0) shift = narrowest;
         if (sc.shift >= 0 && sc.shift <= maxShift && ((c + (1ll << sc.shift) - 1) >> sc.shift) <= maxBuckets)

@@ -364,7 +364,7 @@ namespace {
 
 // The fullest bucket of a scene's grid keys for every bucket width 2^b cells (b = 0..16, UINT_MAX
 // where there would be more than 1024 buckets), from host positions (float4 per particle).
-std::vector<unsigned> bucket_peaks(const float *pos4, int n, const SceneGeom &g) {
+std::vector<unsigned> bucket_peaks(const float *pos4, int n, const SceneGeom &g, double *load) {
     std::vector<unsigned> keys(n);
     for (int i = 0; i < n; ++i) {
         unsigned c[3];
@@ -385,6 +385,9 @@ std::vector<unsigned> bucket_peaks(const float *pos4, int n, const SceneGeom &g)
         for (unsigned k : keys) ++hist[k >> b];
         peak[b] = *std::max_element(hist.begin(), hist.end());
     }
+    double sum = 0.0;
+    for (unsigned c : hist) sum += (double)c * c;
+    *load = n > 0 ? sum / n : 0.0;
     return peak;
 }
 
@@ -542,7 +545,7 @@ int Engine::build(const std::vector<SceneSource> &src, const ArSimTuning *tuning
                     shapes[s].extent[a] = ((double)geoms[s].boxMax[a] - (double)geoms[s].boxMin[a]) /
                                           (double)geoms[s].cellSize[a];
                 }
-                if (src[s].host) shapes[s].peak = bucket_peaks(src[s].host->pos, pCount[s], geoms[s]);
+                if (src[s].host) shapes[s].peak = bucket_peaks(src[s].host->pos, pCount[s], geoms[s], &shapes[s].load);
                 else if (src[s].from && src[s].from->bucketSort)
                     shapes[s].shift = src[s].from->bkPlan.scenes[src[s].fromScene].shift;
             }

@@ -198,12 +198,13 @@ void launch_pose_key_tiles(const PartBufs &p, const BodyBufs &b, int numParticle
 // fullest bucket to hold ceil(r) / r times the average along each axis a bucket does not span,
 // r = extent / grid size.  A scene that kept its shift from an earlier plan (a rebuild) passes it.
 // False when a scene needs more buckets than its tiles can rank or more than 384 tiles, and for grid keys where
-// the fullest measured bucket is too full at every width.
+// the measured buckets are too full at every width.
 struct BucketSceneShape {
     long long particles = 0;
     unsigned grid[3] = {1, 1, 1};
     double extent[3] = {0.0, 0.0, 0.0};
     std::vector<unsigned> peak;   // empty, or one entry per shift 0 .. maxShift
+    double load = 0.0;            // keys in a measured key's bucket on average, at the narrowest shift of peak
     int shift = -1;
 };
 struct BucketPlan {

@@ -34,8 +34,8 @@ def slab(n, seed):
     return sc
 
 
-# about 9,500 particles in a bucket of any width (a workgroup sorts 7,776) in one of the scenes, or 7,200
-@pytest.mark.parametrize("counts", [(20000,), (15500,), (3000, 20000), (15500, 500)])
+# one scene past the sizes and loads at which it is sorted by digit passes, and below; and several
+@pytest.mark.parametrize("counts", [(70000,), (20000,), (3000, 20000), (150000, 50000)])
 def test_crowded_buckets_vs_oracle(counts):
     print(f"sort of scenes crowded into a plane: {counts}", flush=True)
     run_both([slab(n, 90 + k) for k, n in enumerate(counts)])
