@@ -60,6 +60,8 @@ struct Engine {
     unsigned char *keyBufA = nullptr, *keyBufB = nullptr, *sortWsBuf = nullptr;
     unsigned *valsA = nullptr, *valsB = nullptr;
     unsigned *segStart = nullptr;           // grid: CSR offsets over segments of 2^segBits cells
+    double density = 0.0;                   // grid: particles per cell around a particle, of the scenes as given
+    bool queueContacts = false;             // grid: contacts queued before they are evaluated (launch_dem_grid_seg)
     bool useIndex = false;                  // grid, bucket sort: the compact cell index instead (kernels.hpp)
     uint2 *cellWords = nullptr;
     unsigned *cellStarts = nullptr;

@@ -34,6 +34,94 @@ __global__ void k_reorder(const unsigned *__restrict__ keys, const unsigned *__r
     sVel[i] = v;
 }
 
+// A particle's contact sum F, the walls added, to its body's force or to its velocity.
+__device__ __forceinline__ void dem_write(f3 F, int ra, f3 pa, f3 va, unsigned orig, const DevPhys &ph,
+                                          const SceneGeom &g, const DemOut &o) {
+    if (!((ph.flags & kGrainClamp) && ra < 0)) F = add3(F, wall_force(pa, va, ph, g));
+    if (ra >= 0) {
+        o.pForce[orig] = f4(F, 0.0f);
+        if (o.pTorque) o.pTorque[orig] = f4(cross3(xyz(o.relPos[orig]), F), 0.0f);
+    } else {
+        const float fs = (ph.flags & kRefUnits) ? 1.0f : ph.dt;
+        o.vel[orig] = make_float4(va.x + F.x * fs, va.y + F.y * fs, va.z + F.z * fs, 0.0f);
+    }
+}
+
+// Contacts found first and evaluated later.  A lane's candidate loop only tests distances and appends the sorted
+// positions in reach to the lane's queue in LDS (kQueue entries, lane-interleaved); the pair forces are formed
+// when a queue could overflow or the particle's cells are done, two at a time.  Formed in the candidate loop, a wave
+// ran the pair force in every iteration in which any of its lanes had a contact; queued, it runs it about as often as
+// its fullest lane has contacts.  Three candidates' loads together, 16 entries (12 drain too often: 922 us a step at
+// the pile below, 16 874; two loads 900, four 878).  Settled piles: 2^22 particles 634 -> 534 us, the reference's layout at
+// 300,007 88 -> 65.  Where few candidates are contacts the positions read a second time cost more than that gives.
+constexpr int kQueue = 16, kQueueAhead = 3;
+constexpr int kQueueMax = (1 << 28) - 4;   // particles: an entry holds 16 times a sorted position, read up to kQueueAhead on
+__device__ __forceinline__ float4 at16(const float4 *__restrict__ p, unsigned byteOffset) {
+    return *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(p) + byteOffset);
+}
+struct ContactQueue {
+    unsigned *first, *tail, *full;   // this lane's entries: first, first + stride, ..., tail; full: no room for kQueueAhead more
+    unsigned stride;
+    int cell;                        // code of the cell of the last entry appended
+    f3 F, csum;
+    __device__ __forceinline__ ContactQueue(unsigned *q, unsigned stride_)
+        : first(q), tail(q), full(q + (kQueue - kQueueAhead) * stride_), stride(stride_), cell(-1),
+          F(mk3(0.f, 0.f, 0.f)), csum(mk3(0.f, 0.f, 0.f)) {}
+    // bit 0: the first contact of another cell, whose partial sum starts with it
+    __device__ __forceinline__ void push(unsigned j16, int c) {
+        *tail = j16 | (c != cell ? 1u : 0u);
+        tail += stride;
+        cell = c;
+    }
+    __device__ __forceinline__ void one(unsigned w, const float4 &Q, const float4 &V, f3 pa, f3 va, const DevPhys &ph) {
+        if (w & 1u) {
+            F = add3(F, csum);
+            csum = mk3(0.f, 0.f, 0.f);
+        }
+        f3 fj;
+        if (pair_force(pa, xyz(Q), va, xyz(V), ph, fj)) csum = add3(csum, fj);
+    }
+    __device__ __forceinline__ void drain(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel, f3 pa, f3 va,
+                                          const DevPhys &ph) {
+        for (unsigned *p = first; p < tail; p += 2 * stride) {
+            const unsigned w0 = *p;
+            const bool two = p + stride < tail;
+            const unsigned w1 = two ? p[stride] : w0;
+            const float4 Q0 = at16(sPos, w0 & ~15u), V0 = at16(sVel, w0 & ~15u);
+            const float4 Q1 = at16(sPos, w1 & ~15u), V1 = at16(sVel, w1 & ~15u);
+            __builtin_amdgcn_sched_barrier(0);
+            one(w0, Q0, V0, pa, va, ph);
+            if (two) one(w1, Q1, V1, pa, va, ph);
+        }
+        tail = first;
+    }
+    // Queues the contacts of a run [j, e) whose second and third cells (code + 1, + 2) start at b1 and b2.
+    __device__ __forceinline__ void run(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel, unsigned j,
+                                        unsigned b1, unsigned b2, unsigned e, int code, unsigned i16, int ra, f3 pa, f3 va,
+                                        const DevPhys &ph) {
+        const unsigned e16 = e << 4, b116 = b1 << 4, b216 = b2 << 4;
+        for (unsigned j16 = j << 4; j16 < e16; j16 += 16u * kQueueAhead) {
+            unsigned jj[kQueueAhead];
+            float4 Q[kQueueAhead];
+#pragma unroll
+            for (int u = 0; u < kQueueAhead; ++u) {
+                jj[u] = j16 + 16u * u;
+                if (u && !(jj[u] < e16)) jj[u] = i16;   // the particle itself: never a contact
+                Q[u] = at16(sPos, jj[u]);
+            }
+            __builtin_amdgcn_sched_barrier(0);   // every load issued before the first is waited for
+#pragma unroll
+            for (int u = 0; u < kQueueAhead; ++u) {
+                const f3 rel = sub3(xyz(Q[u]), pa);
+                const bool near = !(dot3(rel, rel) > ph.cd2Reject);
+                if (near & (jj[u] != i16) & pair_allowed(ra, __float_as_int(Q[u].w)))
+                    push(jj[u], code + (jj[u] >= b116 ? 1 : 0) + (jj[u] >= b216 ? 1 : 0));
+            }
+            if (tail > full) drain(sPos, sVel, pa, va, ph);
+        }
+    }
+};
+
 // FindAndHandleRigidBodyCollisionsUniformGridKernel (RigidBodies/UniformGridDEM.cu:133-204) and
 // collideD (particleKernels.cu:302-406): 27 cells in z, y, x order, per-cell partial sums, the
 // contact predicate j != i && (rbA != rbB || rbA == -1), then the wall term.  EMIT writes the
@@ -93,6 +181,34 @@ __global__ void k_dem_grid(const float4 *__restrict__ sPos, const float4 *__rest
         const float fs = (ph.flags & kRefUnits) ? 1.0f : ph.dt;
         o.vel[orig] = make_float4(va.x + F.x * fs, va.y + F.y * fs, va.z + F.z * fs, 0.0f);
     }
+}
+
+// The same sums over queued contacts.
+__global__ void k_dem_grid_ref_queue(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
+                                     const unsigned *__restrict__ sIdx, const unsigned *__restrict__ cs,
+                                     const unsigned *__restrict__ ce, int n, DevPhys ph, SceneGeom g, DemOut o) {
+    extern __shared__ unsigned queueLds[];
+    const int i = xcd_block((int)blockIdx.x, (int)gridDim.x) * (int)blockDim.x + (int)threadIdx.x;
+    if (i >= n) return;
+    const float4 P = sPos[i];
+    const float4 Vq = sVel[i];
+    const int ra = __float_as_int(P.w);
+    const f3 pa = xyz(P), va = xyz(Vq);
+    int gx, gy, gz;
+    grid_pos(pa, g, gx, gy, gz);
+    ContactQueue cq(queueLds + threadIdx.x, blockDim.x);
+    int c = 0;
+    for (int z = -1; z <= 1; ++z)
+        for (int y = -1; y <= 1; ++y)
+            for (int x = -1; x <= 1; ++x, ++c) {
+                const unsigned h = g.cellBase + grid_hash(gx + x, gy + y, gz + z, g);
+                const unsigned st = cs[h];
+                if (st == kEmpty) continue;
+                const unsigned en = ce[h];
+                cq.run(sPos, sVel, st, en, en, en, c, (unsigned)i << 4, ra, pa, va, ph);
+            }
+    cq.drain(sPos, sVel, pa, va, ph);
+    dem_write(add3(cq.F, cq.csum), ra, pa, va, sIdx[i], ph, g, o);
 }
 
 // Engine form of the reorder: the same gather of the sorted copies, but instead of the two
@@ -327,19 +443,6 @@ __device__ __forceinline__ void for_dem_block(const SceneView &sv, const float4 
     if (!one_scene(sVel, lb, n, scene)) return;
     body(lb, sv.table[scene], std::integral_constant<int, kGeomBlock>{});
 }
-// A particle's contact sum F, the walls added, to its body's force or to its velocity.
-__device__ __forceinline__ void dem_write(f3 F, int ra, f3 pa, f3 va, unsigned orig, const DevPhys &ph,
-                                          const SceneGeom &g, const DemOut &o) {
-    if (!((ph.flags & kGrainClamp) && ra < 0)) F = add3(F, wall_force(pa, va, ph, g));
-    if (ra >= 0) {
-        o.pForce[orig] = f4(F, 0.0f);
-        if (o.pTorque) o.pTorque[orig] = f4(cross3(xyz(o.relPos[orig]), F), 0.0f);
-    } else {
-        const float fs = (ph.flags & kRefUnits) ? 1.0f : ph.dt;
-        o.vel[orig] = make_float4(va.x + F.x * fs, va.y + F.y * fs, va.z + F.z * fs, 0.0f);
-    }
-}
-
 template <bool EMIT, bool EXACT, int GEOM>
 __device__ __forceinline__ void dem_seg_block(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
                                               const unsigned *__restrict__ keys, const unsigned *__restrict__ sIdx,
@@ -423,6 +526,57 @@ __global__ void k_dem_grid_seg(const float4 *__restrict__ sPos, const float4 *__
                                DemOut o) {
     for_dem_block<BATCH>(sv, sVel, n, [&](int lb, const SceneGeom &g, auto geom) {
         dem_seg_block<EMIT, EXACT, decltype(geom)::value>(sPos, sVel, keys, sIdx, segStart, segBits, n, ph, sv, o, lb, g);
+    });
+}
+
+// The contact kernel over the exact cell table, contacts queued.
+template <int GEOM>
+__device__ __forceinline__ void dem_queue_block(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
+                                                const unsigned *__restrict__ sIdx,
+                                                const unsigned *__restrict__ segStart, int n, const DevPhys &ph,
+                                                const SceneView &sv, const DemOut &o, int lb, SceneGeom g,
+                                                unsigned *queue) {
+    const int i = lb * (int)blockDim.x + (int)threadIdx.x;
+    if (i >= n) return;
+    const float4 P = sPos[i];
+    const float4 Vq = sVel[i];
+    const int ra = __float_as_int(P.w);
+    if (GEOM == kGeomLane) g = sv.table[__float_as_int(Vq.w)];
+    const f3 pa = xyz(P), va = xyz(Vq);
+    int gx, gy, gz;
+    grid_pos(pa, g, gx, gy, gz);
+    const unsigned x0 = (unsigned)(gx - 1) & g.gridMask[0], x1 = (unsigned)gx & g.gridMask[0],
+                   x2 = (unsigned)(gx + 1) & g.gridMask[0];
+    const bool contiguous = (x0 + 1u == x1) && (x1 + 1u == x2);
+    ContactQueue cq(queue, blockDim.x);
+    for (int r = 0; r < 9; ++r) {
+        const unsigned uz = (unsigned)(gz + (r / 3) - 1) & g.gridMask[2];
+        const unsigned uy = (unsigned)(gy + (r % 3) - 1) & g.gridMask[1];
+        const unsigned row = g.cellBase + uz * g.gxy + uy * g.gx;
+        if (contiguous) {
+            // the row's four offsets in one 16-byte load (4-byte aligned)
+            uint4 bnd;
+            __builtin_memcpy(&bnd, segStart + (row + x0), sizeof(bnd));
+            cq.run(sPos, sVel, bnd.x, bnd.y, bnd.z, bnd.w, 3 * r, (unsigned)i << 4, ra, pa, va, ph);
+        } else {
+#pragma unroll 1
+            for (int k = 0; k < 3; ++k) {
+                const unsigned h = row + (k == 0 ? x0 : k == 1 ? x1 : x2);
+                const unsigned e = segStart[h + 1u];
+                cq.run(sPos, sVel, segStart[h], e, e, e, 3 * r + k, (unsigned)i << 4, ra, pa, va, ph);
+            }
+        }
+    }
+    cq.drain(sPos, sVel, pa, va, ph);
+    dem_write(add3(cq.F, cq.csum), ra, pa, va, sIdx[i], ph, g, o);
+}
+template <bool BATCH>
+__global__ void k_dem_grid_queue(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
+                                 const unsigned *__restrict__ sIdx, const unsigned *__restrict__ segStart, int n,
+                                 DevPhys ph, SceneView sv, DemOut o) {
+    extern __shared__ unsigned queueLds[];
+    for_dem_block<BATCH>(sv, sVel, n, [&](int lb, const SceneGeom &g, auto geom) {
+        dem_queue_block<decltype(geom)::value>(sPos, sVel, sIdx, segStart, n, ph, sv, o, lb, g, queueLds + threadIdx.x);
     });
 }
 
@@ -647,7 +801,8 @@ void launch_fill_long(unsigned *table, unsigned long long tableSize, const LongF
 
 void launch_dem_grid_seg(const float4 *sortedPos, const float4 *sortedVel, const unsigned *sortedKeys,
                          const unsigned *sortedIdx, const unsigned *segStart, int segBits, int n, const DevPhys &ph,
-                         const SceneView &sv, bool sceneInVelW, const DemOut &o, int block, hipStream_t st) {
+                         const SceneView &sv, bool sceneInVelW, const DemOut &o, bool queue, int block,
+                         hipStream_t st) {
     if (n <= 0) return;
     if (block <= 0) block = 128;
     if (!o.pairs && segBits == 0 && n <= kCoopMax) {
@@ -658,6 +813,16 @@ void launch_dem_grid_seg(const float4 *sortedPos, const float4 *sortedVel, const
         return;
     }
     dim3 grid((n + block - 1) / block);
+    if (queue && !o.pairs && segBits == 0 && n < kQueueMax) {
+        const size_t lds = (size_t)block * kQueue * sizeof(unsigned);
+        if (sceneInVelW)
+            hipLaunchKernelGGL(k_dem_grid_queue<true>, dim3(grid.x + (unsigned)sv.count - 1u), dim3(block), lds, st,
+                               sortedPos, sortedVel, sortedIdx, segStart, n, ph, sv, o);
+        else
+            hipLaunchKernelGGL(k_dem_grid_queue<false>, grid, dim3(block), lds, st, sortedPos, sortedVel, sortedIdx,
+                               segStart, n, ph, sv, o);
+        return;
+    }
     auto run = [&](auto single, auto batch) {
         if (sceneInVelW)
             hipLaunchKernelGGL(batch, dim3(grid.x + (unsigned)sv.count - 1u), dim3(block), 0, st, sortedPos, sortedVel,
@@ -711,7 +876,10 @@ void launch_dem_grid(const float4 *sortedPos, const float4 *sortedVel, const uns
         return;
     }
     dim3 grid((n + block - 1) / block);
-    if (o.pairs)
+    if (!o.pairs && !sceneInVelW && n < kQueueMax)
+        hipLaunchKernelGGL(k_dem_grid_ref_queue, grid, dim3(block), (size_t)block * kQueue * sizeof(unsigned), st,
+                           sortedPos, sortedVel, sortedIdx, cellStart, cellEnd, n, ph, sv.single, o);
+    else if (o.pairs)
         hipLaunchKernelGGL(k_dem_grid<true>, grid, dim3(block), 0, st, sortedPos, sortedVel, sortedIdx, cellStart,
                            cellEnd, n, ph, sv, sceneInVelW ? 1 : 0, o);
     else

@@ -253,7 +253,8 @@ unsigned fill_long_capacity(unsigned long long tableSize);
 void launch_fill_long(unsigned *table, unsigned long long tableSize, const LongFill &lf, hipStream_t st);
 void launch_dem_grid_seg(const float4 *sortedPos, const float4 *sortedVel, const unsigned *sortedKeys,
                          const unsigned *sortedIdx, const unsigned *segStart, int segBits, int n, const DevPhys &ph,
-                         const SceneView &sv, bool sceneInVelW, const DemOut &o, int block, hipStream_t st);
+                         const SceneView &sv, bool sceneInVelW, const DemOut &o, bool queue, int block,
+                         hipStream_t st);
 // The same with the compact cell index (forces only).
 void launch_dem_grid_index(const float4 *sortedPos, const float4 *sortedVel, const unsigned *sortedIdx,
                            const CellIndex &ix, int n, const DevPhys &ph, const SceneView &sv, bool sceneInVelW,
