@@ -47,7 +47,7 @@ int sort_common(K **keys, unsigned **vals, K **altKeys, unsigned **altVals, int 
     if (n == 0) return ARSIM_OK;
     if (!ws || wsBytes < sort_workspace_bytes(n, (int)sizeof(K)))
         return fail(ARSIM_ERR_WORKSPACE, "sort_pairs: workspace too small");
-    SortTuning tu;
+    const SortTuning tu = sort_tuning_for(n);
     int rc = sort_pairs<K>(keys, vals, altKeys, altVals, n, beginBit, endBit, false, ws, wsBytes, tu, S(st));
     if (rc) return fail(ARSIM_ERR_INVALID_ARG, "sort_pairs: rejected arguments");
     return check_launch("sort_pairs");

@@ -213,7 +213,7 @@ int Engine::set_static(const float *pos4, const float *norm4, int n) {
         launch_static_hash(dPos, n, g, kA, st);
         int bits = 1;
         while ((1ull << bits) < (unsigned long long)cells) ++bits;
-        SortTuning stt{};
+        const SortTuning stt = sort_tuning_for(n);
         if (sort_pairs<unsigned>(&kA, &vA, &kB, &vB, n, 0, bits, true, ws, wsBytes, stt, st))
             rc = fail(ARSIM_ERR_INVALID_ARG, "engine_set_static: sort rejected");
         else

@@ -19,6 +19,7 @@ struct SortTuning {
 
 // ---------------------------------------------------------------- sort (sort.hip)
 int sort_max_passes(int keyBytes);
+SortTuning sort_tuning_for(int n);   // the tuning of a sort whose caller names none
 size_t sort_workspace_bytes(int n, int keyBytes);
 bool sort_tuning_supported(int ipt, int rbits);
 // Returns 0 on success; swaps *keys/*alt and *vals/*altVals once per pass so that on return

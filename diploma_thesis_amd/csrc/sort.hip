@@ -26,6 +26,8 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
+constexpr int kSmallSort = 1 << 17;   // keys
+constexpr int kLookBack = 8;   // look-back words read together
 constexpr unsigned kFlagAgg = 1u << 30;
 constexpr unsigned kFlagInc = 2u << 30;
 constexpr unsigned kValMask = (1u << 30) - 1u;
@@ -58,7 +60,7 @@ __global__ void k_sort_init(unsigned *hist, int histWords, unsigned *counters, i
     for (int k = i; k < statusWords; k += stride) status0[k] = 0u;
 }
 
-template <class K, int RBITS>
+template <class K, int RBITS, int AHEAD>   // AHEAD: keys a thread loads together
 __global__ __launch_bounds__(kBlock) void k_sort_hist(const K *__restrict__ keys, int n, int beginBit,
                                                        int endBit, int passes, unsigned *__restrict__ hist,
                                                        const unsigned *gate) {
@@ -69,20 +71,28 @@ __global__ __launch_bounds__(kBlock) void k_sort_hist(const K *__restrict__ keys
     for (int k = threadIdx.x; k < passes * RADIX; k += kBlock) sh[k] = 0u;
     __syncthreads();
     int stride = gridDim.x * kBlock;
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) {
-        K key = keys[i];
-        for (int p = 0; p < passes; ++p) {
-            int sh0 = beginBit + p * RBITS;
-            int bits = min(RBITS, endBit - sh0);
-            unsigned d = (unsigned)((key >> sh0) & (K)((1u << bits) - 1u));
-            // keys in spatial order often share a digit across the wave: one add for all of them
-            const uint64_t active = __ballot(1);
-            const int first = __ffsll((long long)active) - 1;
-            const unsigned d0 = __shfl(d, first, 64);
-            if (__ballot(d == d0) == active) {
-                if ((int)(threadIdx.x & 63) == first) atomicAdd(&sh[p * RADIX + d], (unsigned)__popcll(active));
-            } else {
-                atomicAdd(&sh[p * RADIX + d], 1u);
+#pragma unroll 1
+    for (int i0 = blockIdx.x * kBlock + threadIdx.x; i0 < n; i0 += AHEAD * stride) {
+        K ahead[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) ahead[u] = i0 + u * stride < n ? keys[i0 + u * stride] : (K)0;
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            if (i0 + u * stride >= n) continue;
+            const K key = ahead[u];
+            for (int p = 0; p < passes; ++p) {
+                int sh0 = beginBit + p * RBITS;
+                int bits = min(RBITS, endBit - sh0);
+                unsigned d = (unsigned)((key >> sh0) & (K)((1u << bits) - 1u));
+                // keys in spatial order often share a digit across the wave: one add for all of them
+                const uint64_t active = __ballot(1);
+                const int first = __ffsll((long long)active) - 1;
+                const unsigned d0 = __shfl(d, first, 64);
+                if (__ballot(d == d0) == active) {
+                    if ((int)(threadIdx.x & 63) == first) atomicAdd(&sh[p * RADIX + d], (unsigned)__popcll(active));
+                } else {
+                    atomicAdd(&sh[p * RADIX + d], 1u);
+                }
             }
         }
     }
@@ -178,20 +188,35 @@ __global__ __launch_bounds__(kBlock) void k_onesweep(const K *__restrict__ kin, 
         if (tile == 0) {
             excl = globalExcl;
         } else {
-            // decoupled look-back over the tiles before this one
+            // Decoupled look-back over the tiles before this one.  All tiles of a mid-sized sort run at once and
+            // walk far, so a digit's pass takes as long as its chain of reads: eight words read together instead of one
+            // take a sort of 300,007 24-bit keys from 53 to 49 us, of 2^20 from 79 to 73, of 2^22 63-bit keys
+            // from 433 to 394.
             excl = 0u;
-            long long pt = (long long)tile - 1;
-            while (true) {
-                unsigned s = __hip_atomic_load(&status[(size_t)pt * RADIX + tid], __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-                unsigned f = s & ~kValMask;
-                if (f == 0u) {
-                    __builtin_amdgcn_s_sleep(1);
-                    continue;
+            int pt = (int)tile - 1;
+            bool more = true;
+            while (more) {
+                unsigned s[kLookBack];
+#pragma unroll
+                for (int u = 0; u < kLookBack; ++u) {
+                    const int q = pt - u > 0 ? pt - u : 0;
+                    s[u] = __hip_atomic_load(&status[(size_t)q * RADIX + tid], __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
                 }
-                excl += s & kValMask;
-                if (f == kFlagInc) break;
-                --pt;
+                bool open = true;   // every word so far was an aggregate
+#pragma unroll
+                for (int u = 0; u < kLookBack; ++u) {
+                    const unsigned f = s[u] & ~kValMask;
+                    open = open && f != 0u;
+                    if (!open) continue;
+                    excl += s[u] & kValMask;
+                    --pt;
+                    if (f == kFlagInc) {
+                        more = false;
+                        open = false;
+                    }
+                }
+                if (more && !open) __builtin_amdgcn_s_sleep(1);
             }
         }
         __hip_atomic_store(&status[(size_t)tile * RADIX + tid], kFlagInc | ((excl + tileCnt) & kValMask),
@@ -233,10 +258,12 @@ void launch_passes(K **keys, unsigned **vals, K **alt, unsigned **altVals, int n
                    int numTiles, bool doHist, const unsigned *gate, hipStream_t st) {
     const int passes = num_passes(beginBit, endBit, RBITS);
     if (doHist) {
-        int histBlocks = (n + kBlock * 8 - 1) / (kBlock * 8);
+        // eight keys a thread; two where that leaves most CUs without a block (16,384 keys: 33 -> 30 us for the sort)
+        const int each = n <= kSmallSort ? 2 : 8;
+        int histBlocks = (n + kBlock * each - 1) / (kBlock * each);
         histBlocks = histBlocks < 1 ? 1 : (histBlocks > 4096 ? 4096 : histBlocks);
-        hipLaunchKernelGGL((k_sort_hist<K, RBITS>), dim3(histBlocks), dim3(kBlock), 0, st, *keys, n, beginBit, endBit,
-                           passes, hist, gate);
+        auto kernel = each == 2 ? k_sort_hist<K, RBITS, 2> : k_sort_hist<K, RBITS, 8>;
+        hipLaunchKernelGGL(kernel, dim3(histBlocks), dim3(kBlock), 0, st, *keys, n, beginBit, endBit, passes, hist, gate);
     }
     for (int p = 0; p < passes; ++p) {
         int shift = beginBit + p * RBITS;
@@ -364,6 +391,15 @@ hipError_t sort_static_scratch(void **ptr, size_t *bytes) {
     *ptr = g_scratchPtr[dev];
     *bytes = kStaticSortScratchBytes;
     return hipSuccess;
+}
+
+// Tiles of 16 keys a thread leave most CUs idle below about 2^19 keys and make every rank chain as long: with 4 keys
+// 24-bit sorts of 16,384 and 65,536 keys take 28 and 32 us instead of 42 and 42, with 8 of 300,007 45 instead of 49;
+// from there on more tiles only lengthen the look-back (2^20 keys: 73 us with 16, 81 with 8).
+SortTuning sort_tuning_for(int n) {
+    SortTuning tu;
+    tu.ipt = n <= kSmallSort ? 4 : n <= (1 << 19) ? 8 : 16;
+    return tu;
 }
 
 bool sort_tuning_supported(int ipt, int rbits) {
