@@ -258,10 +258,13 @@ void launch_passes(K **keys, unsigned **vals, K **alt, unsigned **altVals, int n
                    int numTiles, bool doHist, const unsigned *gate, hipStream_t st) {
     const int passes = num_passes(beginBit, endBit, RBITS);
     if (doHist) {
-        // eight keys a thread; two where that leaves most CUs without a block (16,384 keys: 33 -> 30 us for the sort)
+        // Eight keys a thread; two where that leaves most CUs without a block (16,384 keys: 33 -> 30 us for the sort).
+        // At most 512 blocks, or 64 keys a thread: every block adds its counts to the same words (2^22 24-bit
+        // keys 172 us with 2,048 blocks, 154 with 512; 2^24 63-bit keys 1,271 with 4,096 and 1,310 with 512).
         const int each = n <= kSmallSort ? 2 : 8;
+        const int most = n / (kBlock * 64) > 512 ? n / (kBlock * 64) : 512;
         int histBlocks = (n + kBlock * each - 1) / (kBlock * each);
-        histBlocks = histBlocks < 1 ? 1 : (histBlocks > 4096 ? 4096 : histBlocks);
+        histBlocks = histBlocks < 1 ? 1 : (histBlocks > most ? most : histBlocks);
         auto kernel = each == 2 ? k_sort_hist<K, RBITS, 2> : k_sort_hist<K, RBITS, 8>;
         hipLaunchKernelGGL(kernel, dim3(histBlocks), dim3(kBlock), 0, st, *keys, n, beginBit, endBit, passes, hist, gate);
     }
