@@ -368,41 +368,42 @@ int Engine::state_checksum(int s, uint64_t *out) {
 namespace {
 
 // The fullest bucket of a scene's grid keys for every bucket width 2^b cells (b = 0..16, UINT_MAX
-// where there would be more than 1024 buckets), from host positions (float4 per particle).
+// where there would be more than 1024 buckets), from host positions (float4 per particle); the keys in a key's
+// bucket on average at the narrowest of them, and the particles per cell around a particle on average, by blocks.
 std::vector<unsigned> bucket_peaks(const float *pos4, int n, const SceneGeom &g, double *load, double *density) {
-    std::vector<unsigned> keys(n);
+    const unsigned long long cells =
+        (unsigned long long)(g.gridMask[0] + 1u) * (g.gridMask[1] + 1u) * (g.gridMask[2] + 1u);
+    int narrow = 0;
+    while (((cells + (1ull << narrow) - 1) >> narrow) > 1024) ++narrow;
+    std::vector<unsigned> peak(17, 0xffffffffu), hist(1024, 0u);
+    // blocks of 4 x 4 x 4 cells, 8 x 8 x 8 in large grids
+    const int e = cells > (1ull << 26) ? 3 : 2;
+    const unsigned bx = (g.gridMask[0] >> e) + 1u, by = (g.gridMask[1] >> e) + 1u, bz = (g.gridMask[2] >> e) + 1u;
+    std::vector<unsigned> block((size_t)bx * by * bz, 0u);
+    const double inv[3] = {1.0 / g.cellSize[0], 1.0 / g.cellSize[1], 1.0 / g.cellSize[2]};
     for (int i = 0; i < n; ++i) {
         unsigned c[3];
         for (int a = 0; a < 3; ++a) {
-            const double q = std::floor(((double)pos4[4 * (size_t)i + a] - g.origin[a]) / g.cellSize[a]);
-            const long long v = q > -1e18 && q < 1e18 ? (long long)q : 0;   // NaN and huge values: cell 0
+            const double q = ((double)pos4[4 * (size_t)i + a] - g.origin[a]) * inv[a];
+            long long v = q > -1e18 && q < 1e18 ? (long long)q : 0;   // NaN and huge values: cell 0
+            v -= q < (double)v ? 1 : 0;
             c[a] = (unsigned)v & g.gridMask[a];
         }
-        keys[i] = c[2] * g.gxy + c[1] * g.gx + c[0];
-    }
-    const unsigned long long cells =
-        (unsigned long long)(g.gridMask[0] + 1u) * (g.gridMask[1] + 1u) * (g.gridMask[2] + 1u);
-    std::vector<unsigned> peak(17, 0xffffffffu);
-    std::vector<unsigned> hist(1024);
-    for (int b = 16; b >= 0; --b) {
-        if (((cells + (1ull << b) - 1) >> b) > 1024) break;
-        std::fill(hist.begin(), hist.end(), 0u);
-        for (unsigned k : keys) ++hist[k >> b];
-        peak[b] = *std::max_element(hist.begin(), hist.end());
+        ++hist[((c[2] * g.gxy + c[1] * g.gx + c[0]) >> narrow) & 1023u];
+        ++block[((size_t)(c[2] >> e) * by + (c[1] >> e)) * bx + (c[0] >> e)];
     }
     double sum = 0.0;
-    for (unsigned c : hist) sum += (double)c * c;
-    *load = n > 0 ? sum / n : 0.0;
-    // particles per cell around a particle, by blocks of 4 x 4 x 4 cells
-    const unsigned bx = (g.gridMask[0] >> 2) + 1u, by = (g.gridMask[1] >> 2) + 1u, bz = (g.gridMask[2] >> 2) + 1u;
-    std::vector<unsigned> block((size_t)bx * by * bz, 0u);
-    for (unsigned k : keys) {
-        const unsigned z = k / g.gxy, y = (k - z * g.gxy) / g.gx, x = k - z * g.gxy - y * g.gx;
-        ++block[((size_t)(z >> 2) * by + (y >> 2)) * bx + (x >> 2)];
-    }
-    sum = 0.0;
     for (unsigned c : block) sum += (double)c * c;
-    *density = n > 0 ? sum / (64.0 * n) : 0.0;
+    *density = n > 0 ? sum / ((double)(1 << 3 * e) * n) : 0.0;
+    sum = 0.0;
+    if (narrow <= 16)
+        for (unsigned c : hist) sum += (double)c * c;
+    *load = n > 0 ? sum / n : 0.0;
+    for (int b = narrow; b <= 16; ++b) {
+        peak[b] = *std::max_element(hist.begin(), hist.end());
+        for (size_t k = 0; k < 512; ++k) hist[k] = hist[2 * k] + hist[2 * k + 1];
+        std::fill(hist.begin() + 512, hist.end(), 0u);
+    }
     return peak;
 }
 
@@ -410,21 +411,19 @@ std::vector<unsigned> bucket_peaks(const float *pos4, int n, const SceneGeom &g,
 // 2^30 (one), at index b of the plan's per-shift peaks (narrower ones: UINT_MAX), from host positions
 // normalised as the device does (for planning only).
 std::vector<unsigned> morton_peaks(const float *pos4, int n, const SceneGeom &g) {
-    auto spread = [](unsigned v) {   // bit k of v to bit 3k
-        unsigned r = 0u;
-        for (int k = 0; k < 10; ++k) r |= ((v >> k) & 1u) << (3 * k);
-        return r;
-    };
+    // the code's upper 10 bits: the upper 4 bits of x's 10, 3 of y's and of z's, interleaved
+    unsigned spread[16];   // bit k of the index to bit 3k
+    for (unsigned v = 0; v < 16u; ++v) spread[v] = (v & 1u) | (v & 2u) << 2 | (v & 4u) << 4 | (v & 8u) << 6;
+    double scale[3];
+    for (int a = 0; a < 3; ++a) scale[a] = g.mExt[a] == 0.0f ? 0.0 : 1024.0 / g.mExt[a];
     std::vector<unsigned> peak(31, 0xffffffffu), hist(1024, 0u);
     for (int i = 0; i < n; ++i) {
         unsigned q[3];
         for (int a = 0; a < 3; ++a) {
-            const double u = g.mExt[a] == 0.0f ? 0.0 : ((double)pos4[4 * (size_t)i + a] - g.mLo[a]) / g.mExt[a];
-            const double v = u * 1024.0;
+            const double v = ((double)pos4[4 * (size_t)i + a] - g.mLo[a]) * scale[a];
             q[a] = v > 0.0 ? (v < 1023.0 ? (unsigned)v : 1023u) : 0u;   // NaN: 0
         }
-        const unsigned code = spread(q[0]) * 4u + spread(q[1]) * 2u + spread(q[2]);
-        ++hist[code >> 20];
+        ++hist[spread[q[0] >> 6] | spread[q[1] >> 7] << 2 | spread[q[2] >> 7] << 1];
     }
     for (int b = 20;; ++b) {
         peak[b] = *std::max_element(hist.begin(), hist.end());
