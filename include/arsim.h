@@ -271,10 +271,11 @@ int arsim_lbvh_refit(const int *sortedIndices, const float *pos, const float *ve
 /* F17  collideBVHSoARigidBodyWrapper (rigidBodyKernelWrappers.h:49-68, RB_BVHKernels.cu:100-244).
  * Stack traversal from the root per sorted leaf; same contact predicate, force, wall term and
  * outputs as arsim_dem_grid.  Neighbour velocities are read from a sorted copy (sortedVel), so
- * no thread reads a velocity another thread is writing.  The per-thread stack holds 64 entries in
- * LDS, as the reference's int stack[64]; a traversal that would exceed it sets the device int
- * *overflowFlag to 1 and writes nothing for that particle (its pForce / pTorque / vel keep their
- * previous contents), so a truncated sum is never returned as a result. */
+ * no thread reads a velocity another thread is writing.  16 consecutive sorted leaves go down together, with
+ * a list of nodes in LDS for which a tree of up to 64 levels (as the reference's int stack[64]) always
+ * has room; where a deeper tree runs out of it the device int *overflowFlag is set to 1 and nothing is
+ * written for the particles concerned (their pForce / pTorque / vel keep their previous contents), so a
+ * truncated sum is never returned as a result. */
 int arsim_dem_lbvh(const int *rbIndices, float *pForce, float *pTorque, float *vel,
                    const float *sortedVel, const float *relativePos, const int *sortedIndices,
                    const int *leftIndices, const int *rightIndices, const float *CMs,
