@@ -26,6 +26,12 @@ constexpr int kBkWaves = kBkThreads / 64;
 // Bucket size sorted in LDS: two buffers of packed words plus the 16 KiB cursor table, the wave sums
 // and the tile map stay within 80 KiB, half of a gfx950 CU's 160 KiB, so two workgroups share a CU.
 constexpr int kBkCap = 7776;
+// Plans whose buckets are all small take workgroups of 256 threads: a bucket of 64 keys leaves 15 of 16 waves idle, and
+// every barrier and scan waits for them: the sort and reorder of 16,384 particles 18 -> 12 us (the step 39 -> 33), of
+// 65,000 19 -> 16, the codes of a forest of 40 scenes of 9,000 32 -> 21.
+constexpr int kBkSmallThreads = 256;
+constexpr int kBkSmallCap = 3840;   // keys sorted in LDS
+constexpr unsigned kBkSmallPeak = 1024;   // of the fullest measured bucket: room for the particles to move
 constexpr int kBkMaxTiles = 384;  // tiles of one scene, which a bucket gathers from (2^20 keys: 256)
 constexpr int kBkLdsBytes = 2 * kBkCap * 4 + kBkWaves * 256 * 4 + kBkWaves * 4 + 2 * kBkMaxTiles * 4;
 static_assert(kBkLdsBytes <= 80 * 1024, "two bucket workgroups must fit in one CU's LDS");
@@ -62,6 +68,7 @@ __device__ __forceinline__ unsigned block_excl_scan(unsigned v, unsigned *sWave)
     return before + x - v;
 }
 
+template <int THREADS>
 __device__ __forceinline__ unsigned block_sum(unsigned v, unsigned *sWave) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
@@ -69,7 +76,7 @@ __device__ __forceinline__ unsigned block_sum(unsigned v, unsigned *sWave) {
     if (lane == 0) sWave[wave] = v;
     __syncthreads();
     unsigned s = 0u;
-    for (int w = 0; w < kBkWaves; ++w) s += sWave[w];
+    for (int w = 0; w < (THREADS / 64); ++w) s += sWave[w];
     __syncthreads();
     return s;
 }
@@ -104,16 +111,16 @@ struct GlobalItems {
 // the segment in order 64 at a time, a lane's rank among equal digits of its group coming from
 // ballots, so the order of equal digits is kept.  (The ballots are the pass's VALU cost: a wave64
 // instruction takes four cycles, so the count phase does without them.)
-template <class IT>
+template <int THREADS, class IT>
 __device__ void stable_pass(const IT &src, const IT &dst, int cnt, int shift, int bits, unsigned (*sCur)[256],
                             unsigned *sWave) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const unsigned mask = (1u << bits) - 1u;
     const int radix = 1 << bits;
-    const int seg = ((cnt + kBkThreads - 1) / kBkThreads) * 64;
+    const int seg = ((cnt + THREADS - 1) / THREADS) * 64;
     const int s0 = min(wave * seg, cnt), s1 = min(s0 + seg, cnt);
     const uint64_t lower = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    for (int k = threadIdx.x; k < kBkWaves * 256; k += kBkThreads) (&sCur[0][0])[k] = 0u;
+    for (int k = threadIdx.x; k < (THREADS / 64) * 256; k += THREADS) (&sCur[0][0])[k] = 0u;
     __syncthreads();
     // the counts need no order: an LDS atomic per item
     for (int i = s0 + lane; i < s1; i += 64) atomicAdd(&sCur[wave][src.digit(i, shift, mask)], 1u);
@@ -121,15 +128,15 @@ __device__ void stable_pass(const IT &src, const IT &dst, int cnt, int shift, in
     // cursors: digits in order, and within a digit the waves in order
     {
         const int t = threadIdx.x;
-        unsigned c[kBkWaves], tot = 0u;
-        for (int w = 0; w < kBkWaves; ++w) {
+        unsigned c[(THREADS / 64)], tot = 0u;
+        for (int w = 0; w < (THREADS / 64); ++w) {
             c[w] = t < radix ? sCur[w][t] : 0u;
             tot += c[w];
         }
         const unsigned excl = block_excl_scan(tot, sWave);
         if (t < radix) {
             unsigned run = excl;
-            for (int w = 0; w < kBkWaves; ++w) {
+            for (int w = 0; w < (THREADS / 64); ++w) {
                 sCur[w][t] = run;
                 run += c[w];
             }
@@ -150,17 +157,18 @@ __device__ void stable_pass(const IT &src, const IT &dst, int cnt, int shift, in
 }
 
 // Fills table[a, b) with v using the whole workgroup (16-byte stores for the aligned middle).
+template <int THREADS>
 __device__ __forceinline__ void block_fill(unsigned *table, unsigned long long a, unsigned long long b, unsigned v) {
     if (a >= b) return;
     const unsigned long long a4 = (a + 3ull) & ~3ull, b4 = b & ~3ull;
     if (a4 >= b4) {
-        for (unsigned long long k = a + threadIdx.x; k < b; k += kBkThreads) table[k] = v;
+        for (unsigned long long k = a + threadIdx.x; k < b; k += THREADS) table[k] = v;
         return;
     }
     if (threadIdx.x < a4 - a) table[a + threadIdx.x] = v;
     if (threadIdx.x < b - b4) table[b4 + threadIdx.x] = v;
     const uint4 v4 = make_uint4(v, v, v, v);
-    for (unsigned long long k = a4 + 4ull * threadIdx.x; k < b4; k += 4ull * kBkThreads)
+    for (unsigned long long k = a4 + 4ull * threadIdx.x; k < b4; k += 4ull * THREADS)
         *reinterpret_cast<uint4 *>(table + k) = v4;
 }
 
@@ -172,20 +180,23 @@ enum { kOutKeys = 0, kOutTable = 1, kOutIndex = 2 };
 // with few particles, whose buckets span more than 2^(32 - POSBITS) codes, and 2^20 keys in 512 buckets
 // instead of 1,024: the LBVH30 step 342 -> 328 us): key and position apart.
 // kOut64 (a forest's Morton keys): the sorted keys as scene << 30 | code there instead of in kOut.
+// THREADS: kBkThreads, or kBkSmallThreads for plans of small buckets.
 // Eight waves per SIMD (two workgroups per CU): registers are held to that occupancy.
-template <int POSBITS, int OUT, bool WIDE>
-__global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_bucket_sort(
+template <int POSBITS, int OUT, bool WIDE, int THREADS>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(8))) void k_bucket_sort(
     TileKeyOut to, int split, unsigned *__restrict__ kOut, unsigned *__restrict__ vOut,
     const float4 *__restrict__ rec, float4 *__restrict__ sPos, float4 *__restrict__ sVel,
     unsigned *__restrict__ table, unsigned numCells, uint64_t *__restrict__ kOut64, CellIndex ix) {
     constexpr bool REORDER = OUT != kOutKeys;
-    constexpr int kCap = kBkCap < (1 << POSBITS) ? kBkCap : (1 << POSBITS);
-    constexpr int kLds = WIDE ? kCap : kBkCap;
+    constexpr int kMost = THREADS == kBkThreads ? kBkCap : kBkSmallCap;
+    constexpr int kCap = kMost < (1 << POSBITS) ? kMost : (1 << POSBITS);
+    constexpr int kLds = WIDE ? kCap : kMost;
+    static_assert(OUT != kOutIndex || THREADS == kBkThreads, "the index's words take the whole cursor table");
     static_assert(!(WIDE && REORDER), "grid keys fit the packed words");
     __shared__ unsigned sA[kLds], sB[kLds];
     __shared__ unsigned short sPosA[WIDE ? kCap : 1], sPosB[WIDE ? kCap : 1];
-    __shared__ unsigned sCur[kBkWaves][256];
-    __shared__ unsigned sWave[kBkWaves];
+    __shared__ unsigned sCur[(THREADS / 64)][256];
+    __shared__ unsigned sWave[(THREADS / 64)];
     __shared__ unsigned sOff[kBkMaxTiles], sSrc[kBkMaxTiles];   // tile map: bucket offset and source slot
     const unsigned *__restrict__ tKeys = to.keys;
     const unsigned *__restrict__ tVals = to.vals;
@@ -201,7 +212,7 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
     const int numTiles = bs.tiles;
     const unsigned hPrev = t < j ? hist[t] : 0u;
     const unsigned tileWord = t < numTiles ? to.info[(size_t)bs.infoBase + (size_t)j * numTiles + t] : 0u;
-    const unsigned start = bs.pStart + block_sum(hPrev, sWave);
+    const unsigned start = bs.pStart + block_sum<THREADS>(hPrev, sWave);
     const int cnt = (int)hist[j];
     constexpr unsigned kPosMask = (1u << POSBITS) - 1u;
     const bool inLds = cnt <= kCap;
@@ -217,9 +228,9 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
                                   : c0 + (1ull << lowBits) < sceneEnd ? c0 + (1ull << lowBits) : sceneEnd;
     if (cnt == 0) {
         const unsigned long long n = c1 - c0;
-        if (OUT == kOutTable) block_fill(table, c0 + n * part / split, c0 + n * (part + 1) / split, start);
+        if (OUT == kOutTable) block_fill<THREADS>(table, c0 + n * part / split, c0 + n * (part + 1) / split, start);
         if (OUT == kOutIndex && part == 0)
-            for (unsigned w = t; w < (unsigned)(c1 - c0) >> 5; w += kBkThreads)
+            for (unsigned w = t; w < (unsigned)(c1 - c0) >> 5; w += THREADS)
                 ix.words[(c0 >> 5) + w] = make_uint2(0u, 0u);
         return;
     }
@@ -248,13 +259,13 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
     auto fill_table = [&](auto low) {
         // head: cells up to the first key; tail: cells past the last key
         const unsigned kFirst = low(0), kLast = low(cnt - 1);
-        if (part == 0) block_fill(table, c0, c0 + kFirst + 1ull < c1 ? c0 + kFirst + 1ull : c1, start);
-        if (part == nparts - 1) block_fill(table, c0 + kLast + 1ull, c1, start + (unsigned)cnt);
+        if (part == 0) block_fill<THREADS>(table, c0, c0 + kFirst + 1ull < c1 ? c0 + kFirst + 1ull : c1, start);
+        if (part == nparts - 1) block_fill<THREADS>(table, c0 + kLast + 1ull, c1, start + (unsigned)cnt);
         // between keys: the cells (k[i-1], k[i]] start at sorted position i (a lane per key, waves help
         // with long runs); this workgroup's share of the positions
-        const int rounds = (i1 - i0 + kBkThreads - 1) / kBkThreads;
+        const int rounds = (i1 - i0 + THREADS - 1) / THREADS;
         for (int r = 0; r < rounds; ++r) {
-            const int i = i0 + r * kBkThreads + t;
+            const int i = i0 + r * THREADS + t;
             const bool ok = i > 0 && i < i1;
             const unsigned kp = ok ? low(i - 1) : 0u, ki = ok ? low(i) : 0u;
             const bool has = ok && ki != kp;
@@ -270,9 +281,9 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
         unsigned *sBits = &sCur[0][0], *sBase = sBits + 2048;   // 2^16 cells at most
         const unsigned words = (unsigned)(c1 - c0) >> 5;
         const int lane = t & 63, wave = t >> 6;
-        const int seg = ((cnt + kBkThreads - 1) / kBkThreads) * 64;
+        const int seg = ((cnt + THREADS - 1) / THREADS) * 64;
         const int s0 = min(wave * seg, cnt), s1 = min(s0 + seg, cnt);
-        for (unsigned w = t; w < words; w += kBkThreads) sBits[w] = 0u;
+        for (unsigned w = t; w < words; w += THREADS) sBits[w] = 0u;
         unsigned heads = 0u;
         for (int g0 = s0; g0 < s1; g0 += 64) {
             const int i = g0 + lane;
@@ -281,7 +292,7 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
         if (lane == 0) sWave[wave] = heads;
         __syncthreads();
         unsigned k = start, all = 0u;
-        for (int w = 0; w < kBkWaves; ++w) {
+        for (int w = 0; w < (THREADS / 64); ++w) {
             if (w < wave) k += sWave[w];
             all += sWave[w];
         }
@@ -301,7 +312,7 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
         if (part == nparts - 1 && t == 0) ix.starts[start + all] = start + (unsigned)cnt;
         __syncthreads();
         const unsigned wa = words * (unsigned)part / (unsigned)nparts, wb = words * (unsigned)(part + 1) / (unsigned)nparts;
-        for (unsigned w = wa + t; w < wb; w += kBkThreads) ix.words[(c0 >> 5) + w] = make_uint2(sBits[w], sBase[w]);
+        for (unsigned w = wa + t; w < wb; w += THREADS) ix.words[(c0 >> 5) + w] = make_uint2(sBits[w], sBase[w]);
     };
     const unsigned base = (unsigned)c0;
     const uint64_t sceneKey = (uint64_t)(unsigned)to.bucketScene[g] << 30;
@@ -313,22 +324,22 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
         // every slot found first (LDS only), then every key and value load in flight at once; the
         // values wait in registers while the keys are sorted, then go to the buffer the sort left free,
         // so that the gathers below find a sorted key's value in LDS rather than in global memory
-        constexpr int kPer = (kCap + kBkThreads - 1) / kBkThreads;
+        constexpr int kPer = (kCap + THREADS - 1) / THREADS;
         unsigned sl[kPer], kv[kPer], vv[kPer];
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            const int i = t + q * kBkThreads;
+            const int i = t + q * THREADS;
             sl[q] = i < cnt ? slot((unsigned)i) : 0u;
         }
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            const int i = t + q * kBkThreads;
+            const int i = t + q * THREADS;
             kv[q] = i < cnt ? tKeys[sl[q]] : 0u;
             vv[q] = i < cnt ? tVals[sl[q]] : 0u;
         }
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            const int i = t + q * kBkThreads;
+            const int i = t + q * THREADS;
             if (i < cnt) {
                 if (WIDE) {
                     sA[i] = kv[q] - base;
@@ -343,8 +354,8 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
         unsigned short *srcP = sPosA, *dstP = sPosB;
         for (int sh = 0; sh < lowBits; sh += 8) {
             const int bits = min(8, lowBits - sh);
-            if (WIDE) stable_pass(LdsPairs{src, srcP}, LdsPairs{dst, dstP}, cnt, sh, bits, sCur, sWave);
-            else stable_pass(LdsItems{src}, LdsItems{dst}, cnt, POSBITS + sh, bits, sCur, sWave);
+            if (WIDE) stable_pass<THREADS>(LdsPairs{src, srcP}, LdsPairs{dst, dstP}, cnt, sh, bits, sCur, sWave);
+            else stable_pass<THREADS>(LdsItems{src}, LdsItems{dst}, cnt, POSBITS + sh, bits, sCur, sWave);
             unsigned *x = src;
             src = dst;
             dst = x;
@@ -356,12 +367,12 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
         unsigned *valAt = dst;          // valAt[i]: the value of the bucket's i-th key in gather order
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            const int i = t + q * kBkThreads;
+            const int i = t + q * THREADS;
             if (i < cnt) valAt[i] = vv[q];
         }
         __syncthreads();
         if (WIDE) {
-            for (int i = i0 + t; i < i1; i += kBkThreads) {
+            for (int i = i0 + t; i < i1; i += THREADS) {
                 store_key(i, base + sorted[i]);
                 vOut[start + i] = valAt[srcP[i]];
             }
@@ -370,7 +381,7 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
         // the gathers of the first two rounds of positions are issued before the table is filled, so
         // that their latency overlaps the table's stores; a lane past the part's end loads sorted
         // position 0 (the bucket is not empty) and stores nothing, so the loads need no branch
-        const int ia = i0 + t, ib = ia + kBkThreads;
+        const int ia = i0 + t, ib = ia + THREADS;
         const bool ha = ia < i1, hb = ib < i1;
         const unsigned wa = sorted[ha ? ia : 0], wb = sorted[hb ? ib : 0];
         const unsigned va = valAt[wa & kPosMask], vb = valAt[wb & kPosMask];
@@ -401,8 +412,8 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
         }
         // further rounds in pairs: both positions' gathers are issued before either's stores (a load
         // after a store also waits for the store); a position past the end reloads the first one
-        for (int i = ib + kBkThreads; i < i1; i += 2 * kBkThreads) {
-            const int i2 = i + kBkThreads;
+        for (int i = ib + THREADS; i < i1; i += 2 * THREADS) {
+            const int i2 = i + THREADS;
             const bool h2 = i2 < i1;
             const unsigned w = sorted[i], w2 = sorted[h2 ? i2 : i];
             const unsigned val = valAt[w & kPosMask], val2 = valAt[w2 & kPosMask];
@@ -433,7 +444,7 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
         // gathered into (kOut, vOut) at [start, start + cnt) as offsets from c0, and the sorted-copy
         // arrays' range (16 B per key) serves as the second buffer of the passes until the copies are
         // written; the keys get c0 back at the end
-        for (int i = t; i < cnt; i += kBkThreads) {
+        for (int i = t; i < cnt; i += THREADS) {
             const unsigned src = slot((unsigned)i);
             kOut[start + i] = tKeys[src] - base;
             vOut[start + i] = tVals[src];
@@ -443,18 +454,18 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
                                                      reinterpret_cast<unsigned *>(sVel + start)};
         int passes = 0;
         for (int sh = 0; sh < lowBits; sh += 8, ++passes) {
-            if ((passes & 1) == 0) stable_pass(a, b, cnt, sh, min(8, lowBits - sh), sCur, sWave);
-            else stable_pass(b, a, cnt, sh, min(8, lowBits - sh), sCur, sWave);
+            if ((passes & 1) == 0) stable_pass<THREADS>(a, b, cnt, sh, min(8, lowBits - sh), sCur, sWave);
+            else stable_pass<THREADS>(b, a, cnt, sh, min(8, lowBits - sh), sCur, sWave);
         }
         if (passes & 1) {
-            for (int i = t; i < cnt; i += kBkThreads) {
+            for (int i = t; i < cnt; i += THREADS) {
                 a.k[i] = b.k[i];
                 a.v[i] = b.v[i];
             }
             __syncthreads();
         }
         if (REORDER) {
-            for (int i = t; i < cnt; i += kBkThreads) {
+            for (int i = t; i < cnt; i += THREADS) {
                 const unsigned val = vOut[start + i];
                 sPos[start + i] = rec[2 * (size_t)val];
                 sVel[start + i] = rec[2 * (size_t)val + 1];
@@ -464,7 +475,7 @@ __global__ __launch_bounds__(kBkThreads) __attribute__((amdgpu_waves_per_eu(8)))
             else fill_table([&](int i) -> unsigned { return kOut[start + i]; });
             __syncthreads();
         }
-        for (int i = t; i < cnt; i += kBkThreads) store_key(i, kOut[start + i] + base);
+        for (int i = t; i < cnt; i += THREADS) store_key(i, kOut[start + i] + base);
     }
 }
 
@@ -576,6 +587,7 @@ bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *o
         if (sc.shift >= 0 && sc.shift <= maxShift && ((c + (1ll << sc.shift) - 1) >> sc.shift) <= maxBuckets)
             shift = sc.shift;
         if (shift < 0) return false;
+        if (!measured || sc.peak[shift] > kBkSmallPeak || tiles > kBkSmallThreads) p.small = false;
         BucketScene &b = p.scenes[s];
         b.pStart = (unsigned)pBase;
         b.n = (unsigned)n;
@@ -598,6 +610,7 @@ bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *o
         if (cBase > 0xffffffffll || info > 0x7fffffffll) return false;
     }
     p.infoWords = (size_t)info;
+    if (tk == kTileKeys || maxSceneBuckets > kBkSmallThreads) p.small = false;
     p.bucketBits = maxSceneBuckets <= 256 ? 8 : maxSceneBuckets <= 512 ? 9 : 10;
     *out = std::move(p);
     return true;
@@ -607,24 +620,25 @@ void launch_bucket_sort(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, co
                         float4 *sortedVel, unsigned *table, unsigned numCells, int split, const CellIndex &ix,
                         hipStream_t st) {
     if (to.numBuckets <= 0) return;
-    if (ix.words) {
-        hipLaunchKernelGGL((k_bucket_sort<16, kOutIndex, false>), dim3(to.numBuckets * split), dim3(kBkThreads), 0, st, to,
-                           split, kOut, vOut, rec, sortedPos, sortedVel, nullptr, numCells, nullptr, ix);
-        return;
-    }
-    hipLaunchKernelGGL((k_bucket_sort<16, kOutTable, false>), dim3(to.numBuckets * split), dim3(kBkThreads), 0, st, to, split,
-                       kOut, vOut, rec, sortedPos, sortedVel, table, numCells, nullptr, ix);
+    auto run = [&](auto kernel, int threads, unsigned *tab) {
+        hipLaunchKernelGGL(kernel, dim3(to.numBuckets * split), dim3(threads), 0, st, to, split, kOut, vOut, rec, sortedPos,
+                           sortedVel, tab, numCells, nullptr, ix);
+    };
+    if (ix.words) run(k_bucket_sort<16, kOutIndex, false, kBkThreads>, kBkThreads, nullptr);
+    else if (to.small) run(k_bucket_sort<16, kOutTable, false, kBkSmallThreads>, kBkSmallThreads, table);
+    else run(k_bucket_sort<16, kOutTable, false, kBkThreads>, kBkThreads, table);
 }
 
 void launch_bucket_sort_morton(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, float4 *scratchA,
                                float4 *scratchB, uint64_t *kOut64, int maxShift, hipStream_t st) {
     if (to.numBuckets <= 0) return;
-    auto run = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(to.numBuckets), dim3(kBkThreads), 0, st, to, 1, kOut, vOut, nullptr, scratchA,
+    auto run = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(to.numBuckets), dim3(threads), 0, st, to, 1, kOut, vOut, nullptr, scratchA,
                            scratchB, nullptr, 0u, kOut64, CellIndex{});
     };
-    if (maxShift <= 32 - 12) run(k_bucket_sort<12, kOutKeys, false>);
-    else run(k_bucket_sort<12, kOutKeys, true>);
+    if (maxShift <= 32 - 12) run(k_bucket_sort<12, kOutKeys, false, kBkThreads>, kBkThreads);
+    else if (to.small) run(k_bucket_sort<12, kOutKeys, true, kBkSmallThreads>, kBkSmallThreads);
+    else run(k_bucket_sort<12, kOutKeys, true, kBkThreads>, kBkThreads);
 }
 
 }  // namespace arsim

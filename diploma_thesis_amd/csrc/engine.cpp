@@ -843,7 +843,7 @@ int Engine::enqueue_grid_broadphase(const BodyBufs &bb, const PartBufs &pb, cons
             rec();
         }
         const TileKeyOut to{(unsigned *)keysB, valsB, tileInfo, bucketHist, bkScenesD, tileSceneD, bucketSceneD,
-                            numTiles, numBuckets, tileKeys, bkPlan.bucketBits};
+                            numTiles, numBuckets, tileKeys, bkPlan.bucketBits, bkPlan.small};
         launch_pose_key_tiles(pb, ahead ? ahead_bufs() : bb, N, ph, sv, to, grainVelDead, st);
         rec();
         const int split = tu.bucketSplit == 1 || tu.bucketSplit == 2 ? tu.bucketSplit : (numBuckets < 512 ? 2 : 1);
@@ -958,7 +958,7 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
             rec();
         }
         TileKeyOut to{(unsigned *)keysB, valsB, tileInfo, bucketHist, bkScenesD, tileSceneD, bucketSceneD,
-                      numTiles, numBuckets, tileKeys, bkPlan.bucketBits};
+                      numTiles, numBuckets, tileKeys, bkPlan.bucketBits, bkPlan.small};
         const bool m63 = method == ARSIM_METHOD_LBVH63;
         to.morton = m63 ? 2 : 1;
         to.code63 = code63;

@@ -183,6 +183,7 @@ struct TileKeyOut {
     const int *tileScene, *bucketScene;   // scene of each tile and of each bucket
     int numTiles, numBuckets, tileKeys;
     int bucketBits;                       // a scene has at most 2^bucketBits buckets (8, 9 or 10)
+    bool small = false;                   // every bucket is small (the plan's)
     // Morton keys (each scene's codes cut into buckets of 2^shift, 20 <= shift <= 30): 1 = 30-bit codes;
     // 2 = 63-bit codes, whose top 30 bits (the 30-bit code) are the tile keys while the full codes go to
     // code63 in particle order
@@ -213,6 +214,7 @@ struct BucketPlan {
     std::vector<int> tileScene, bucketScene;
     size_t infoWords = 0;
     int tileKeys = kTileKeys;
+    bool small = true;    // every measured bucket is small, and a scene's tiles and buckets few: small workgroups
     int bucketBits = 8;   // the most buckets of one scene, rounded up to a power of two (at least 2^8)
 };
 // maxShift / capKeys: the widest bucket (2^maxShift cells) and the most keys a bucket sorted in LDS holds
