@@ -270,7 +270,7 @@ __device__ __forceinline__ uint64_t pose_key_one(int i, PartBufs p, BodyBufs b, 
 // the grid sort: the bucket kernel gathers each bucket's keys from its scene's tiles' runs, in tile
 // order.  Wave w owns particles [tile + 256 w, tile + 256 w + 256), four per lane, so (wave, item,
 // lane) order is particle order.
-constexpr int kTileItems = 4;   // particles per thread
+constexpr int kTileItems = 4;   // particles per thread (two in tiles of 512)
 
 template <int BITS>
 __device__ __forceinline__ uint64_t match_bits(unsigned d, bool ok) {
@@ -285,11 +285,11 @@ __device__ __forceinline__ uint64_t match_bits(unsigned d, bool ok) {
     return peers;
 }
 
-template <int MODE, int THREADS, int BITS>
+template <int MODE, int THREADS, int BITS, int ITEMS>
 __global__ __launch_bounds__(THREADS) void k_pose_key_tiles(PartBufs p, BodyBufs b, int N, DevPhys ph, SceneView sv,
                                                             TileKeyOut to, int grainVelDead) {
     constexpr int WAVES = THREADS / 64;
-    constexpr int TILE = THREADS * kTileItems;
+    constexpr int TILE = THREADS * ITEMS;
     constexpr int RADIX = 1 << BITS;   // buckets a scene may have
     static_assert(RADIX <= THREADS, "a thread per bucket");
     __shared__ unsigned sWaveHist[WAVES][RADIX];
@@ -303,16 +303,16 @@ __global__ __launch_bounds__(THREADS) void k_pose_key_tiles(PartBufs p, BodyBufs
     const long long tileBase = (long long)bs.pStart + (long long)kt * TILE;
     const long long sceneEnd = (long long)bs.pStart + bs.n;
     const long long tileEnd = tileBase + TILE < sceneEnd ? tileBase + TILE : sceneEnd;
-    const long long waveBase = tileBase + (long long)wave * (kTileItems * 64);
+    const long long waveBase = tileBase + (long long)wave * (ITEMS * 64);
     KeyOut ko{};
     ko.grainVelDead = grainVelDead != 0;
     if (MODE == kKeyMorton63) ko.keys = to.code63;   // the full codes, in particle order
     // the scene's geometry and every item's rbIndex requested first: the items' poses depend on them,
     // and the stores of one item's pose keep the compiler from moving the next item's loads above them
     const SceneGeom geom = sv.table[scene];
-    int rbv[kTileItems];
+    int rbv[ITEMS];
 #pragma unroll
-    for (int k = 0; k < kTileItems; ++k) {
+    for (int k = 0; k < ITEMS; ++k) {
         const long long i = waveBase + k * 64 + lane;
         rbv[k] = i < tileEnd && p.rb ? p.rb[i] : -1;
     }
@@ -322,10 +322,10 @@ __global__ __launch_bounds__(THREADS) void k_pose_key_tiles(PartBufs p, BodyBufs
     __builtin_amdgcn_s_waitcnt(0x0f70);
     // items in pairs: both items' loads are issued before either item's stores, so a pair costs one
     // round trip (a load after a store also waits for the store)
-    unsigned keys[kTileItems];
-    static_assert(kTileItems % 2 == 0, "items in pairs");
+    unsigned keys[ITEMS];
+    static_assert(ITEMS % 2 == 0, "items in pairs");
 #pragma unroll
-    for (int k = 0; k < kTileItems; k += 2) {
+    for (int k = 0; k < ITEMS; k += 2) {
         const long long iA = waveBase + k * 64 + lane, iB = iA + 64;
         PoseIn inA{}, inB{};
         if (iA < tileEnd) inA = pose_load((int)iA, rbv[k], p, b, 1, 1);
@@ -342,9 +342,9 @@ __global__ __launch_bounds__(THREADS) void k_pose_key_tiles(PartBufs p, BodyBufs
     __syncthreads();
     // ranks within the wave, in particle order
     const uint64_t lower = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    unsigned rank[kTileItems];
+    unsigned rank[ITEMS];
 #pragma unroll
-    for (int k = 0; k < kTileItems; ++k) {
+    for (int k = 0; k < ITEMS; ++k) {
         const bool valid = waveBase + k * 64 + lane < tileEnd;
         const unsigned d = valid ? (keys[k] - bs.cellBase) >> bs.shift : 0u;
         const uint64_t peers = match_bits<BITS>(d, valid);
@@ -386,7 +386,7 @@ __global__ __launch_bounds__(THREADS) void k_pose_key_tiles(PartBufs p, BodyBufs
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kTileItems; ++k) {
+    for (int k = 0; k < ITEMS; ++k) {
         const long long i = waveBase + k * 64 + lane;
         if (i < tileEnd) {
             const unsigned d = (keys[k] - bs.cellBase) >> bs.shift;
@@ -759,10 +759,11 @@ void launch_pose_key_tiles(const PartBufs &p, const BodyBufs &b, int numParticle
     };
     auto of_mode = [&](auto mode) {
         constexpr int M = decltype(mode)::value;
-        if (to.tileKeys == 1024) run(k_pose_key_tiles<M, 256, 8>, 256);
-        else if (to.bucketBits <= 8) run(k_pose_key_tiles<M, 1024, 8>, 1024);
-        else if (to.bucketBits == 9) run(k_pose_key_tiles<M, 1024, 9>, 1024);
-        else run(k_pose_key_tiles<M, 1024, 10>, 1024);
+        if (to.tileKeys == 512) run(k_pose_key_tiles<M, 256, 8, 2>, 256);
+        else if (to.tileKeys == 1024) run(k_pose_key_tiles<M, 256, 8, kTileItems>, 256);
+        else if (to.bucketBits <= 8) run(k_pose_key_tiles<M, 1024, 8, kTileItems>, 1024);
+        else if (to.bucketBits == 9) run(k_pose_key_tiles<M, 1024, 9, kTileItems>, 1024);
+        else run(k_pose_key_tiles<M, 1024, 10, kTileItems>, 1024);
     };
     if (to.morton == 2) of_mode(std::integral_constant<int, kKeyMorton63>{});
     else if (to.morton) of_mode(std::integral_constant<int, kKeyMorton30>{});

@@ -525,9 +525,10 @@ bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *o
         nTot += sh.particles;
         tiles4k += (sh.particles + kTileKeys - 1) / kTileKeys;
     }
-    // tiles of 4096 particles, or of 1024 for at most 65,536 particles (too few tiles otherwise) and
-    // where more than a fifth of the larger tiles' slots would lie past scene ends
-    const int tk = nTot <= 65536 || (double)tiles4k * kTileKeys > 1.25 * (double)nTot ? 1024 : kTileKeys;
+    // tiles of 4096 particles, or of 512 for at most 65,536 particles (too few tiles otherwise: with tiles of 1024 the
+    // step of 16,384 particles takes 32.8 us, with 512 30.9; 65,000 48.3 and 47.2) and of 1024 where more than a
+    // fifth of the larger tiles' slots would lie past scene ends
+    const int tk = nTot <= 65536 ? 512 : (double)tiles4k * kTileKeys > 1.25 * (double)nTot ? 1024 : kTileKeys;
     // keys per bucket on average: a 512th of all keys (512 buckets fill the GPU with one workgroup
     // each; 256 buckets with two workgroups each, which sort every bucket twice, and 1,024 buckets
     // were slower at 2^20 keys), at least 64 and at most 3/4 of what a workgroup sorts in LDS

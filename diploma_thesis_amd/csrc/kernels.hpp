@@ -163,7 +163,7 @@ void launch_reorder_seg(const unsigned *sortedKeys, const unsigned *sortedIdx, c
 // The bucket sort's plan (bucket.hip).  Scene s holds particles [pStart, pStart + n) and cells
 // [cellBase, cellBase + cells); the scenes' cell ranges are packed in scene order, so the keys of
 // scene s sort below those of scene s + 1 and the scene's sorted range is its particle range.  A
-// scene's cells are cut into `buckets` (at most 1,024; 256 with tiles of 1024) ranges of 2^shift cells
+// scene's cells are cut into `buckets` (at most 1,024; 256 with tiles of 512 or 1024) ranges of 2^shift cells
 // (shift <= 16), the scene's bucket j being global bucket bucketBase + j; its particles into `tiles`
 // tiles of tileKeys particles, global tiles tileBase .. tileBase + tiles - 1.  One scene of 2^20
 // particles over 2^24 cells is cut into 512 buckets of its top 9 key bits.

@@ -41,6 +41,12 @@ def test_small_scene_vs_oracle(n, method):
     run_both([scenes.mix_scene(n, 7 + n % 5, method)])
 
 
+@pytest.mark.parametrize("n", [511, 512, 513, 65536, 65537])
+def test_tile_edges_vs_oracle(n):
+    print(f"small buckets: {n} particles at the edges of the tiles", flush=True)
+    run_both([scenes.mix_scene(n, 9)])
+
+
 @pytest.mark.parametrize("method", METHODS[:2], ids=["grid", "lbvh30"])
 def test_small_batch_vs_oracle(method):
     print(f"small buckets: batch, method {method}", flush=True)
