@@ -448,8 +448,11 @@ int Engine::build(const std::vector<SceneSource> &src, const ArSimTuning *tuning
         ARSIM_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
         ownStream = true;
     }
-    // a rebuild starts from a clean step state; buffers are kept where they are large enough
+    // a rebuild starts from a clean step state; buffers are kept where they are large enough, but what the
+    // last step left in them belongs to the layout before
     invalidate_graph();
+    lastKeys = nullptr;
+    lastIdx = nullptr;
     free_static();
     if (tuning) tu = *tuning;
     if (tu.demBlock <= 0 || tu.demBlock > 1024 || (tu.demBlock & 63)) return fail(ARSIM_ERR_INVALID_ARG, "bad demBlock");
@@ -1385,10 +1388,10 @@ int arsim_engine_debug_buffers(arsim_engine *e, void **sortedKeys, void **sorted
     Engine &E = e->e;
     if (sortedKeys) *sortedKeys = E.lastKeys;
     if (sortedIndex) *sortedIndex = E.lastIdx;
-    if (cellStart) {
+    if (cellStart) {   // the engine's cell index: CSR offsets over cell segments
         if (int rc = E.table_for_view()) return rc;   // (a step with the compact index keeps no table)
+        *cellStart = E.useIndex && !E.lastKeys ? nullptr : E.segStart;
     }
-    if (cellStart) *cellStart = E.segStart;   // the engine's cell index: CSR offsets over cell segments
     if (cellEnd) *cellEnd = nullptr;
     if (sortedPos) *sortedPos = E.sortedPos;
     if (sortedVel) *sortedVel = E.method == ARSIM_METHOD_GRID ? (void *)E.sortedVel : (void *)E.tree.sortedVel;
