@@ -5,6 +5,8 @@
 #include <string>
 #include <vector>
 
+#include <mutex>
+
 #include "../../include/arsim.h"
 #include "kernels.hpp"
 
@@ -115,8 +117,9 @@ struct Engine {
     hipGraphExec_t gexec = nullptr;
     bool graphReady = false;
 
-    // pinned host memory that small reads of the state come through (allocated at the first one)
+    // pinned host memory that small reads of the state come through (allocated at the first one), one read at a time
     unsigned *fetchBuf = nullptr;
+    std::mutex fetchLock;
     struct Fetch {
         void *dst;
         const void *src;
