@@ -52,8 +52,7 @@ __device__ __forceinline__ void dem_write(f3 F, int ra, f3 pa, f3 va, unsigned o
 // when a queue could overflow or the particle's cells are done, two at a time.  Formed in the candidate loop, a wave
 // ran the pair force in every iteration in which any of its lanes had a contact; queued, it runs it about as often as
 // its fullest lane has contacts.  Three candidates' loads together, 16 entries (12 drain too often: 922 us a step at
-// the pile below, 16 874; two loads 900, four 878).  Settled piles: 2^22 particles 634 -> 534 us, the reference's layout at
-// 300,007 88 -> 65.  Where few candidates are contacts the positions read a second time cost more than that gives.
+// the pile below, 16 874; two loads 900, four 878).  Settled pile of 2^22 particles: 634 -> 534 us.  Where few candidates are contacts the positions read a second time cost more than that gives.
 constexpr int kQueue = 16, kQueueAhead = 3;
 constexpr int kQueueMax = (1 << 28) - 4;   // particles: an entry holds 16 times a sorted position, read up to kQueueAhead on
 __device__ __forceinline__ float4 at16(const float4 *__restrict__ p, unsigned byteOffset) {
@@ -183,7 +182,12 @@ __global__ void k_dem_grid(const float4 *__restrict__ sPos, const float4 *__rest
     }
 }
 
-// The same sums over queued contacts.
+// The same sums over queued contacts, a row's three cells together: their starts in one round trip, then their ends,
+// and where the cells' runs follow each other (unless x wraps they do in a sorted point set) one run of candidates.
+// Bound by the table's lines: in a scattered scene with twice 64 MB of tables every row is a miss, and read cell by
+// cell the eight waves a SIMD evicted each other's lines between a row's reads.  Cell by cell with one candidate at a
+// time and no queue, cell by cell with the queue, and now: 2^20 scattered particles 157, 240 and 117 us, piles of
+// 300,007 77, 57 and 49, of 2^22 848, 692 and 555, a mixed scene of 800,000 211, 192 and 163.
 __global__ void k_dem_grid_ref_queue(const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
                                      const unsigned *__restrict__ sIdx, const unsigned *__restrict__ cs,
                                      const unsigned *__restrict__ ce, int n, DevPhys ph, SceneGeom g, DemOut o) {
@@ -197,16 +201,32 @@ __global__ void k_dem_grid_ref_queue(const float4 *__restrict__ sPos, const floa
     int gx, gy, gz;
     grid_pos(pa, g, gx, gy, gz);
     ContactQueue cq(queueLds + threadIdx.x, blockDim.x);
-    int c = 0;
-    for (int z = -1; z <= 1; ++z)
-        for (int y = -1; y <= 1; ++y)
-            for (int x = -1; x <= 1; ++x, ++c) {
-                const unsigned h = g.cellBase + grid_hash(gx + x, gy + y, gz + z, g);
-                const unsigned st = cs[h];
-                if (st == kEmpty) continue;
-                const unsigned en = ce[h];
-                cq.run(sPos, sVel, st, en, en, en, c, (unsigned)i << 4, ra, pa, va, ph);
+    for (int r = 0; r < 9; ++r) {
+        const int y = gy + r % 3 - 1, z = gz + r / 3 - 1;
+        const unsigned h[3] = {g.cellBase + grid_hash(gx - 1, y, z, g), g.cellBase + grid_hash(gx, y, z, g),
+                               g.cellBase + grid_hash(gx + 1, y, z, g)};
+        unsigned b[3], e[3];
+        bool some[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) b[k] = cs[h[k]];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) e[k] = b[k] != kEmpty ? ce[h[k]] : 0u;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) some[k] = b[k] < e[k];
+        // the cells' runs lie one after another unless x wraps (or a caller's own table says otherwise)
+        const unsigned last = some[2] ? e[2] : some[1] ? e[1] : e[0];
+        const unsigned b2 = some[2] ? b[2] : last, b1 = some[1] ? b[1] : b2;
+        const bool joined = (!some[0] || e[0] == b1) & (!some[1] || e[1] == b2);
+        if (joined) {
+            cq.run(sPos, sVel, some[0] ? b[0] : b1, b1, b2, last, 3 * r, (unsigned)i << 4, ra, pa, va, ph);
+        } else {
+#pragma unroll 1
+            for (int k = 0; k < 3; ++k) {
+                const unsigned st = k == 0 ? b[0] : k == 1 ? b[1] : b[2], en = k == 0 ? e[0] : k == 1 ? e[1] : e[2];
+                if (st < en) cq.run(sPos, sVel, st, en, en, en, 3 * r + k, (unsigned)i << 4, ra, pa, va, ph);
             }
+        }
+    }
     cq.drain(sPos, sVel, pa, va, ph);
     dem_write(add3(cq.F, cq.csum), ra, pa, va, sIdx[i], ph, g, o);
 }
