@@ -32,6 +32,7 @@ struct SceneView {
     // several scenes: scene s's particles are the sorted positions [sceneStart[s], sceneStart[s + 1])
     // (NULL where the caller has no such table)
     const int *sceneStart;
+    int boundaryBlocks;   // several scenes: workgroups of the contact kernels for the boundaries between them
 };
 
 struct DevPhys {

@@ -252,8 +252,12 @@ SceneView Engine::scene_view() const {
     SceneView sv{};
     sv.count = S;
     sv.table = geomD;
-    if (S == 1) sv.single = geoms[0];
-    else sv.sceneStart = sceneStartD;
+    if (S == 1) {
+        sv.single = geoms[0];
+    } else {
+        sv.sceneStart = sceneStartD;
+        sv.boundaryBlocks = (S - 1 + 7) / 8 * 8;
+    }
     return sv;
 }
 

@@ -431,7 +431,9 @@ enum { kGeomSingle = 0, kGeomBlock = 1, kGeomLane = 2 };
 // block that holds the boundary with kGeomLane (if the boundary lies strictly inside a block and no
 // earlier boundary lies strictly inside the same one), then every block, those of one scene being
 // taken with kGeomBlock.  As a launch of their own after the others the boundary blocks were alone on the
-// chip for 27 to 37 us: 128 scenes' step 314 -> 289 us, 24 larger scenes' 50 steps 14.7 -> 13.5 ms.
+// chip for 27 to 37 us: 128 scenes' step 314 -> 289 us, 24 larger scenes' 50 steps 14.7 -> 13.5 ms.  They are filled up
+// to a multiple of the XCDs (sv.boundaryBlocks), so that the blocks after them run on the XCD whose L2 the bucket sort left
+// them in, and the next step's bucket sort finds its own: 8 scenes of 16,000 particles step 68.8 -> 61.9 us.
 __device__ __forceinline__ bool boundary_block(const SceneView &sv, int n, int &lb) {
     const int k = (int)blockIdx.x + 1, bs = (int)blockDim.x;
     const int b = sv.sceneStart[k], pb = sv.sceneStart[k - 1];
@@ -452,9 +454,10 @@ __device__ __forceinline__ void for_dem_block(const SceneView &sv, const float4 
         body(xcd_block((int)blockIdx.x, (int)gridDim.x), sv.single, std::integral_constant<int, kGeomSingle>{});
         return;
     }
-    const int boundaries = sv.count - 1;
+    const int boundaries = sv.boundaryBlocks;
     int lb, scene;
     if ((int)blockIdx.x < boundaries) {
+        if ((int)blockIdx.x >= sv.count - 1) return;   // (a block that only fills up)
         if (!boundary_block(sv, n, lb) || one_scene(sVel, lb, n, scene)) return;
         body(lb, SceneGeom{}, std::integral_constant<int, kGeomLane>{});
         return;
@@ -838,7 +841,7 @@ void launch_dem_grid_seg(const float4 *sortedPos, const float4 *sortedVel, const
     if (queue && !o.pairs && segBits == 0 && n < kQueueMax) {
         const size_t lds = (size_t)block * kQueue * sizeof(unsigned);
         if (sceneInVelW)
-            hipLaunchKernelGGL(k_dem_grid_queue<true>, dim3(grid.x + (unsigned)sv.count - 1u), dim3(block), lds, st,
+            hipLaunchKernelGGL(k_dem_grid_queue<true>, dim3(grid.x + (unsigned)sv.boundaryBlocks), dim3(block), lds, st,
                                sortedPos, sortedVel, sortedIdx, segStart, n, ph, sv, o);
         else
             hipLaunchKernelGGL(k_dem_grid_queue<false>, grid, dim3(block), lds, st, sortedPos, sortedVel, sortedIdx,
@@ -847,7 +850,7 @@ void launch_dem_grid_seg(const float4 *sortedPos, const float4 *sortedVel, const
     }
     auto run = [&](auto single, auto batch) {
         if (sceneInVelW)
-            hipLaunchKernelGGL(batch, dim3(grid.x + (unsigned)sv.count - 1u), dim3(block), 0, st, sortedPos, sortedVel,
+            hipLaunchKernelGGL(batch, dim3(grid.x + (unsigned)sv.boundaryBlocks), dim3(block), 0, st, sortedPos, sortedVel,
                                sortedKeys, sortedIdx, segStart, segBits, n, ph, sv, o);
         else
             hipLaunchKernelGGL(single, grid, dim3(block), 0, st, sortedPos, sortedVel, sortedKeys, sortedIdx, segStart,
@@ -870,7 +873,7 @@ void launch_dem_grid_index(const float4 *sortedPos, const float4 *sortedVel, con
     const unsigned all = (unsigned)((n + block - 1) / block);
     const size_t lds = (size_t)9 * block * sizeof(unsigned);
     if (sceneInVelW)
-        hipLaunchKernelGGL(k_dem_grid_index<true>, dim3(all + (unsigned)sv.count - 1u), dim3(block), lds, st, sortedPos,
+        hipLaunchKernelGGL(k_dem_grid_index<true>, dim3(all + (unsigned)sv.boundaryBlocks), dim3(block), lds, st, sortedPos,
                            sortedVel, sortedIdx, ix, n, ph, sv, o);
     else
         hipLaunchKernelGGL(k_dem_grid_index<false>, dim3(all), dim3(block), lds, st, sortedPos, sortedVel, sortedIdx, ix,
