@@ -36,6 +36,7 @@ namespace {
 // 40 of 32,768 (8) 197 -> 203, 50 of 24,000 (11) 183 -> 179, 60 of 16,384 (16) 144 -> 134, the
 // 2^20-particle scene (16) 148 -> 136.
 constexpr double kIndexCells = 10.0;
+constexpr int kIndexMin = 3 << 16;   // and more particles than this
 // Contacts are queued before they are evaluated (launch_dem_grid_seg) where the particles lie as densely as this: in
 // a settled pile (2.3) the contact kernel of 10^6 particles takes 138 us against 178, of 2^22 534 against 634, in one
 // mixed scene of 800,000 (5.4) 164 against 172, and in scattered scenes (0.3) 30 against 27.  With several scenes two
@@ -586,7 +587,8 @@ int Engine::build(const std::vector<SceneSource> &src, const ArSimTuning *tuning
             }
             bucketSort = plan_bucket_sort(shapes, &bkPlan);
             queueContacts = density >= (S > 1 ? kQueueDensityBatch : kQueueDensity);
-            useIndex = bucketSort && N > kCoopMax && (double)numCells >= kIndexCells * (double)N && !(flags & ARSIM_CONTACT_SIS) && !tu.fuseReduce;
+            coopContacts = N <= (S > 1 ? kCoopMaxBatch : density >= kCoopDensity ? kCoopMaxDense : kCoopMax);
+            useIndex = bucketSort && N > kIndexMin && (double)numCells >= kIndexCells * (double)N && !(flags & ARSIM_CONTACT_SIS) && !tu.fuseReduce;
             for (int s = 0; useIndex && s < S; ++s)   // rows within a bucket, buckets of whole words
                 useIndex = (1u << bkPlan.scenes[s].shift) >= std::max(geoms[s].gridMask[0] + 1u, 32u) &&
                            bkPlan.scenes[s].cells % 32u == 0u;
@@ -956,7 +958,7 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
                 launch_dem_grid_index(sortedPos, sortedVel, vA, cell_index(), N, ph, sv, S > 1, o, tu.demBlock, st);
             else
                 launch_dem_grid_seg(sortedPos, sortedVel, kA, vA, segStart, segBits, N, ph, sv, S > 1, o,
-                                    queueContacts, tu.demBlock, st);
+                                    coopContacts, queueContacts, tu.demBlock, st);
             if (numStatic)
                 launch_dem_static(sortedPos, sortedVel, vA, N, stPos, stNorm, nullptr, stTable, nullptr, ph, geoms[0],
                                   pForce, nullptr, relPos, false, st);
@@ -1120,7 +1122,7 @@ int Engine::enqueue_broadphase(int *pairsD, int *countsD, int maxPer) {
         launch_fill_u32(longCnt, 0u, 1, st);
         launch_reorder_seg(kA, vA, pos, vel, rb, S > 1 ? scene : nullptr, gatherRec, sortedPos, sortedVel, segStart,
                            segBits, numSegs, N, long_fill(), st);
-        launch_dem_grid_seg(sortedPos, sortedVel, kA, vA, segStart, segBits, N, ph, sv, S > 1, o, false, tu.demBlock, st);
+        launch_dem_grid_seg(sortedPos, sortedVel, kA, vA, segStart, segBits, N, ph, sv, S > 1, o, false, false, tu.demBlock, st);
         prevSorted = kA;
         lastKeys = kA;
         lastIdx = vA;

@@ -63,6 +63,7 @@ struct Engine {
     unsigned *valsA = nullptr, *valsB = nullptr;
     unsigned *segStart = nullptr;           // grid: CSR offsets over segments of 2^segBits cells
     double density = 0.0;                   // grid: particles per cell around a particle, of the scenes as given
+    bool coopContacts = false;              // grid: 16 lanes a particle (launch_dem_grid_seg)
     bool queueContacts = false;             // grid: contacts queued before they are evaluated (launch_dem_grid_seg)
     bool useIndex = false;                  // grid, bucket sort: the compact cell index instead (kernels.hpp)
     uint2 *cellWords = nullptr;

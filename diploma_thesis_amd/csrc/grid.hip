@@ -696,10 +696,14 @@ __global__ __attribute__((amdgpu_waves_per_eu(8))) void k_dem_grid_index(const f
 
 // The contact kernel with 16 lanes per particle (coop_cells): cells of the reference's cellStart / cellEnd (REF)
 // or of the exact table (cs = segStart); sceneTable: each particle's scene (its id in sortedVel.w), else the one
-// scene g.  Up to kCoopMax particles there are too few waves to hide a thread's chain of lookups and
-// candidate loads: 16,384 particles of c0's cubes 15.2 -> 9.6 us, 50,021 mixed ones 25 -> 17, piles of 65,536
-// and 131,072 61 -> 28 and 60 -> 47; at 200,003 58.8 -> 57.7, and a pile of 300,007 is slower (86 -> 93): there
-// the lanes' shared steps (slots, ranks, the ordered adds) cost more than the chains.
+// scene g.  For the sizes at which there are too few waves to hide a thread's chain of lookups and candidate loads:
+// 16,384 particles of c0's cubes 15.2 -> 9.6 us, 50,021 mixed ones 25 -> 17, a pile of 65,536 61 -> 28.  The lanes'
+// shared steps (slots, ranks, the ordered adds) cost more than the chains from about (per thread and with 16 lanes, us)
+//   one scene: 91,000 mixed 32 and 26.5, 98,000 25.7 and 27.1, 196,608 48 and 55; cubes 91,000 26 and 23, 196,608 30
+//   and 43; piles 131,000 48.8 and 46.6 (the queue), 150,000 51.2 and 52.0, 196,608 54 and 64
+//   several: 4 of 17,000 21.8 and 18.8, 24 of 3,000 21.4 and 20.2, 5 of 16,000 17.7 and 21.1,
+//   12 of 16,000 21 and 40, 100 of 1,900 23 and 40
+//   the reference's layout: 91,000 mixed 28 and 25, 98,000 20 and 26; piles 91,000 36 and 33, 115,000 36 and 40
 constexpr int kCoopBlock = 128;
 template <bool REF>
 __global__ __launch_bounds__(kCoopBlock) void k_dem_grid_coop(const float4 *__restrict__ sPos,
@@ -826,11 +830,11 @@ void launch_fill_long(unsigned *table, unsigned long long tableSize, const LongF
 
 void launch_dem_grid_seg(const float4 *sortedPos, const float4 *sortedVel, const unsigned *sortedKeys,
                          const unsigned *sortedIdx, const unsigned *segStart, int segBits, int n, const DevPhys &ph,
-                         const SceneView &sv, bool sceneInVelW, const DemOut &o, bool queue, int block,
-                         hipStream_t st) {
+                         const SceneView &sv, bool sceneInVelW, const DemOut &o, bool coop, bool queue,
+                         int block, hipStream_t st) {
     if (n <= 0) return;
     if (block <= 0) block = 128;
-    if (!o.pairs && segBits == 0 && n <= kCoopMax) {
+    if (coop && !o.pairs && segBits == 0) {
         const int per = kCoopBlock / kCoopLanes;
         hipLaunchKernelGGL(k_dem_grid_coop<false>, dim3((n + per - 1) / per), dim3(kCoopBlock), 0, st, sortedPos,
                            sortedVel, sortedIdx, segStart, nullptr, n, ph, sv.single, sceneInVelW ? sv.table : nullptr,

@@ -256,14 +256,16 @@ unsigned fill_long_capacity(unsigned long long tableSize);
 void launch_fill_long(unsigned *table, unsigned long long tableSize, const LongFill &lf, hipStream_t st);
 void launch_dem_grid_seg(const float4 *sortedPos, const float4 *sortedVel, const unsigned *sortedKeys,
                          const unsigned *sortedIdx, const unsigned *segStart, int segBits, int n, const DevPhys &ph,
-                         const SceneView &sv, bool sceneInVelW, const DemOut &o, bool queue, int block,
+                         const SceneView &sv, bool sceneInVelW, const DemOut &o, bool coop, bool queue, int block,
                          hipStream_t st);
 // The same with the compact cell index (forces only).
 void launch_dem_grid_index(const float4 *sortedPos, const float4 *sortedVel, const unsigned *sortedIdx,
                            const CellIndex &ix, int n, const DevPhys &ph, const SceneView &sv, bool sceneInVelW,
                            const DemOut &o, int block, hipStream_t st);
-// Up to this many particles the contact kernel takes 16 lanes per particle and the exact cell table.
-constexpr int kCoopMax = 3 << 16;
+// Up to this many particles the contact kernels take 16 lanes per particle: one scene, one of kCoopDensity particles
+// per cell and more around a particle, several scenes together.
+constexpr int kCoopMax = 11 << 13, kCoopMaxDense = 1 << 17, kCoopMaxBatch = 9 << 13;
+constexpr double kCoopDensity = 2.0;
 // Grid DEM fused with the per-body reduction and apply (exact cell table, no static collider set):
 // bodies take one wave each, grains 64 per wave.  rec is the pose kernel's gather record in the
 // original order (pos.xyz + rbIndex bits, vel.xyz + scene id); grainIdx lists every grain's index.
