@@ -43,6 +43,16 @@ constexpr int kIndexMin = 3 << 16;   // and more particles than this
 // piles of 500,000 148 against 179, but 24 mixed scenes (1.7 and less) 1 % longer.
 constexpr double kQueueDensity = 1.0, kQueueDensityBatch = 2.0;
 
+// Morton buckets past the LDS are sorted in global memory by one workgroup each, about 5 us per 1,000 keys, so scenes in
+// a small part of their Morton box take the onesweep passes: 8,000 particles in one bucket 51 us against 45 for
+// 30-bit codes and 53 against 89 for 63-bit ones, 16,000 90 and 93 against 46 and 91, 65,000 319 and 338 against 47 and 94.
+constexpr unsigned kMostMorton30 = 7168u, kMostMorton63 = 14336u;
+// 63-bit codes that share their upper 30 bits are ranked among each other (k_morton63_ties), about 0.12 us for each of the
+// longest run, which up to 256 is less than the onesweep passes cost more (50 us): 300 to a code 52 us against 58, 1,000 140
+// against 67.  Looked for up to kTieParticles, while the count's table stays in the host's cache.
+constexpr unsigned kMostTies = 256u;
+constexpr int kTieParticles = 1 << 16;
+
 int ceil_log2(long long v) {
     int b = 0;
     while ((1ll << b) < v) ++b;
@@ -424,14 +434,15 @@ std::vector<unsigned> bucket_peaks(const float *pos4, int n, const SceneGeom &g,
 
 // The fullest bucket of a scene's 30-bit Morton codes for every bucket width of 2^20 codes (1,024 buckets) to
 // 2^30 (one), at index b of the plan's per-shift peaks (narrower ones: UINT_MAX), from host positions
-// normalised as the device does (for planning only).
-std::vector<unsigned> morton_peaks(const float *pos4, int n, const SceneGeom &g) {
+// normalised as the device does (for planning only).  ties (when given): the most particles of one 30-bit code, as
+// counted by a hash of it.
+std::vector<unsigned> morton_peaks(const float *pos4, int n, const SceneGeom &g, unsigned *ties) {
     // the code's upper 10 bits: the upper 4 bits of x's 10, 3 of y's and of z's, interleaved
     unsigned spread[16];   // bit k of the index to bit 3k
     for (unsigned v = 0; v < 16u; ++v) spread[v] = (v & 1u) | (v & 2u) << 2 | (v & 4u) << 4 | (v & 8u) << 6;
     double scale[3];
     for (int a = 0; a < 3; ++a) scale[a] = g.mExt[a] == 0.0f ? 0.0 : 1024.0 / g.mExt[a];
-    std::vector<unsigned> peak(31, 0xffffffffu), hist(1024, 0u);
+    std::vector<unsigned> peak(31, 0xffffffffu), hist(1024, 0u), code(ties ? 1u << 17 : 0u, 0u);
     for (int i = 0; i < n; ++i) {
         unsigned q[3];
         for (int a = 0; a < 3; ++a) {
@@ -439,7 +450,9 @@ std::vector<unsigned> morton_peaks(const float *pos4, int n, const SceneGeom &g)
             q[a] = v > 0.0 ? (v < 1023.0 ? (unsigned)v : 1023u) : 0u;   // NaN: 0
         }
         ++hist[spread[q[0] >> 6] | spread[q[1] >> 7] << 2 | spread[q[2] >> 7] << 1];
+        if (ties) ++code[(q[0] << 20 | q[1] << 10 | q[2]) * 2654435761u >> 15];
     }
+    if (ties) *ties = *std::max_element(code.begin(), code.end());
     for (int b = 20;; ++b) {
         peak[b] = *std::max_element(hist.begin(), hist.end());
         if (b == 30) return peak;
@@ -616,14 +629,18 @@ int Engine::build(const std::vector<SceneSource> &src, const ArSimTuning *tuning
         // particles' 63-bit codes 90 -> 17 us and their step 198 -> 116, a forest of 48 scenes 93 -> 38 us
         // and its step 334 -> 269, the body integration's launch among it)
         std::vector<BucketSceneShape> shapes(S);
+        const bool m63 = method == ARSIM_METHOD_LBVH63;
+        unsigned ties = 0u;
         for (int s = 0; s < S; ++s) {
             shapes[s].particles = pCount[s];
             shapes[s].grid[0] = shapes[s].grid[1] = shapes[s].grid[2] = 1024u;
-            if (src[s].host) shapes[s].peak = morton_peaks(src[s].host->pos, pCount[s], geoms[s]);
+            if (src[s].host)
+                shapes[s].peak = morton_peaks(src[s].host->pos, pCount[s], geoms[s], m63 && N <= kTieParticles ? &ties : nullptr);
             else if (src[s].from && src[s].from->mortonBucket)
                 shapes[s].shift = src[s].from->bkPlan.scenes[src[s].fromScene].shift;
         }
-        mortonBucket = plan_bucket_sort(shapes, &bkPlan, 30, 4096, true);
+        mortonBucket = ties <= kMostTies &&
+                       plan_bucket_sort(shapes, &bkPlan, 30, 4096, true, m63 ? kMostMorton63 : kMostMorton30);
     }
 
     // ---- allocation (everything a step touches, once)

@@ -219,9 +219,9 @@ struct BucketPlan {
 };
 // maxShift / capKeys: the widest bucket (2^maxShift cells) and the most keys a bucket sorted in LDS holds
 // (grid keys: 2^16 and 7,776; Morton keys: 2^30 and 4,096).  sharedCells: every scene's keys lie in the same range (Morton codes) instead of one
-// scene's after another's.
+// scene's after another's.  mostKeys: no plan where a measured bucket would hold more.
 bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *out, int maxShift = 16,
-                      int capKeys = 7776, bool sharedCells = false);
+                      int capKeys = 7776, bool sharedCells = false, unsigned mostKeys = 0xffffffffu);
 // The grid sort finished per bucket (bucket.hip): each bucket gathers its keys from its scene's
 // tiles' runs (tile order keeps the sort stable), `split` workgroups (1 or 2) sort it by the low bits,
 // each writing its share of the sorted keys / indices to (kOut, vOut), of the gathered sorted copies
