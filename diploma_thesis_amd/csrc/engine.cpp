@@ -569,6 +569,10 @@ int Engine::build(const std::vector<SceneSource> &src, const ArSimTuning *tuning
     N = (int)nTot;
     B = (int)bTot;
     sceneBits = S > 1 ? ceil_log2(S) : 0;
+    std::vector<SceneMeasure> known(S);
+    for (int s = 0; s < S; ++s)
+        if (src[s].from && (size_t)src[s].fromScene < src[s].from->measure.size())
+            known[s] = src[s].from->measure[src[s].fromScene];
     if (method == ARSIM_METHOD_GRID) {
         // scenes' cell ranges are packed back to back: key = cellBase[scene] + cell hash
         cellBits = maxCellBits;
@@ -581,8 +585,8 @@ int Engine::build(const std::vector<SceneSource> &src, const ArSimTuning *tuning
         segBits = keyBits > kExactTableBits ? keyBits - kExactTableBits : 0;
         numSegs = (long long)((numCells - 1) >> segBits) + 1;
         if (segBits == 0) {
-            // bucket widths from the particles of host scenes, kept for scenes carried over from an
-            // engine that planned them
+            // bucket widths from the particles of host scenes, kept with what was measured for scenes carried
+            // over from an engine that planned them
             std::vector<BucketSceneShape> shapes(S);
             for (int s = 0; s < S; ++s) {
                 shapes[s].particles = pCount[s];
@@ -591,14 +595,16 @@ int Engine::build(const std::vector<SceneSource> &src, const ArSimTuning *tuning
                     shapes[s].extent[a] = ((double)geoms[s].boxMax[a] - (double)geoms[s].boxMin[a]) /
                                           (double)geoms[s].cellSize[a];
                 }
-                double around = 0.0;
-                if (src[s].host) shapes[s].peak = bucket_peaks(src[s].host->pos, pCount[s], geoms[s], &shapes[s].load, &around);
-                else if (src[s].from) around = src[s].from->density;
-                density += around * ((double)pCount[s] / (double)std::max(N, 1));
+                SceneMeasure &m = known[s];
+                if (src[s].host) m.peak = bucket_peaks(src[s].host->pos, pCount[s], geoms[s], &m.load, &m.density);
+                shapes[s].peak.swap(m.peak);
+                shapes[s].load = m.load;
+                density += m.density * ((double)pCount[s] / (double)std::max(N, 1));
                 if (src[s].from && src[s].from->bucketSort)
                     shapes[s].shift = src[s].from->bkPlan.scenes[src[s].fromScene].shift;
             }
             bucketSort = plan_bucket_sort(shapes, &bkPlan);
+            for (int s = 0; s < S; ++s) known[s].peak.swap(shapes[s].peak);
             queueContacts = density >= (S > 1 ? kQueueDensityBatch : kQueueDensity);
             coopContacts = N <= (S > 1 ? kCoopMaxBatch : density >= kCoopDensity ? kCoopMaxDense : kCoopMax);
             useIndex = bucketSort && N > kIndexMin && (double)numCells >= kIndexCells * (double)N && !(flags & ARSIM_CONTACT_SIS) && !tu.fuseReduce;
@@ -634,14 +640,20 @@ int Engine::build(const std::vector<SceneSource> &src, const ArSimTuning *tuning
         for (int s = 0; s < S; ++s) {
             shapes[s].particles = pCount[s];
             shapes[s].grid[0] = shapes[s].grid[1] = shapes[s].grid[2] = 1024u;
+            SceneMeasure &m = known[s];
             if (src[s].host)
-                shapes[s].peak = morton_peaks(src[s].host->pos, pCount[s], geoms[s], m63 && N <= kTieParticles ? &ties : nullptr);
-            else if (src[s].from && src[s].from->mortonBucket)
+                m.peak = morton_peaks(src[s].host->pos, pCount[s], geoms[s], m63 && N <= kTieParticles ? &m.ties : nullptr);
+            shapes[s].peak.swap(m.peak);
+            ties = std::max(ties, m.ties);
+            if (src[s].from && src[s].from->mortonBucket)
                 shapes[s].shift = src[s].from->bkPlan.scenes[src[s].fromScene].shift;
         }
         mortonBucket = ties <= kMostTies &&
                        plan_bucket_sort(shapes, &bkPlan, 30, 4096, true, m63 ? kMostMorton63 : kMostMorton30);
+        for (int s = 0; s < S; ++s) known[s].peak.swap(shapes[s].peak);
     }
+
+    measure = std::move(known);
 
     // ---- allocation (everything a step touches, once)
     int rc = 0;

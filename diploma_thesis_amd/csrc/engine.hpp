@@ -62,7 +62,15 @@ struct Engine {
     unsigned char *keyBufA = nullptr, *keyBufB = nullptr, *sortWsBuf = nullptr;
     unsigned *valsA = nullptr, *valsB = nullptr;
     unsigned *segStart = nullptr;           // grid: CSR offsets over segments of 2^segBits cells
-    double density = 0.0;                   // grid: particles per cell around a particle, of the scenes as given
+    // What the plans were made from, per scene: measured when the scene came from the host, carried over with it
+    struct SceneMeasure {
+        std::vector<unsigned> peak;         // fullest bucket by width (BucketSceneShape)
+        double load = 0.0;                  // (BucketSceneShape)
+        double density = 0.0;               // grid: particles per cell around a particle
+        unsigned ties = 0u;                 // 63-bit codes: the most particles of one 30-bit code
+    };
+    std::vector<SceneMeasure> measure;
+    double density = 0.0;                   // grid: of all scenes, by particles
     bool coopContacts = false;              // grid: 16 lanes a particle (launch_dem_grid_seg)
     bool queueContacts = false;             // grid: contacts queued before they are evaluated (launch_dem_grid_seg)
     bool useIndex = false;                  // grid, bucket sort: the compact cell index instead (kernels.hpp)
