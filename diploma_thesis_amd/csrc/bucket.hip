@@ -28,10 +28,12 @@ constexpr int kBkWaves = kBkThreads / 64;
 constexpr int kBkCap = 7776;
 // Plans whose buckets are all small take workgroups of 256 threads: a bucket of 64 keys leaves 15 of 16 waves idle, and
 // every barrier and scan waits for them: the sort and reorder of 16,384 particles 18 -> 12 us (the step 39 -> 33), of
-// 65,000 19 -> 16, the codes of a forest of 40 scenes of 9,000 32 -> 21.
+// 65,000 19 -> 16, the codes of a forest of 40 scenes of 9,000 32 -> 21.  The measured peak leaves room for the particles to
+// move.  Where they crowd past it, the sort of 20,000 with a bucket of 1,068 takes 18 us (with 1024 threads 19.7), of 2,222
+// 24 (21), of 45,000 with one of 5,066 69 (28), of 65,000 with one of 7,192 96 (35): a bucket of more than
+// kBucketSmallMost keys sets to.outgrown, and the engine takes the workgroups of 1024 when it next learns of it.
 constexpr int kBkSmallThreads = 256;
 constexpr int kBkSmallCap = 3840;   // keys sorted in LDS
-constexpr unsigned kBkSmallPeak = 1024;   // of the fullest measured bucket: room for the particles to move
 constexpr int kBkMaxTiles = 384;  // tiles of one scene, which a bucket gathers from (2^20 keys: 256)
 constexpr int kBkLdsBytes = 2 * kBkCap * 4 + kBkWaves * 256 * 4 + kBkWaves * 4 + 2 * kBkMaxTiles * 4;
 static_assert(kBkLdsBytes <= 80 * 1024, "two bucket workgroups must fit in one CU's LDS");
@@ -216,6 +218,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(8))) vo
     const int cnt = (int)hist[j];
     constexpr unsigned kPosMask = (1u << POSBITS) - 1u;
     const bool inLds = cnt <= kCap;
+    if (THREADS == kBkSmallThreads && cnt > (int)kBucketSmallMost && t == 0 && to.outgrown) *to.outgrown = 1;
     // a bucket too large for LDS is sorted in global memory by its first workgroup alone
     if (!inLds && part != 0) return;
     const int nparts = inLds ? split : 1;
@@ -612,7 +615,7 @@ bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *o
             shift = sc.shift;
         if (shift < 0) return false;
         if (measured && sc.peak[shift] > mostKeys) return false;
-        if (!measured || sc.peak[shift] > kBkSmallPeak || tiles > kBkSmallThreads) p.small = false;
+        if (!measured || sc.peak[shift] > kBucketSmallPeak || tiles > kBkSmallThreads) p.small = false;
         BucketScene &b = p.scenes[s];
         b.pStart = (unsigned)pBase;
         b.n = (unsigned)n;

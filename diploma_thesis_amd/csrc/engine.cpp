@@ -156,6 +156,12 @@ int Engine::fetch(const std::vector<Fetch> &what) {
             if (f.bytes) ARSIM_HIP(hipMemcpy(f.dst, f.src, f.bytes, hipMemcpyDeviceToHost));
         return ARSIM_OK;
     }
+    const bool flag = jobs.n < kFetchMax && (words + 4) * 4 <= kFetchBytes;   // overflowD rides along
+    if (flag) {
+        jobs.src[jobs.n] = (const unsigned *)overflowD;
+        jobs.words[jobs.n] = 4u;
+        jobs.at[jobs.n++] = (unsigned)words;
+    }
     int current = device;
     ARSIM_HIP(hipGetDevice(&current));
     if (current != device) ARSIM_HIP(hipSetDevice(device));
@@ -174,9 +180,11 @@ int Engine::fetch(const std::vector<Fetch> &what) {
             if (e == hipSuccess && f.bytes) e = hipMemcpy(f.dst, f.src, f.bytes, hipMemcpyDeviceToHost);
     if (current != device) hipSetDevice(current);
     if (e != hipSuccess) return fail(ARSIM_ERR_HIP, std::string("engine read: ") + hipGetErrorString(e));
+    if (!fetchBuf) return ARSIM_OK;
     int k = 0;
     for (const Fetch &f : what)
-        if (fetchBuf && f.bytes) std::memcpy(f.dst, fetchBuf + jobs.at[k++], f.bytes);
+        if (f.bytes) std::memcpy(f.dst, fetchBuf + jobs.at[k++], f.bytes);
+    if (flag && fetchBuf[words + 1]) outgrown = true;
     return ARSIM_OK;
 }
 
@@ -826,7 +834,8 @@ int Engine::build(const std::vector<SceneSource> &src, const ArSimTuning *tuning
     ARSIM_HIP(hipMemcpyAsync(sceneStartD, hStart.data(), 4 * (size_t)S, hipMemcpyHostToDevice, st));
     ARSIM_HIP(hipMemcpyAsync(sceneCountD, hCount.data(), 4 * (size_t)S, hipMemcpyHostToDevice, st));
     if (tree.sceneRoot) launch_fill_u32((unsigned *)tree.sceneRoot, 0xffffffffu, (size_t)S, st);
-    launch_fill_u32((unsigned *)overflowD, 0u, 1, st);
+    launch_fill_u32((unsigned *)overflowD, 0u, 4, st);
+    outgrown = false;
     if (longCnt) launch_fill_u32(longCnt, 0u, 1, st);
     maxSceneBodies = 0;
     for (int s = 0; s < S; ++s) maxSceneBodies = std::max(maxSceneBodies, bCount[s]);
@@ -891,7 +900,7 @@ int Engine::enqueue_grid_broadphase(const BodyBufs &bb, const PartBufs &pb, cons
             rec();
         }
         const TileKeyOut to{(unsigned *)keysB, valsB, tileInfo, bucketHist, bkScenesD, tileSceneD, bucketSceneD,
-                            numTiles, numBuckets, tileKeys, bkPlan.bucketBits, bkPlan.small};
+                            numTiles, numBuckets, tileKeys, bkPlan.bucketBits, bkPlan.small, overflowD + 1};
         launch_pose_key_tiles(pb, ahead ? ahead_bufs() : bb, N, ph, sv, to, grainVelDead, st);
         rec();
         const int split = tu.bucketSplit == 1 || tu.bucketSplit == 2 ? tu.bucketSplit : (numBuckets < 512 ? 2 : 1);
@@ -1006,7 +1015,7 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
             rec();
         }
         TileKeyOut to{(unsigned *)keysB, valsB, tileInfo, bucketHist, bkScenesD, tileSceneD, bucketSceneD,
-                      numTiles, numBuckets, tileKeys, bkPlan.bucketBits, bkPlan.small};
+                      numTiles, numBuckets, tileKeys, bkPlan.bucketBits, bkPlan.small, overflowD + 1};
         const bool m63 = method == ARSIM_METHOD_LBVH63;
         to.morton = m63 ? 2 : 1;
         to.code63 = code63;
@@ -1103,6 +1112,12 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
 }
 
 int Engine::step(int n) {
+    if (bkPlan.small && outgrown.load()) {
+        bkPlan.small = false;
+        for (SceneMeasure &m : measure)   // (and for the engines that carry the scenes over)
+            for (unsigned &p : m.peak) p = std::max(p, kBucketSmallPeak + 1u);
+        invalidate_graph();
+    }
     if (n > 0 && integrate_ahead() && !primed)
         if (int rc = prime()) return rc;
     for (int i = 0; i < n; ++i) {
@@ -1241,10 +1256,11 @@ int arsim_engine_step(arsim_engine *e, int numSteps) {
 int arsim_engine_synchronize(arsim_engine *e) {
     if (!e) return fail(ARSIM_ERR_INVALID_ARG, "null engine");
     ARSIM_HIP(hipStreamSynchronize(e->e.st));
-    int ov = 0;
+    int ov[2] = {0, 0};
     if (e->e.overflowD) {
-        ARSIM_HIP(hipMemcpy(&ov, e->e.overflowD, 4, hipMemcpyDeviceToHost));
-        if (ov) return fail(ARSIM_ERR_OVERFLOW, "LBVH traversal stack overflow");
+        ARSIM_HIP(hipMemcpy(ov, e->e.overflowD, 8, hipMemcpyDeviceToHost));
+        if (ov[1]) e->e.outgrown = true;
+        if (ov[0]) return fail(ARSIM_ERR_OVERFLOW, "LBVH traversal stack overflow");
     }
     return ARSIM_OK;
 }

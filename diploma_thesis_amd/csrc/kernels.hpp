@@ -184,6 +184,7 @@ struct TileKeyOut {
     int numTiles, numBuckets, tileKeys;
     int bucketBits;                       // a scene has at most 2^bucketBits buckets (8, 9 or 10)
     bool small = false;                   // every bucket is small (the plan's)
+    int *outgrown = nullptr;              // with small: set where a bucket no longer is
     // Morton keys (each scene's codes cut into buckets of 2^shift, 20 <= shift <= 30): 1 = 30-bit codes;
     // 2 = 63-bit codes, whose top 30 bits (the 30-bit code) are the tile keys while the full codes go to
     // code63 in particle order
@@ -201,6 +202,10 @@ void launch_pose_key_tiles(const PartBufs &p, const BodyBufs &b, int numParticle
 // r = extent / grid size.  A scene that kept its shift from an earlier plan (a rebuild) passes it.
 // False when a scene needs more buckets than its tiles can rank or more than 384 tiles, and for grid keys where
 // the measured buckets are too full at every width.
+// Plans whose buckets all measured at most kBucketSmallPeak keys are sorted by workgroups of 256 threads (bucket.hip),
+// which say (TileKeyOut.outgrown) when one holds more than kBucketSmallMost: from about there on the workgroups of 1024 are
+// faster.
+constexpr unsigned kBucketSmallPeak = 1024, kBucketSmallMost = 2048;
 struct BucketSceneShape {
     long long particles = 0;
     unsigned grid[3] = {1, 1, 1};
