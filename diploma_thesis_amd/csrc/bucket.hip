@@ -218,7 +218,10 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(8))) vo
     const int cnt = (int)hist[j];
     constexpr unsigned kPosMask = (1u << POSBITS) - 1u;
     const bool inLds = cnt <= kCap;
-    if (THREADS == kBkSmallThreads && cnt > (int)kBucketSmallMost && t == 0 && to.outgrown) *to.outgrown = 1;
+    if (t == 0 && to.outgrown) {
+        if (THREADS == kBkSmallThreads && cnt > (int)kBucketSmallMost) to.outgrown[0] = to.bucketScene[g] + 1;
+        if (!REORDER && (unsigned)cnt > to.mostKeys) to.outgrown[1] = to.bucketScene[g] + 1;
+    }
     // a bucket too large for LDS is sorted in global memory by its first workgroup alone
     if (!inLds && part != 0) return;
     const int nparts = inLds ? split : 1;
@@ -488,7 +491,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(8))) vo
 constexpr int kTieStep = 8;
 __global__ void k_morton63_ties(const unsigned *__restrict__ k30, const unsigned *__restrict__ vIn,
                                 const uint64_t *__restrict__ code63, int n, uint64_t *__restrict__ kOut,
-                                unsigned *__restrict__ vOut) {
+                                unsigned *__restrict__ vOut, int *__restrict__ outgrown, int mostTies) {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= n) return;
     const unsigned c = k30[i];
@@ -523,6 +526,7 @@ __global__ void k_morton63_ties(const unsigned *__restrict__ k30, const unsigned
         }
         e = hi;
     }
+    if (i == a && e - a > mostTies && outgrown) outgrown[1] = 1;
     int rank = 0;
     for (int j = a; j < e; j += kTieStep) {
         uint64_t kj[kTieStep];
@@ -539,9 +543,10 @@ __global__ void k_morton63_ties(const unsigned *__restrict__ k30, const unsigned
 }  // namespace
 
 void launch_morton63_ties(const unsigned *k30, const unsigned *vIn, const uint64_t *code63, int n, uint64_t *kOut,
-                          unsigned *vOut, hipStream_t st) {
+                          unsigned *vOut, int *outgrown, int mostTies, hipStream_t st) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_morton63_ties, dim3((n + 255) / 256), dim3(256), 0, st, k30, vIn, code63, n, kOut, vOut);
+    hipLaunchKernelGGL(k_morton63_ties, dim3((n + 255) / 256), dim3(256), 0, st, k30, vIn, code63, n, kOut, vOut,
+                       outgrown, mostTies);
 }
 
 bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *out, int maxShift, int capKeys,

@@ -46,6 +46,7 @@ constexpr double kQueueDensity = 1.0, kQueueDensityBatch = 2.0;
 // Morton buckets past the LDS are sorted in global memory by one workgroup each, about 5 us per 1,000 keys, so scenes in
 // a small part of their Morton box take the onesweep passes: 8,000 particles in one bucket 51 us against 45 for
 // 30-bit codes and 53 against 89 for 63-bit ones, 16,000 90 and 93 against 46 and 91, 65,000 319 and 338 against 47 and 94.
+// Scenes that come to that later go over when the engine next learns of it (TileKeyOut.outgrown).
 constexpr unsigned kMostMorton30 = 7168u, kMostMorton63 = 14336u;
 // 63-bit codes that share their upper 30 bits are ranked among each other (k_morton63_ties), about 0.12 us for each of the
 // longest run, which up to 256 is less than the onesweep passes cost more (50 us): 300 to a code 52 us against 58, 1,000 140
@@ -184,7 +185,8 @@ int Engine::fetch(const std::vector<Fetch> &what) {
     int k = 0;
     for (const Fetch &f : what)
         if (f.bytes) std::memcpy(f.dst, fetchBuf + jobs.at[k++], f.bytes);
-    if (flag && fetchBuf[words + 1]) outgrown = true;
+    if (flag && fetchBuf[words + 1]) outgrown = (int)fetchBuf[words + 1];
+    if (flag && fetchBuf[words + 2]) overfull = (int)fetchBuf[words + 2];
     return ARSIM_OK;
 }
 
@@ -835,7 +837,7 @@ int Engine::build(const std::vector<SceneSource> &src, const ArSimTuning *tuning
     ARSIM_HIP(hipMemcpyAsync(sceneCountD, hCount.data(), 4 * (size_t)S, hipMemcpyHostToDevice, st));
     if (tree.sceneRoot) launch_fill_u32((unsigned *)tree.sceneRoot, 0xffffffffu, (size_t)S, st);
     launch_fill_u32((unsigned *)overflowD, 0u, 4, st);
-    outgrown = false;
+    outgrown = overfull = 0;
     if (longCnt) launch_fill_u32(longCnt, 0u, 1, st);
     maxSceneBodies = 0;
     for (int s = 0; s < S; ++s) maxSceneBodies = std::max(maxSceneBodies, bCount[s]);
@@ -1018,6 +1020,7 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
                       numTiles, numBuckets, tileKeys, bkPlan.bucketBits, bkPlan.small, overflowD + 1};
         const bool m63 = method == ARSIM_METHOD_LBVH63;
         to.morton = m63 ? 2 : 1;
+        to.mostKeys = m63 ? kMostMorton63 : kMostMorton30;
         to.code63 = code63;
         launch_pose_key_tiles(pb, ahead ? ahead_bufs() : bb, N, ph, sv, to, false, st);
         rec();
@@ -1035,7 +1038,8 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
         void *kS = keysA;
         unsigned *vS = valsA;
         if (m63) {
-            launch_morton63_ties((const unsigned *)keysA, valsA, code63, N, (uint64_t *)keysB, valsB, st);
+            launch_morton63_ties((const unsigned *)keysA, valsA, code63, N, (uint64_t *)keysB, valsB, overflowD + 1,
+                                 N <= kTieParticles ? (int)kMostTies : INT_MAX, st);
             kS = keysB;
             vS = valsB;
         }
@@ -1112,11 +1116,20 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
 }
 
 int Engine::step(int n) {
+    // buckets that outgrew the plan (also noted for the engines that carry the scene over)
+    auto outgrow = [&](int scene, unsigned peak) {
+        if ((size_t)scene <= measure.size())
+            for (unsigned &p : measure[scene - 1].peak) p = std::max(p, peak);
+        invalidate_graph();
+    };
     if (bkPlan.small && outgrown.load()) {
         bkPlan.small = false;
-        for (SceneMeasure &m : measure)   // (and for the engines that carry the scenes over)
-            for (unsigned &p : m.peak) p = std::max(p, kBucketSmallPeak + 1u);
-        invalidate_graph();
+        outgrow(outgrown.load(), kBucketSmallPeak + 1u);
+    }
+    if (mortonBucket && overfull.load()) {   // the onesweep passes from here on
+        mortonBucket = false;
+        primed = false;                      // (which integrate the bodies in the step itself)
+        outgrow(overfull.load(), 0xfffffffeu);
     }
     if (n > 0 && integrate_ahead() && !primed)
         if (int rc = prime()) return rc;
@@ -1256,10 +1269,11 @@ int arsim_engine_step(arsim_engine *e, int numSteps) {
 int arsim_engine_synchronize(arsim_engine *e) {
     if (!e) return fail(ARSIM_ERR_INVALID_ARG, "null engine");
     ARSIM_HIP(hipStreamSynchronize(e->e.st));
-    int ov[2] = {0, 0};
+    int ov[3] = {0, 0, 0};
     if (e->e.overflowD) {
-        ARSIM_HIP(hipMemcpy(ov, e->e.overflowD, 8, hipMemcpyDeviceToHost));
-        if (ov[1]) e->e.outgrown = true;
+        ARSIM_HIP(hipMemcpy(ov, e->e.overflowD, 12, hipMemcpyDeviceToHost));
+        if (ov[1]) e->e.outgrown = ov[1];
+        if (ov[2]) e->e.overfull = ov[2];
         if (ov[0]) return fail(ARSIM_ERR_OVERFLOW, "LBVH traversal stack overflow");
     }
     return ARSIM_OK;

@@ -101,7 +101,7 @@ struct Engine {
     float4 *aPos = nullptr, *aVel = nullptr, *aAng = nullptr, *aQinc = nullptr, *aQcum = nullptr;
     float *aIw = nullptr;
     uint64_t *code63 = nullptr;     // LBVH63 bucket path: the 63-bit codes in particle order
-    int *overflowD = nullptr, *flagD = nullptr;   // overflowD[1]: a bucket outgrew the small workgroups (kernels.hpp)
+    int *overflowD = nullptr, *flagD = nullptr;   // overflowD[1], [2]: TileKeyOut.outgrown
     float4 *aabbPart = nullptr, *aabbBox = nullptr;
     // static collider set (one-scene engines): points and normals sorted by cell, exact cell table
     int numStatic = 0;
@@ -130,8 +130,8 @@ struct Engine {
     // pinned host memory that small reads of the state come through (allocated at the first one), one read at a time
     unsigned *fetchBuf = nullptr;
     std::mutex fetchLock;
-    // overflowD[1] as last read, by a small read of the state or a synchronize; the next step acts on it
-    std::atomic<bool> outgrown{false};
+    // overflowD[1] and [2] as last read, by a small read of the state or a synchronize; the next step acts on them
+    std::atomic<int> outgrown{0}, overfull{0};
     struct Fetch {
         void *dst;
         const void *src;

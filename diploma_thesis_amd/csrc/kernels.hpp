@@ -184,7 +184,10 @@ struct TileKeyOut {
     int numTiles, numBuckets, tileKeys;
     int bucketBits;                       // a scene has at most 2^bucketBits buckets (8, 9 or 10)
     bool small = false;                   // every bucket is small (the plan's)
-    int *outgrown = nullptr;              // with small: set where a bucket no longer is
+    // set to a scene + 1: outgrown[0] (with small) where a bucket of it no longer is small, [1] where one holds more
+    // than mostKeys
+    int *outgrown = nullptr;
+    unsigned mostKeys = 0xffffffffu;
     // Morton keys (each scene's codes cut into buckets of 2^shift, 20 <= shift <= 30): 1 = 30-bit codes;
     // 2 = 63-bit codes, whose top 30 bits (the 30-bit code) are the tile keys while the full codes go to
     // code63 in particle order
@@ -247,8 +250,9 @@ void launch_bucket_sort(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, co
 // vIn the sorted top 30 bits and particle indices.  Writes the sorted 63-bit codes and indices; within
 // a run of equal top bits the members are ranked by their full codes, equal codes keeping the run's
 // (particle) order, so the result is the stable sort by the 63-bit code.
+// outgrown[1] is set (TileKeyOut) where a run is longer than mostTies.
 void launch_morton63_ties(const unsigned *k30, const unsigned *vIn, const uint64_t *code63, int n, uint64_t *kOut,
-                          unsigned *vOut, hipStream_t st);
+                          unsigned *vOut, int *outgrown, int mostTies, hipStream_t st);
 // The same for 30-bit Morton keys ranked per tile by bucket (TileKeyOut.morton): each bucket of up to 4,096
 // keys sorted by its low bits in LDS (maxShift: the widest scene's), written as sorted keys and indices
 // only; a larger bucket is sorted in global memory with scratchA / scratchB (16 B per key, N entries) as

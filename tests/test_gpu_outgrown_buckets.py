@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import oracle
-from diploma_thesis_amd import Engine, capi
+from diploma_thesis_amd import Engine, capi, scenes
 from test_gpu_engine import assert_state_equal
 from test_gpu_small_buckets import METHODS, gathered
 
@@ -28,12 +28,13 @@ def test_outgrown_vs_oracle(method, learn):
         assert_state_equal(e.download(), st, "outgrown")
 
 
-def test_outgrown_then_rebuilt():
-    print("outgrown buckets: rebuild", flush=True)
-    sc = gathered(20000, 14, capi.METHOD_GRID)
+@pytest.mark.parametrize("method", METHODS, ids=["grid", "lbvh30", "lbvh63"])
+def test_outgrown_then_rebuilt(method):
+    print(f"outgrown buckets: rebuild, method {method}", flush=True)
+    sc = gathered(20000, 14, method)
     st = oracle.State(sc, np.float32)
     st.step(4)
-    with Engine(sc) as e, Engine(gathered(300, 2, capi.METHOD_GRID)) as other:
+    with Engine(sc) as e, Engine(gathered(300, 2, method)) as other:
         e.step(1)
         e.sync()
         e.step(1)
@@ -42,3 +43,31 @@ def test_outgrown_then_rebuilt():
         other.sync()
         other.step(1)
         assert_state_equal(other.download(), st, "carried")
+
+
+@pytest.mark.parametrize("method", [capi.METHOD_LBVH30, capi.METHOD_LBVH63], ids=["lbvh30", "lbvh63"])
+@pytest.mark.parametrize("n,size", [(30000, 6.0), (3000, 1e-3)], ids=["bucket", "codes"])
+def test_overfull_morton_buckets(method, n, size):
+    """Bodies that gather in one Morton bucket, or under one 30-bit code, after a scattered start: from the step
+    after the read on the codes are sorted by digit passes."""
+    print(f"outgrown buckets: {n} particles gather in {size}, method {method}", flush=True)
+    sc = scenes.mix_scene(n, 15, method).copy()
+    sc.rb_pos[:, :3] = 20.0 + np.random.default_rng(n).uniform(0, size, (sc.b, 3))
+    for a in range(3):
+        sc.cfg.boxMax[a] = 4096.0
+    sc.cfg.wallMask = 0
+    grains = sc.rb < 0
+    sc.pos[:, :3] = np.random.default_rng(1).uniform(0, 4096.0, (sc.n, 3))   # (the bodies' own are posed from them)
+    sc.vel[grains, :3] = 0.0
+    st = oracle.State(sc, np.float32)
+    with Engine(sc) as e:
+        before = [name for name, _ in e.profile()]
+        e.step(2)
+        e.render_state(0)
+        e.step(1)
+        e.sync()
+        after = [name for name, _ in e.profile()]
+        st.step(5)
+        assert_state_equal(e.download(), st, "overfull")
+    if n == 30000 or method == capi.METHOD_LBVH63:
+        assert before != after
