@@ -376,7 +376,7 @@ int arsim_dem_lbvh(const int *rbIndices, float *pForce, float *pTorque, float *v
     DemOut o{};
     o.pForce = (float4 *)pForce; o.pTorque = (float4 *)pTorque; o.vel = (float4 *)vel;
     o.relPos = (const float4 *)relativePos;
-    launch_dem_lbvh(sortedIndices, t, n, make_phys(*params, *cfg), sv, false, o, 128, S(st), overflowFlag);
+    launch_dem_lbvh(sortedIndices, t, n, make_phys(*params, *cfg), sv, o, 128, S(st), overflowFlag);
     return check_launch("dem_lbvh");
 }
 
@@ -425,7 +425,7 @@ int arsim_contact_pairs_lbvh(const int *rbIndices, const int *sortedIndices, con
     t.sortedVel = (float4 *)CMs;   // not read in pair mode beyond w
     DemOut o{};
     o.pairs = pairs; o.counts = counts; o.maxPer = maxPer;
-    launch_dem_lbvh(sortedIndices, t, n, make_phys(*params, cfg), sv, false, o, 128, S(st), overflowFlag);
+    launch_dem_lbvh(sortedIndices, t, n, make_phys(*params, cfg), sv, o, 128, S(st), overflowFlag);
     return check_launch("contact_pairs_lbvh");
 }
 

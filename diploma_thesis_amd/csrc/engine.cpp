@@ -34,7 +34,9 @@ namespace {
 // saves writing four bytes a cell and most of the table's reads, and costs each particle about a fifth
 // more instructions: 20 scenes of 65,536 particles (4 cells a particle) step 204 -> 221 us with it,
 // 40 of 32,768 (8) 197 -> 203, 50 of 24,000 (11) 183 -> 179, 60 of 16,384 (16) 144 -> 134, the
-// 2^20-particle scene (16) 148 -> 136.
+// 2^20-particle scene (16) 148 -> 136.  Like the queue below it is chosen from the first positions and kept: that scene
+// falling until it has settled (28,000 steps of 0.5 ms) goes 135 -> 256 us a step with the index, 148 -> 261 with the
+// table, and the settled state planned anew takes 266.
 constexpr double kIndexCells = 10.0;
 constexpr int kIndexMin = 3 << 16;   // and more particles than this
 // Contacts are queued before they are evaluated (launch_dem_grid_seg) where the particles lie as densely as this: in
@@ -1050,7 +1052,7 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
         rec();
         DemOut o{};
         o.pForce = pForce; o.vel = vel; o.relPos = relPos;
-        launch_dem_lbvh((const int *)vS, tree, N, ph, sv, S > 1, o, tu.demBlock, st, overflowD);
+        launch_dem_lbvh((const int *)vS, tree, N, ph, sv, o, tu.demBlock, st, overflowD);
         if (numStatic)
             launch_dem_static(tree.cms, tree.sortedVel, vS, N, stPos, stNorm, nullptr, stTable, nullptr, ph,
                               geoms[0], pForce, nullptr, relPos, false, st);
@@ -1100,7 +1102,7 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
         rec();
         DemOut o{};
         o.pForce = pForce; o.vel = vel; o.relPos = relPos;
-        launch_dem_lbvh((const int *)vA, tree, N, ph, sv, S > 1, o, tu.demBlock, st, overflowD);
+        launch_dem_lbvh((const int *)vA, tree, N, ph, sv, o, tu.demBlock, st, overflowD);
         if (numStatic)
             launch_dem_static(tree.cms, tree.sortedVel, vA, N, stPos, stNorm, nullptr, stTable, nullptr, ph,
                               geoms[0], pForce, nullptr, relPos, false, st);
@@ -1204,7 +1206,7 @@ int Engine::enqueue_broadphase(int *pairsD, int *countsD, int maxPer) {
         }
         launch_lbvh_build(sortedKeys, keyBytes, N, S > 1 ? 30 : 0, sceneStartD, sceneCountD, S, tree, st);
         launch_lbvh_refit((const int *)vA, pos, vel, rb, S > 1 ? scene : nullptr, gatherRec, ph.r, N, tree, st);
-        launch_dem_lbvh((const int *)vA, tree, N, ph, sv, S > 1, o, tu.demBlock, st, overflowD);
+        launch_dem_lbvh((const int *)vA, tree, N, ph, sv, o, tu.demBlock, st, overflowD);
         lastKeys = sortedKeys;
         lastIdx = vA;
     }

@@ -175,7 +175,7 @@ struct BucketScene {
 // body.hip): the tile's keys and particle indices in bucket order (stable), info[infoBase + j * tiles
 // + k] = count << 16 | first slot of bucket j in the scene's tile k, and every bucket's count
 // accumulated into hist[bucketBase + j] (zeroed beforehand).  Tiles hold tileKeys particles: 4096
-// (kTileKeys), or 1024 where tiles of 4096 would be too few to fill the GPU or scenes are small.
+// (kTileKeys), 512 for few particles or 1024 where scenes are small (plan_bucket_sort).
 constexpr int kTileKeys = 4096;
 struct TileKeyOut {
     unsigned *keys, *vals, *info, *hist;
@@ -196,6 +196,10 @@ struct TileKeyOut {
 };
 void launch_pose_key_tiles(const PartBufs &p, const BodyBufs &b, int numParticles, const DevPhys &ph,
                            const SceneView &sv, const TileKeyOut &to, bool grainVelDead, hipStream_t st);
+// Plans whose buckets all measured at most kBucketSmallPeak keys are sorted by workgroups of 256 threads (bucket.hip),
+// which say (TileKeyOut.outgrown) when one holds more than kBucketSmallMost: from about there on the workgroups of 1024 are
+// faster.
+constexpr unsigned kBucketSmallPeak = 1024, kBucketSmallMost = 2048;
 // The host side of the plan: tiles of `tileKeys` particles, and per scene the widest shift whose
 // buckets fit in LDS.  A scene is described by its particle count, its grid (cells per axis), and
 // either the fullest bucket measured on its particles for every shift (peak[b], b = 0..16), or the
@@ -205,10 +209,6 @@ void launch_pose_key_tiles(const PartBufs &p, const BodyBufs &b, int numParticle
 // r = extent / grid size.  A scene that kept its shift from an earlier plan (a rebuild) passes it.
 // False when a scene needs more buckets than its tiles can rank or more than 384 tiles, and for grid keys where
 // the measured buckets are too full at every width.
-// Plans whose buckets all measured at most kBucketSmallPeak keys are sorted by workgroups of 256 threads (bucket.hip),
-// which say (TileKeyOut.outgrown) when one holds more than kBucketSmallMost: from about there on the workgroups of 1024 are
-// faster.
-constexpr unsigned kBucketSmallPeak = 1024, kBucketSmallMost = 2048;
 struct BucketSceneShape {
     long long particles = 0;
     unsigned grid[3] = {1, 1, 1};
@@ -226,15 +226,10 @@ struct BucketPlan {
     int bucketBits = 8;   // the most buckets of one scene, rounded up to a power of two (at least 2^8)
 };
 // maxShift / capKeys: the widest bucket (2^maxShift cells) and the most keys a bucket sorted in LDS holds
-// (grid keys: 2^16 and 7,776; Morton keys: 2^30 and 4,096).  sharedCells: every scene's keys lie in the same range (Morton codes) instead of one
-// scene's after another's.  mostKeys: no plan where a measured bucket would hold more.
+// (grid keys: 2^16 and 7,776; Morton keys: 2^30 and 4,096).  sharedCells: every scene's keys lie in the same range
+// (Morton codes) instead of one scene's after another's.  mostKeys: no plan where a measured bucket would hold more.
 bool plan_bucket_sort(const std::vector<BucketSceneShape> &shapes, BucketPlan *out, int maxShift = 16,
                       int capKeys = 7776, bool sharedCells = false, unsigned mostKeys = 0xffffffffu);
-// The grid sort finished per bucket (bucket.hip): each bucket gathers its keys from its scene's
-// tiles' runs (tile order keeps the sort stable), `split` workgroups (1 or 2) sort it by the low bits,
-// each writing its share of the sorted keys / indices to (kOut, vOut), of the gathered sorted copies
-// and of the bucket's range of the exact cell table (whose last entry, numCells, the last bucket writes).
-// ix (words set): the compact cell index instead of the table.
 // Compact cell index: words[c / 32] = (a bit per occupied cell of the 32, slot of the first of them in starts);
 // starts lists, per bucket from the bucket's first sorted position on, where its occupied cells start, and then
 // the bucket's end.  A row of three cells is one 16-byte load of two words and, unless it is empty, one of
@@ -243,9 +238,20 @@ struct CellIndex {
     uint2 *words = nullptr;      // cells / 32 entries and one more
     unsigned *starts = nullptr;  // N + 4 entries
 };
+// The grid sort finished per bucket (bucket.hip): each bucket gathers its keys from its scene's
+// tiles' runs (tile order keeps the sort stable), `split` workgroups (1 or 2) sort it by the low bits,
+// each writing its share of the sorted keys / indices to (kOut, vOut), of the gathered sorted copies
+// and of the bucket's range of the exact cell table (whose last entry, numCells, the last bucket writes).
+// ix (words set): the compact cell index instead of the table.
 void launch_bucket_sort(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, const float4 *rec, float4 *sortedPos,
                         float4 *sortedVel, unsigned *table, unsigned numCells, int split, const CellIndex &ix,
                         hipStream_t st);
+// The same for 30-bit Morton keys ranked per tile by bucket (TileKeyOut.morton): each bucket of up to 4,096
+// keys sorted by its low bits in LDS (maxShift: the widest scene's), written as sorted keys and indices
+// only; a larger bucket is sorted in global memory with scratchA / scratchB (16 B per key, N entries) as
+// its second buffer.  kOut64 (a forest): the keys as scene << 30 | code there, kOut being scratch.
+void launch_bucket_sort_morton(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, float4 *scratchA,
+                               float4 *scratchB, uint64_t *kOut64, int maxShift, hipStream_t st);
 // The 63-bit order from the stable sort by the codes' top 30 bits: code63 is in particle order, k30 /
 // vIn the sorted top 30 bits and particle indices.  Writes the sorted 63-bit codes and indices; within
 // a run of equal top bits the members are ranked by their full codes, equal codes keeping the run's
@@ -253,12 +259,6 @@ void launch_bucket_sort(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, co
 // outgrown[1] is set (TileKeyOut) where a run is longer than mostTies.
 void launch_morton63_ties(const unsigned *k30, const unsigned *vIn, const uint64_t *code63, int n, uint64_t *kOut,
                           unsigned *vOut, int *outgrown, int mostTies, hipStream_t st);
-// The same for 30-bit Morton keys ranked per tile by bucket (TileKeyOut.morton): each bucket of up to 4,096
-// keys sorted by its low bits in LDS (maxShift: the widest scene's), written as sorted keys and indices
-// only; a larger bucket is sorted in global memory with scratchA / scratchB (16 B per key, N entries) as
-// its second buffer.  kOut64 (a forest): the keys as scene << 30 | code there, kOut being scratch.
-void launch_bucket_sort_morton(const TileKeyOut &to, unsigned *kOut, unsigned *vOut, float4 *scratchA,
-                               float4 *scratchB, uint64_t *kOut64, int maxShift, hipStream_t st);
 // Capacity of the long-run list of a table of tableSize entries (runs are disjoint and longer than
 // kLongRange), and the launch that fills the listed runs.
 unsigned fill_long_capacity(unsigned long long tableSize);
@@ -328,9 +328,9 @@ void launch_lbvh_refit(const int *sortedIdx, const float4 *pos, const float4 *ve
 // Fills t.bounds (2 float4 per node) from the leaf centres (box = centre -/+ radius) and the packed
 // traversal records of a range refit that ran without bounds.
 void launch_lbvh_bounds(const Lbvh &t, int n, float radius, hipStream_t st);
-// overflow: device int set to 1 when a traversal stack would exceed its LDS depth.
+// overflow: device int set to 1 when a packet's list of nodes would exceed its LDS.
 void launch_dem_lbvh(const int *sortedIdx, const Lbvh &t, int n, const DevPhys &ph, const SceneView &sv,
-                     bool sceneInVelW, const DemOut &o, int block, hipStream_t st, int *overflow);
+                     const DemOut &o, int block, hipStream_t st, int *overflow);
 
 // ---------------------------------------------------------------- static collider set (static.hip)
 struct RangeCamera {

@@ -952,8 +952,7 @@ void launch_lbvh_bounds(const Lbvh &t, int n, float radius, hipStream_t st) {
 }
 
 void launch_dem_lbvh(const int *sortedIdx, const Lbvh &t, int n, const DevPhys &ph, const SceneView &sv,
-                     bool sceneInVelW, const DemOut &o, int block, hipStream_t st, int *overflow) {
-    (void)sceneInVelW;
+                     const DemOut &o, int block, hipStream_t st, int *overflow) {
     if (n <= 0) return;
     if (block <= 0) block = 128;
     block = (block + 63) & ~63;
