@@ -48,13 +48,19 @@ constexpr double kQueueDensity = 1.0, kQueueDensityBatch = 2.0;
 // Morton buckets past the LDS are sorted in global memory by one workgroup each, about 5 us per 1,000 keys, so scenes in
 // a small part of their Morton box take the onesweep passes: 8,000 particles in one bucket 51 us against 45 for
 // 30-bit codes and 53 against 89 for 63-bit ones, 16,000 90 and 93 against 46 and 91, 65,000 319 and 338 against 47 and 94.
-// Scenes that come to that later go over when the engine next learns of it (TileKeyOut.outgrown).
+// Scenes that come to that later go over when the engine next learns of it (TileKeyOut.outgrown).  Looked at up to
+// kCrowdParticles and in forests.  One larger scene keeps the buckets at any load: a settled pile of 838,861 particles
+// has 4,170 keys in its fullest; 200,000 particles in 1/64 of their box take 215 us a step, and 181 by the passes.
 constexpr unsigned kMostMorton30 = 7168u, kMostMorton63 = 14336u;
 // 63-bit codes that share their upper 30 bits are ranked among each other (k_morton63_ties), about 0.12 us for each of the
 // longest run, which up to 256 is less than the onesweep passes cost more (50 us): 300 to a code 52 us against 58, 1,000 140
-// against 67.  Looked for up to kTieParticles, while the count's table stays in the host's cache.
+// against 67.  Looked for up to kCrowdParticles, while the count's table stays in the host's cache.
 constexpr unsigned kMostTies = 256u;
-constexpr int kTieParticles = 1 << 16;
+constexpr int kCrowdParticles = 1 << 16;
+unsigned most_morton_keys(bool m63, int n, int scenes) {
+    if (scenes == 1 && n > kCrowdParticles) return 0xffffffffu;
+    return m63 ? kMostMorton63 : kMostMorton30;
+}
 
 int ceil_log2(long long v) {
     int b = 0;
@@ -654,14 +660,14 @@ int Engine::build(const std::vector<SceneSource> &src, const ArSimTuning *tuning
             shapes[s].grid[0] = shapes[s].grid[1] = shapes[s].grid[2] = 1024u;
             SceneMeasure &m = known[s];
             if (src[s].host)
-                m.peak = morton_peaks(src[s].host->pos, pCount[s], geoms[s], m63 && N <= kTieParticles ? &m.ties : nullptr);
+                m.peak = morton_peaks(src[s].host->pos, pCount[s], geoms[s], m63 && N <= kCrowdParticles ? &m.ties : nullptr);
             shapes[s].peak.swap(m.peak);
             ties = std::max(ties, m.ties);
             if (src[s].from && src[s].from->mortonBucket)
                 shapes[s].shift = src[s].from->bkPlan.scenes[src[s].fromScene].shift;
         }
         mortonBucket = ties <= kMostTies &&
-                       plan_bucket_sort(shapes, &bkPlan, 30, 4096, true, m63 ? kMostMorton63 : kMostMorton30);
+                       plan_bucket_sort(shapes, &bkPlan, 30, 4096, true, most_morton_keys(m63, N, S));
         for (int s = 0; s < S; ++s) known[s].peak.swap(shapes[s].peak);
     }
 
@@ -1022,7 +1028,7 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
                       numTiles, numBuckets, tileKeys, bkPlan.bucketBits, bkPlan.small, overflowD + 1};
         const bool m63 = method == ARSIM_METHOD_LBVH63;
         to.morton = m63 ? 2 : 1;
-        to.mostKeys = m63 ? kMostMorton63 : kMostMorton30;
+        to.mostKeys = most_morton_keys(m63, N, S);
         to.code63 = code63;
         launch_pose_key_tiles(pb, ahead ? ahead_bufs() : bb, N, ph, sv, to, false, st);
         rec();
@@ -1041,7 +1047,7 @@ int Engine::enqueue_step(hipEvent_t *ev, int *numStages) {
         unsigned *vS = valsA;
         if (m63) {
             launch_morton63_ties((const unsigned *)keysA, valsA, code63, N, (uint64_t *)keysB, valsB, overflowD + 1,
-                                 N <= kTieParticles ? (int)kMostTies : INT_MAX, st);
+                                 N <= kCrowdParticles ? (int)kMostTies : INT_MAX, st);
             kS = keysB;
             vS = valsB;
         }
