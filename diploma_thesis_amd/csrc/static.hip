@@ -96,42 +96,84 @@ __global__ void k_static_reorder(const unsigned *__restrict__ keys, const unsign
 //  engine: the exact static cell table and sorted normals, body particles only: pForce += F (the
 //    torque is relativePos x pForce, formed by the reduction).
 // A workgroup first tests its particles one per thread for any candidate (the 9 rows of cells, three
-// consecutive cells each), then takes those that have some 16 lanes each (coop_cells): the walk of a
-// particle on a scanned surface, about a thousand candidates, was one serial chain per thread, bound by
-// the latency of its loads.  16,384 particles on the points of a 640 x 480 depth image: 1,280 -> 97 us;
+// consecutive cells each), then takes those that have some 16 lanes each (coop_cells) or, where that is the longer way,
+// one thread each: the walk of a particle on a scanned surface, about a thousand candidates, is one serial chain per
+// thread, bound by the latency of its loads.  16,384 particles on the points of a 640 x 480 depth image: 1,280 -> 97 us;
 // a 2^20-particle scene over a floor of 2^20 points (few particles near it): step 286 -> 210 us.  Without
 // the first test every particle takes 16 lanes, and that scene over 65,536 points costs 240 us a step
 // instead of 187 (one thread per particle: 213).
 constexpr int kStaticBlock = 128;
-template <bool REF>
+// Whether `count` particles of a workgroup with `candidates` of theirs in all take one thread each.  With 16 lanes eight at a
+// time do, each in a time that grows with a 16th of the candidates; with one thread all of them at once.  (The numbers are
+// a fit of both forms, 10^3 to 10^6 particles on points 1/50 of a cell to a cell apart.)  Every particle near the points, one
+// thread each, 16 lanes each, and weighed (us): 10^6 and 9 points a particle 116, 260, 109; 36 points 201, 406, 183; 900
+// points on a 16th of the scene 781, 1,482, 777; 200,000 and 9 points 37, 70, 37; 36 points 79, 104, 69; 900 points 773, 438, 504.
+__device__ __forceinline__ bool one_thread_each(int count, unsigned candidates) {
+    const long long rounds = (count + kStaticBlock / kCoopLanes - 1) / (kStaticBlock / kCoopLanes);
+    return rounds * (47ll * count + candidates) > 75ll * count + 7ll * candidates;
+}
+// WEIGH: both forms are weighed (launch_dem_static), else 16 lanes each.
+template <bool REF, bool WEIGH>
 __global__ __launch_bounds__(kStaticBlock) void k_dem_static(
     const float4 *__restrict__ sPos, const float4 *__restrict__ sVel, const unsigned *__restrict__ sIdx, int n,
-    int perBlock, const float4 *__restrict__ stPos, const float4 *__restrict__ stNorm,
+    int perBlock, int byXcd, const float4 *__restrict__ stPos, const float4 *__restrict__ stNorm,
     const unsigned *__restrict__ stIdx, const unsigned *__restrict__ cs, const unsigned *__restrict__ ce, DevPhys ph,
     SceneGeom g, float4 *__restrict__ pForce, float4 *__restrict__ pTorque, const float4 *__restrict__ relPos) {
     __shared__ CoopGroupLds sGroup[kStaticBlock / kCoopLanes];
     __shared__ int sList[kStaticBlock];
     __shared__ int sCount;
-    const int t = (int)threadIdx.x, first = xcd_block((int)blockIdx.x, (int)gridDim.x) * perBlock;
-    if (t == 0) sCount = 0;
+    __shared__ unsigned sCand;
+    const int t = (int)threadIdx.x,
+              first = (byXcd ? xcd_block((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x) * perBlock;
+    // cell h's run of candidates
+    auto cell_run = [&](unsigned h, unsigned &b, unsigned &e) {
+        b = cs[h];
+        if (!REF) e = cs[h + 1];
+        else if (b == kEmpty || (e = ce[h]) < b) b = e = 0u;   // an empty cell's end is not defined
+    };
+    if (t == 0) {
+        sCount = 0;
+        sCand = 0u;
+    }
     __syncthreads();
+    unsigned rows = 0u;   // of this thread's particle: those that have candidates
     if (t < perBlock && first + t < n) {
         const float4 P = sPos[first + t];
-        bool some = false;
+        unsigned cand = 0u;
         if (REF || __float_as_int(P.w) >= 0) {
             int gx, gy, gz;
             grid_pos(xyz(P), g, gx, gy, gz);
+            constexpr unsigned kMost = 4096u;   // (counted of one row or cell, so that the sum fits)
+            unsigned cells = 0u, at = 0u;
             for (int r = 0; r < 9; ++r) {
                 const unsigned h0 = grid_hash(gx - 1, gy + r % 3 - 1, gz + r / 3 - 1, g);
                 const unsigned h1 = grid_hash(gx, gy + r % 3 - 1, gz + r / 3 - 1, g);
                 const unsigned h2 = grid_hash(gx + 1, gy + r % 3 - 1, gz + r / 3 - 1, g);
-                if (REF) some = some | (cs[h0] != kEmpty) | (cs[h1] != kEmpty) | (cs[h2] != kEmpty);
-                else if (h2 == h0 + 2u) some = some | (cs[h0] != cs[h0 + 3u]);
-                else some = some | (cs[h0] != cs[h0 + 1u]) | (cs[h1] != cs[h1 + 1u]) | (cs[h2] != cs[h2 + 1u]);
+                unsigned some;
+                if (REF) {
+                    const unsigned c0 = cs[h0], c1 = cs[h1], c2 = cs[h2];
+                    some = (c0 != kEmpty ? 1u : 0u) + (c1 != kEmpty ? 1u : 0u) + (c2 != kEmpty ? 1u : 0u);
+                    at = c0 != kEmpty ? h0 : c1 != kEmpty ? h1 : c2 != kEmpty ? h2 : at;
+                    cells += some;
+                } else {
+                    if (h2 == h0 + 2u) some = min(cs[h0 + 3u] - cs[h0], kMost);
+                    else
+                        some = min(cs[h0 + 1u] - cs[h0], kMost) + min(cs[h1 + 1u] - cs[h1], kMost) +
+                               min(cs[h2 + 1u] - cs[h2], kMost);
+                    cand += some;
+                }
+                rows |= some ? 1u << r : 0u;
+            }
+            if (REF && WEIGH && cells) {   // estimated: every cell as full as one of them
+                unsigned b, e;
+                cell_run(at, b, e);
+                cand = cells * max(min(e - b, kMost), 1u);
             }
         }
-        if (some) sList[atomicAdd(&sCount, 1)] = first + t;   // (each particle is written by itself: any order)
-        else if (REF) {   // nothing to add: a sum of no contacts is +0
+        if (rows) {   // (each particle is written by itself: any order)
+            sList[atomicAdd(&sCount, 1)] = first + t;
+            if (WEIGH) atomicAdd(&sCand, cand);
+        } else if (REF) {   // nothing to add: a sum of no contacts is +0
             const unsigned o = sIdx[first + t];
             const float4 f = pForce[o], q = pTorque[o];
             const f3 tq = cross3(xyz(relPos[o]), mk3(0.f, 0.f, 0.f));
@@ -140,6 +182,37 @@ __global__ __launch_bounds__(kStaticBlock) void k_dem_static(
         }
     }
     __syncthreads();
+    if (WEIGH && one_thread_each(sCount, sCand)) {
+        if (!rows) return;
+        const int i = first + t;
+        const f3 pa = xyz(sPos[i]), va = xyz(sVel[i]);
+        int gx, gy, gz;
+        grid_pos(pa, g, gx, gy, gz);
+        f3 F = mk3(0.f, 0.f, 0.f);
+        for (; rows; rows &= rows - 1u) {   // (the others have no contact to add)
+            const int r = __builtin_ctz(rows);
+            for (int x = -1; x <= 1; ++x) {
+                unsigned j, e;
+                cell_run(grid_hash(gx + x, gy + r % 3 - 1, gz + r / 3 - 1, g), j, e);
+                f3 csum = mk3(0.f, 0.f, 0.f);
+                for (; j < e; ++j) {   // (a candidate's normal is read with its position, not after it)
+                    const f3 ps = xyz(stPos[j]), ns = xyz(stNorm[REF ? stIdx[j] : j]);
+                    f3 fj;
+                    if (static_force(pa, ps, ns, va, ph, fj)) csum = add3(csum, fj);
+                }
+                F = add3(F, csum);
+            }
+        }
+        const unsigned o = sIdx[i];
+        const float4 old = pForce[o];
+        pForce[o] = make_float4(old.x + F.x, old.y + F.y, old.z + F.z, old.w + 0.0f);
+        if (REF) {
+            const float4 q = pTorque[o];
+            const f3 tq = cross3(xyz(relPos[o]), F);
+            pTorque[o] = make_float4(q.x + tq.x, q.y + tq.y, q.z + tq.z, q.w + 0.0f);
+        }
+        return;
+    }
     const int count = sCount, gl = t / kCoopLanes, l = t & (kCoopLanes - 1);
     // (a wave's four groups stay together: the bound is the wave's, not the group's)
     for (int k0 = (t >> 6) * (64 / kCoopLanes); k0 < count; k0 += kStaticBlock / kCoopLanes) {
@@ -152,10 +225,7 @@ __global__ __launch_bounds__(kStaticBlock) void k_dem_static(
         const float F = coop_cells(
             sGroup[gl], valid,
             [&](int c, unsigned &b, unsigned &e) {
-                const unsigned h = grid_hash(gx + c % 3 - 1, gy + (c / 3) % 3 - 1, gz + c / 9 - 1, g);
-                b = cs[h];
-                e = REF ? ce[h] : cs[h + 1];
-                if (REF && (b == kEmpty || e < b)) b = e = 0u;   // an empty cell's end is not defined
+                cell_run(grid_hash(gx + c % 3 - 1, gy + (c / 3) % 3 - 1, gz + c / 9 - 1, g), b, e);
             },
             [&](unsigned j, f3 &f) {
                 const f3 ps = xyz(stPos[j]);
@@ -206,19 +276,21 @@ void launch_dem_static(const float4 *sPos, const float4 *sVel, const unsigned *s
                        const DevPhys &ph, const SceneGeom &g, float4 *pForce, float4 *pTorque,
                        const float4 *relPos, bool refLayout, hipStream_t st) {
     if (n <= 0) return;
-    // particles per workgroup: one per group of 16 lanes up to 8,192 workgroups (32 a CU: the particles near a
-    // surface, few and together, spread over the chip), then more, up to one per thread
-    const int groups = kStaticBlock / kCoopLanes;
-    int perBlock = (n + 8191) / 8192;
-    if (perBlock < groups) perBlock = groups;
-    if (perBlock > kStaticBlock) perBlock = kStaticBlock;
+    // Up to 65,536 particles a workgroup takes one per group of 16 lanes, so that the particles near a surface, few and
+    // together, spread over the chip.  More of them load the chip either way, and then the two forms are weighed, in
+    // workgroups of 32 as long as fuller ones would be too few, of 64, and of 128.  Consecutive workgroups run on one XCD
+    // while the scene is small enough for its L2 to matter more than an even load (a scan that covers a 16th of 10^6
+    // particles: 1,090 us by XCD, 778 in turn; one under all of 200,000 53 and 63).
+    const bool weigh = n > 65536;
+    const int perBlock = !weigh ? kStaticBlock / kCoopLanes : n <= (7 << 15) ? 32 : n <= 524288 ? 64 : kStaticBlock;
+    const int byXcd = n <= 262144 ? 1 : 0;
     const dim3 grid((n + perBlock - 1) / perBlock);
-    if (refLayout)
-        hipLaunchKernelGGL(k_dem_static<true>, grid, dim3(kStaticBlock), 0, st, sPos, sVel, sIdx, n, perBlock, stPos,
-                           stNorm, stIdx, cs, ce, ph, g, pForce, pTorque, relPos);
-    else
-        hipLaunchKernelGGL(k_dem_static<false>, grid, dim3(kStaticBlock), 0, st, sPos, sVel, sIdx, n, perBlock, stPos,
-                           stNorm, stIdx, cs, ce, ph, g, pForce, pTorque, relPos);
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kStaticBlock), 0, st, sPos, sVel, sIdx, n, perBlock, byXcd, stPos, stNorm,
+                           stIdx, cs, ce, ph, g, pForce, pTorque, relPos);
+    };
+    if (refLayout) weigh ? run(k_dem_static<true, true>) : run(k_dem_static<true, false>);
+    else weigh ? run(k_dem_static<false, true>) : run(k_dem_static<false, false>);
 }
 
 }  // namespace arsim
