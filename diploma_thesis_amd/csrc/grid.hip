@@ -52,7 +52,8 @@ __device__ __forceinline__ void dem_write(f3 F, int ra, f3 pa, f3 va, unsigned o
 // when a queue could overflow or the particle's cells are done, two at a time.  Formed in the candidate loop, a wave
 // ran the pair force in every iteration in which any of its lanes had a contact; queued, it runs it about as often as
 // its fullest lane has contacts.  Three candidates' loads together, 16 entries (12 drain too often: 922 us a step at
-// the pile below, 16 874; two loads 900, four 878).  Settled pile of 2^22 particles: 634 -> 534 us.  Where few candidates are contacts the positions read a second time cost more than that gives.
+// the pile below, 16 874; two loads 900, four 878).  Settled pile of 2^22 particles: 634 -> 534 us.
+// Where few candidates are contacts the positions read a second time cost more than that gives.
 constexpr int kQueue = 16, kQueueAhead = 3;
 constexpr int kQueueMax = (1 << 28) - 4;   // particles: an entry holds 16 times a sorted position, read up to kQueueAhead on
 __device__ __forceinline__ float4 at16(const float4 *__restrict__ p, unsigned byteOffset) {

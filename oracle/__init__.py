@@ -1,7 +1,7 @@
 """TEST INFRASTRUCTURE ONLY: numpy-facing loader of the host oracle (oracle/liboracle.so).
 
 Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may import this package.
-It is the checker of the gfx950 kernels, never part of the product path.
+The gfx950 kernels are compared with it; it is never part of the product path.
 """
 import ctypes as C
 import os

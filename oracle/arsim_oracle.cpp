@@ -2,7 +2,7 @@
  * arsim_oracle.cpp -- TEST INFRASTRUCTURE ONLY.
  *
  * A clean-room, single-threaded host restatement of AR_Sim's per-step DEM pipeline, used as
- * the checker for the gfx950 kernels.  Only tests/, __graft_entry__.smoke() and bench.py's
+ * what the gfx950 kernels are compared with.  Only tests/, __graft_entry__.smoke() and bench.py's
  * cpu_baseline leg may load it; the product library never links or calls it.
  *
  * Two instantiations of every stage:
